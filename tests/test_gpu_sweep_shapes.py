@@ -1,0 +1,53 @@
+"""The sweep kernels at the sizes where their splits and tiles have edges,
+against the CPU oracle: counts bit for bit, forces and energy against the
+sums' own scales (each particle's summed contribution lengths S_p, and the
+energy's summed magnitudes), at the bars of the precisions: 1e-12 in FP64,
+2e-6 (forces) and 1e-6 (energy) in FP32-mixed."""
+import numpy as np
+import pytest
+
+import threebodymdalgorithms_amd as tb3
+
+pytestmark = pytest.mark.gpu
+
+BARS = {"fp64": (1e-12, 1e-12), "fp32": (2e-6, 1e-6)}
+
+
+def jittered(n, seed, spacing=0.8, sd=0.05):
+    """n random sites of a cubic grid, each moved by N(0, sd)."""
+    per = int(np.ceil(round(n ** (1 / 3), 9)))
+    rng = np.random.default_rng(seed)
+    site = rng.permutation(per ** 3)[:n]
+    grid = np.stack([site % per, site // per % per, site // per ** 2], 1)
+    return (grid + 0.5) * spacing + rng.normal(0.0, sd, (n, 3))
+
+
+@pytest.fixture(scope="module")
+def eng():
+    with tb3.Engine(0) as e:
+        yield e
+
+
+def check(eng, oracle, P, precision, cutoff=-1.0, L=None):
+    E, f, dnu, cnt = eng.energy_grad()
+    *_, fo, co = oracle.sweep(P, cutoff=cutoff, L=L, mode="owner")
+    Eo = oracle.energy(P, cutoff=cutoff, L=L)
+    Eo = Eo[0] if isinstance(Eo, tuple) else Eo
+    Es = oracle.energy_scale(P, cutoff=cutoff, L=L)
+    Es = Es[0] if isinstance(Es, tuple) else Es
+    S = oracle.force_scale(P, cutoff=cutoff, L=L)
+    bar_f, bar_e = BARS[precision]
+    assert cnt == co
+    assert np.all(np.linalg.norm(f - fo, axis=1) <= bar_f * S)
+    assert abs(E - Eo) <= bar_e * Es and dnu == E
+    E2, cnt2 = eng.energy()
+    assert cnt2 == co and abs(E2 - Eo) <= bar_e * Es
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [3, 4, 63, 64, 65, 127, 128, 129, 193, 450])
+def test_all_triplets_tile_edges(eng, oracle, n, precision):
+    P = jittered(n, n)
+    eng.set_particles(P)
+    eng.configure("auta", precision=precision)
+    check(eng, oracle, P, precision)

@@ -322,15 +322,17 @@ __device__ __forceinline__ float rsqrt_t(float x) { return rsqrt_f32(x); }
 // without cancellation; the coefficient paired with the sum is then rebuilt
 // as sum - partner in FP64 (exact for FP32 operands), so that the third
 // particle sees sum * (its vector) plus partner * (the short side).
+// `live` scales the reciprocal root: 1, or 0 for a triplet that does not
+// count (its coefficients and energy are then zero).
 __device__ __forceinline__ void at_coeffs_mixed(double u64, double v64, double w64, float nu, float K, double &cu,
-                                                double &cv, double &cw, float &e, bool need_w)
+                                                double &cv, double &cw, float &e, bool need_w, float live = 1.0f)
 {
     const float u = (float)u64, v = (float)v64, w = (float)w64;
     const float A = (float)((u64 + v64) - w64);
     const float B = (float)((u64 - v64) + w64);
     const float C = (float)((v64 - u64) + w64);
     const float uv = u * v;
-    const float s = rsqrt_f32(uv * w);
+    const float s = rsqrt_f32(uv * w) * live;
     const float s2 = s * s;
     const float X = B * C, Y = A * C, Z = A * B;
     const float Q = (A * X) * s2;
@@ -398,6 +400,31 @@ __device__ __forceinline__ void at_coeffs(T u, T v, T w, T nu, T K, T &eu, T &ev
     if constexpr (NEED_W) ew = c2s5 * fma_t<T>(R, uv, fma_t<T>(m2K, X, KS));
     else ew = T(0);
     e = (s2 * s) * fma_t<T>(K, Q, nu);
+}
+
+// at_coeffs in FP64 with s = (u v w)^-1/2 given; s = 0 (u, v, w finite) gives
+// zero coefficients and energy.
+template <bool WANT_E>
+__device__ __forceinline__ void at_coeffs_roots(double u, double v, double w, double s, double nu, double K,
+                                                double &eu, double &ev, double &ew, double &e)
+{
+    const double s2 = s * s;
+    const double d = u - v;
+    const double A = (u + v) - w;
+    const double B = d + w;
+    const double C = w - d;
+    const double X = B * C, Y = A * C, Z = A * B;
+    const double Q = (A * X) * s2;
+    const double R = __builtin_fma(-5.0 * K, Q, -3.0 * nu);
+    const double S = (X + Y) + Z;
+    const double KS = (2.0 * K) * S;
+    const double m4K = -4.0 * K;
+    const double s3 = s2 * s;
+    const double s5 = s2 * s3;
+    eu = s5 * __builtin_fma(R, v * w, __builtin_fma(m4K, Z, KS));
+    ev = s5 * __builtin_fma(R, u * w, __builtin_fma(m4K, Y, KS));
+    ew = s5 * __builtin_fma(R, u * v, __builtin_fma(m4K, X, KS));
+    e = WANT_E ? s3 * __builtin_fma(K, Q, nu) : 0.0;
 }
 
 template <class T, bool NEED_W>

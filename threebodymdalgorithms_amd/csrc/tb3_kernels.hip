@@ -2535,14 +2535,37 @@ __global__ __launch_bounds__(WAVE, 5) void k_p3bca_exact(CutDev a)
 // Fast all-triplets sweep over tile triples (NATA / AUTA, or P3BCA without a
 // cutoff).
 //
-// A wave takes a triple of 64-particle tiles t0 <= t1 <= t2 and every
-// triplet (i, j, k) in it with i < j < k.  Lane l owns i = 64 t0 + l; j runs
-// over tile t1 in lock step (broadcast from LDS); k runs over tile t2 skewed
-// by lane, k = 64 t2 + ((l + s) mod 64), so at every step the 64 lanes touch
-// 64 distinct k and can update k's force accumulator in LDS without
-// conflicts.  j's force is reduced across lanes once per j.  The three tiles'
-// forces are added to global memory with one FP64 atomic per particle and
+// A wave takes a triple of 64-particle tiles t0 <= t1 <= t2 (or a share of
+// its j, below) and every triplet (i, j, k) in it with i < j < k.  Lane l owns
+// i = 64 t0 + l; j runs over tile t1 in lock step, TILE_JB at a time; k runs
+// over tile t2 skewed by lane, k = 64 t2 + ((l + s) mod 64), so at every step
+// the 64 lanes touch 64 distinct k and update k's accumulators in LDS without
+// conflicts.
+//
+// The sweep is bound by VALU issue, so what a triplet shares with others is
+// taken out of its own arithmetic:
+//  * a side's square and its power -1/2 belong to a pair, not to a triplet:
+//    (j, k)'s are computed once per j by the lane of k and read from LDS by
+//    every i, (i, k)'s once per TILE_JB triplets, (i, j)'s once per 64; the
+//    triplet's (u v w)^-1/2 is then the product of three (the mixed form
+//    keeps its FP32 reciprocal root of the product);
+//  * the gradient is summed per pair as well: (i, j)'s and (i, k)'s
+//    coefficients over k and over the j of a block in registers, (j, k)'s
+//    over i in LDS, and each sum multiplies its pair's difference once;
+//  * a pair in the wrong order, or with a padding slot, gets the power 0
+//    (the mixed form: the factor 0), which zeroes its triplets' coefficients
+//    and energy without a test per triplet, and the count of the triplets is
+//    arithmetic on the tile indices.
+// The forces are added to global memory with one FP64 atomic per particle and
 // component at the end.
+//
+// What remains per triplet is about 45 VALU instructions, 35 of them the
+// coefficients.  N = 2048: 2.13 ms in place of 4.5, 77 TFLOP/s of the 115
+// FLOP a triplet counts for; N = 3001 mixed 8.4 in place of 13.7 ms (its FP32
+// coefficients are as they were, ~75 instructions).
+//
+// A launch with few triples is split: `jparts` waves share a triple's j and
+// `sparts` the steps over k (tile_parts).
 
 struct TileDev {
     int n;
@@ -2552,7 +2575,7 @@ struct TileDev {
     double *fx, *fy, *fz;
     Status *st;
     int count_slot;
-    int want_energy;
+    int jparts, sparts;  // waves per triple: shares of the j, times shares of the steps over k (powers of two)
 };
 
 __device__ __forceinline__ void unpack_triple(unsigned long long t, int &t0, int &t1, int &t2)
@@ -2562,114 +2585,163 @@ __device__ __forceinline__ void unpack_triple(unsigned long long t, int &t0, int
     t2 = (int)((t >> 42) & 0x1fffffull);
 }
 
-template <class T, bool GRAD>
-__global__ __launch_bounds__(WAVE) void k_forces_tiles(TileDev a)
+template <class T, bool GRAD, bool WANT_E, int TILE_JB>
+__global__ __launch_bounds__(WAVE, TILE_JB > 4 ? 3 : 4) void k_forces_tiles(TileDev a)
 {
-    __shared__ double jx[WAVE], jy[WAVE], jz[WAVE];
+    constexpr bool FP64 = sizeof(T) == 8;
     __shared__ double kx[WAVE], ky[WAVE], kz[WAVE];
     __shared__ double fkx[WAVE], fky[WAVE], fkz[WAVE];
-    __shared__ double fjx[WAVE], fjy[WAVE], fjz[WAVE];
+    __shared__ double pw[TILE_JB][WAVE];  // (j, k): squared side
+    __shared__ T ps[TILE_JB][WAVE];       // its power -1/2, or 0; mixed: 1 or 0
+    __shared__ double pc[TILE_JB][WAVE];  // its summed coefficient
     int t0, t1, t2;
-    unpack_triple(a.triples[blockIdx.x], t0, t1, t2);
+    unpack_triple(a.triples[blockIdx.x / (unsigned)(a.jparts * a.sparts)], t0, t1, t2);
+    const int part = (int)(blockIdx.x % (unsigned)(a.jparts * a.sparts));
+    const int sp = part % a.sparts, jn = WAVE / a.jparts;
+    const int jlo = part / a.sparts * jn, jhi = jlo + jn;
     const int lane = lane_id();
     const int n = a.n;
-    const int i = t0 * WAVE + lane;
-    {
-        const int j = t1 * WAVE + lane, k = t2 * WAVE + lane;
-        // Padding slots get distinct far-away coordinates so the (masked)
-        // arithmetic on them stays finite.
-        const double far = 1.0e6 + 16.0 * lane;
-        jx[lane] = j < n ? a.x[j] : far;
-        jy[lane] = j < n ? a.y[j] : far;
-        jz[lane] = j < n ? a.z[j] : far;
-        kx[lane] = k < n ? a.x[k] : -far;
-        ky[lane] = k < n ? a.y[k] : -far;
-        kz[lane] = k < n ? a.z[k] : -far;
-        fkx[lane] = fky[lane] = fkz[lane] = 0.0;
-        fjx[lane] = fjy[lane] = fjz[lane] = 0.0;
-    }
-    const double xi = i < n ? a.x[i] : 3.0e6, yi = i < n ? a.y[i] : 3.0e6, zi = i < n ? a.z[i] : 3.0e6;
-    __syncthreads();
+    const int jbase = t1 * WAVE, kbase = t2 * WAVE;
+    const int i = t0 * WAVE + lane, jl = jbase + lane, kl = kbase + lane;
+    // Padding slots get distinct far-away coordinates so the arithmetic on
+    // them stays finite.
+    const double far = 1.0e6 + 16.0 * lane;
+    const double xi = i < n ? a.x[i] : far, yi = i < n ? a.y[i] : far, zi = i < n ? a.z[i] : far;
+    kx[lane] = kl < n ? a.x[kl] : -far;
+    ky[lane] = kl < n ? a.y[kl] : -far;
+    kz[lane] = kl < n ? a.z[kl] : -far;
+    fkx[lane] = fky[lane] = fkz[lane] = 0.0;
 
     const T nu = (T)a.nu, K = (T)(0.375 * a.nu);
-    double gix = 0.0, giy = 0.0, giz = 0.0, esum = 0.0;
-    unsigned cnt = 0;
-    const int jbase = t1 * WAVE, kbase = t2 * WAVE;
+    double gix = 0.0, giy = 0.0, giz = 0.0;  // i's gradient
+    double gjx = 0.0, gjy = 0.0, gjz = 0.0;  // that of j = jbase + lane
+    double esum = 0.0;
+    // tiles in which some (i, k) is no pair (wrong order, itself or padding):
+    // such a pair's side is set to 1, so that only finite numbers meet the
+    // zeros of the triplet's other sides
+    const bool edge = t0 == t2 || kbase + WAVE > n;
 
-    for (int jj = 0; jj < WAVE; ++jj) {
-        const int j = jbase + jj;
-        if (j >= n) break;
-        const double xj = jx[jj], yj = jy[jj], zj = jz[jj];
-        const double dijx = xj - xi, dijy = yj - yi, dijz = zj - zi;
-        const double u64 = __builtin_fma(dijx, dijx, __builtin_fma(dijy, dijy, dijz * dijz));
-        const bool ij_ok = i < j;
-        double gjx = 0.0, gjy = 0.0, gjz = 0.0;
-        for (int s = 0; s < WAVE; ++s) {
-            const int kk = (lane + s) & (WAVE - 1);
-            const int k = kbase + kk;
-            const bool ok = ij_ok && j < k && k < n;
-            const double xk = kx[kk], yk = ky[kk], zk = kz[kk];
-            const double dikx = xk - xi, diky = yk - yi, dikz = zk - zi;
-            const double djkx = xk - xj, djky = yk - yj, djkz = zk - zj;
-            const double v = __builtin_fma(dikx, dikx, __builtin_fma(diky, diky, dikz * dikz));
-            const double w = __builtin_fma(djkx, djkx, __builtin_fma(djky, djky, djkz * djkz));
-            double cu, cv, cw;
-            T et;
-            at_coeffs_from64<T, true>(u64, v, w, nu, K, cu, cv, cw, et);
-            cu = ok ? cu : 0.0;
-            cv = ok ? cv : 0.0;
-            cw = ok ? cw : 0.0;
-            if (GRAD) {
-                gix = __builtin_fma(-cu, dijx, __builtin_fma(-cv, dikx, gix));
-                giy = __builtin_fma(-cu, dijy, __builtin_fma(-cv, diky, giy));
-                giz = __builtin_fma(-cu, dijz, __builtin_fma(-cv, dikz, giz));
-                gjx = __builtin_fma(cu, dijx, __builtin_fma(-cw, djkx, gjx));
-                gjy = __builtin_fma(cu, dijy, __builtin_fma(-cw, djky, gjy));
-                gjz = __builtin_fma(cu, dijz, __builtin_fma(-cw, djkz, gjz));
-                fkx[kk] = __builtin_fma(cv, dikx, __builtin_fma(cw, djkx, fkx[kk]));
-                fky[kk] = __builtin_fma(cv, diky, __builtin_fma(cw, djky, fky[kk]));
-                fkz[kk] = __builtin_fma(cv, dikz, __builtin_fma(cw, djkz, fkz[kk]));
+    for (int j0 = jlo; j0 < jhi; j0 += TILE_JB) {
+        if (jbase + j0 >= n) break;
+        double u[TILE_JB], cu_sum[TILE_JB];
+        T su[TILE_JB];
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < TILE_JB; ++q) {
+            const int j = jbase + j0 + q, jc = min(j, n - 1);  // uniform
+            const double xj = a.x[jc], yj = a.y[jc], zj = a.z[jc];
+            // (i, j) in this lane
+            const double dx = xj - xi, dy = yj - yi, dz = zj - zi;
+            const double uu = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+            const bool ij = i < j && j < n;
+            u[q] = ij ? uu : 1.0;
+            if constexpr (FP64) su[q] = ij ? rsqrt_f64(uu) : 0.0;
+            else su[q] = ij ? T(1) : T(0);
+            cu_sum[q] = 0.0;
+            // (j, k) for k = kbase + lane
+            const double ex = kx[lane] - xj, ey = ky[lane] - yj, ez = kz[lane] - zj;
+            const double ww = __builtin_fma(ex, ex, __builtin_fma(ey, ey, ez * ez));
+            const bool jk = j < kl && kl < n;
+            pw[q][lane] = jk ? ww : 1.0;
+            if constexpr (FP64) ps[q][lane] = jk ? rsqrt_f64(ww) : 0.0;
+            else ps[q][lane] = jk ? T(1) : T(0);
+            if (GRAD) pc[q][lane] = 0.0;
+        }
+        wave_sync();
+        // k > j alone counts: where j and k share a tile, the last half,
+        // quarter, ... of it holds every k of the later j (several lanes
+        // then meet at a k, which the LDS adds allow)
+        int m = WAVE;
+        if (t1 == t2)
+            while (2 * (WAVE - 1 - j0) <= m && m > a.sparts) m >>= 1;
+        const int ks = m / a.sparts;
+#pragma unroll 1
+        for (int s = sp * ks; s < (sp + 1) * ks; ++s) {
+            const int kk = WAVE - m + ((lane + s) & (m - 1));
+            const double dx = kx[kk] - xi, dy = ky[kk] - yi, dz = kz[kk] - zi;
+            double v = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+            if (edge && !(i < kbase + kk && kbase + kk < n)) v = 1.0;
+            T sv = T(1);
+            if constexpr (FP64) sv = rsqrt_f64(v);
+            double cv_sum = 0.0;
+#pragma unroll
+            for (int q = 0; q < TILE_JB; ++q) {
+                const double w = pw[q][kk];
+                double cu, cv, cw;
+                T et;
+                if constexpr (FP64) at_coeffs_roots<WANT_E>(u[q], v, w, (su[q] * sv) * ps[q][kk], nu, K, cu, cv, cw, et);
+                else at_coeffs_mixed(u[q], v, w, nu, K, cu, cv, cw, et, GRAD, su[q] * ps[q][kk]);
+                if (GRAD) {
+                    cu_sum[q] += cu;
+                    cv_sum += cv;
+                    lds_add(&pc[q][kk], cw);
+                }
+                if (WANT_E) esum += (double)et;
             }
-            if (ok) {
-                esum += (double)et;
-                ++cnt;
+            if (GRAD) {
+                const double tx = cv_sum * dx, ty = cv_sum * dy, tz = cv_sum * dz;
+                gix -= tx;
+                giy -= ty;
+                giz -= tz;
+                lds_add(&fkx[kk], tx);
+                lds_add(&fky[kk], ty);
+                lds_add(&fkz[kk], tz);
             }
         }
         if (GRAD) {
-            gjx = wave_sum(gjx);
-            gjy = wave_sum(gjy);
-            gjz = wave_sum(gjz);
-            if (lane == 0) {
-                fjx[jj] += gjx;
-                fjy[jj] += gjy;
-                fjz[jj] += gjz;
+            wave_sync();
+#pragma unroll
+            for (int q = 0; q < TILE_JB; ++q) {
+                const int jc = min(jbase + j0 + q, n - 1);
+                const double xj = a.x[jc], yj = a.y[jc], zj = a.z[jc];
+                const double cw = pc[q][lane];
+                const double tx = cw * (kx[lane] - xj), ty = cw * (ky[lane] - yj), tz = cw * (kz[lane] - zj);
+                fkx[lane] += tx;
+                fky[lane] += ty;
+                fkz[lane] += tz;
+                const double ux = cu_sum[q] * (xj - xi), uy = cu_sum[q] * (yj - yi), uz = cu_sum[q] * (zj - zi);
+                gix -= ux;
+                giy -= uy;
+                giz -= uz;
+                const double sx = wave_total(ux - tx), sy = wave_total(uy - ty), sz = wave_total(uz - tz);
+                if (lane == j0 + q) {
+                    gjx = sx;
+                    gjy = sy;
+                    gjz = sz;
+                }
             }
         }
     }
-    __syncthreads();
+    wave_sync();
     if (GRAD) {
         if (i < n) {
             unsafeAtomicAdd(&a.fx[i], gix);
             unsafeAtomicAdd(&a.fy[i], giy);
             unsafeAtomicAdd(&a.fz[i], giz);
         }
-        const int j = jbase + lane, k = kbase + lane;
-        if (j < n) {
-            unsafeAtomicAdd(&a.fx[j], fjx[lane]);
-            unsafeAtomicAdd(&a.fy[j], fjy[lane]);
-            unsafeAtomicAdd(&a.fz[j], fjz[lane]);
+        if (jl < n && lane >= jlo && lane < jhi) {
+            unsafeAtomicAdd(&a.fx[jl], gjx);
+            unsafeAtomicAdd(&a.fy[jl], gjy);
+            unsafeAtomicAdd(&a.fz[jl], gjz);
         }
-        if (k < n) {
-            unsafeAtomicAdd(&a.fx[k], fkx[lane]);
-            unsafeAtomicAdd(&a.fy[k], fky[lane]);
-            unsafeAtomicAdd(&a.fz[k], fkz[lane]);
+        if (kl < n) {
+            unsafeAtomicAdd(&a.fx[kl], fkx[lane]);
+            unsafeAtomicAdd(&a.fy[kl], fky[lane]);
+            unsafeAtomicAdd(&a.fz[kl], fkz[lane]);
         }
     }
-    if (a.want_energy) esum = wave_sum(esum);
-    const unsigned long long c = wave_sum_u64(cnt);
+    // this j's triplets: the i of tile t0 below it times the k of tile t2 above it
+    unsigned c = 0;
+    if (lane >= jlo && lane < jhi && jl < n && sp == 0) {
+        const int ni = min(max(jl - t0 * WAVE, 0), WAVE);
+        const int nk = min(max(min(n, kbase + WAVE) - max(jl + 1, kbase), 0), WAVE);
+        c = (unsigned)(ni * nk);
+    }
+    const unsigned long long cw = wave_sum_u64(c);
+    if (WANT_E) esum = wave_sum(esum);
     if (lane == 0) {
-        if (a.want_energy) add_energy(a.st, esum);
-        add_count(a.st, a.count_slot, c);
+        if (WANT_E) add_energy(a.st, esum);
+        add_count(a.st, a.count_slot, cw);
     }
 }
 
@@ -3081,6 +3153,48 @@ void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *s
     hipLaunchKernelGGL(k_auta_exact, dim3((unsigned)(3 * d.n)), dim3(WAVE), 0, s, a);
 }
 
+// The j per block: 8 halve what a block of 4 shares again, but take 127
+// VGPRs and 15 KB of LDS, 3 waves per SIMD instead of 4.  FP64 from 1024
+// triples (23 tiles: N = 2048 2.16 against 2.27 ms, N = 1400 810 against 847
+// us, but N = 1000, whose waves are fewer, 386 against 371 us); the mixed
+// form never (9.05 against 8.5 ms at N = 3001: its live registers spill).
+static int tile_jb(long long ntriples, int mixed) { return !mixed && ntriples >= 1024 ? 8 : 4; }
+
+// Waves per triple, so that the last waves of a launch end together: shares
+// of the j down to one block until the launch has 32768 waves (N = 3000:
+// 6.65 ms against 7.0 with 16384; N = 2048 does not care), then shares of the
+// k steps until it has 1024, one per SIMD (N = 300: a call of 85 us against
+// 91 with 2048 waves and 127 with 4096, whose atomics meet on few particles).
+static void tile_parts(long long ntriples, int jb, int *jparts, int *sparts)
+{
+    *jparts = *sparts = 1;
+    while (*jparts < WAVE / jb && ntriples * *jparts < 32768) *jparts *= 2;
+    while (*sparts < 8 && ntriples * *jparts * *sparts < 1024) *sparts *= 2;
+}
+
+template <int JB>
+static void launch_tiles_jb(hipStream_t s, const TileDev &a, long long ntriples, int mixed, int grad, int want_energy)
+{
+    const dim3 grid((unsigned)(ntriples * a.jparts * a.sparts)), blk(WAVE);
+#define TB3_TILES(T, G, E, J) hipLaunchKernelGGL((k_forces_tiles<T, G, E, J>), grid, blk, 0, s, a)
+    if (mixed) {
+        if (grad) {
+            if (want_energy) TB3_TILES(float, true, true, 4);
+            else TB3_TILES(float, true, false, 4);
+        } else {
+            TB3_TILES(float, false, true, 4);
+        }
+    } else {
+        if (grad) {
+            if (want_energy) TB3_TILES(double, true, true, JB);
+            else TB3_TILES(double, true, false, JB);
+        } else {
+            TB3_TILES(double, false, true, JB);
+        }
+    }
+#undef TB3_TILES
+}
+
 void launch_forces_tiles(hipStream_t s, const DeviceState &d, const unsigned long long *triples,
                          long long ntriples, double nu, int mixed, int grad, Status *st, int count_slot,
                          int want_energy)
@@ -3098,15 +3212,10 @@ void launch_forces_tiles(hipStream_t s, const DeviceState &d, const unsigned lon
     a.fz = d.fz;
     a.st = st;
     a.count_slot = count_slot;
-    a.want_energy = want_energy;
-    const dim3 grid((unsigned)ntriples), blk(WAVE);
-    if (mixed) {
-        if (grad) hipLaunchKernelGGL((k_forces_tiles<float, true>), grid, blk, 0, s, a);
-        else hipLaunchKernelGGL((k_forces_tiles<float, false>), grid, blk, 0, s, a);
-    } else {
-        if (grad) hipLaunchKernelGGL((k_forces_tiles<double, true>), grid, blk, 0, s, a);
-        else hipLaunchKernelGGL((k_forces_tiles<double, false>), grid, blk, 0, s, a);
-    }
+    const int jb = tile_jb(ntriples, mixed);
+    tile_parts(ntriples, jb, &a.jparts, &a.sparts);
+    if (jb == 8) launch_tiles_jb<8>(s, a, ntriples, mixed, grad, want_energy);
+    else launch_tiles_jb<4>(s, a, ntriples, mixed, grad, want_energy);
 }
 
 void launch_selftest_fp64(hipStream_t s, long long n, const double *a, const double *b, double *sq, double *q,
