@@ -51,3 +51,43 @@ def test_all_triplets_tile_edges(eng, oracle, n, precision):
     eng.set_particles(P)
     eng.configure("auta", precision=precision)
     check(eng, oracle, P, precision)
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 8, 9, 65, 130, 257, 699, 702])
+def test_exact_all_triplets_group_edges(eng, oracle, n):
+    """Bit for bit at the edges of the bit-exact sweep's rounds (64 items and
+    multiples) and particle groups (2 below 700 particles, 4 from there)."""
+    P = jittered(n, 1000 + n)
+    eng.set_particles(P)
+    eng.configure("nata", precision="exact")
+    assert eng.compute_forces() == n * (n - 1) * (n - 2) // 6
+    *_, fo, _ = oracle.sweep(P, mode="owner")
+    assert np.array_equal(eng.get_particles()["f"], fo)
+
+
+def test_exact_all_triplets_out_of_range_side(eng, oracle):
+    """Sides out of the in-range sequences' range: the same bits."""
+    P = jittered(70, 5)
+    P[0] = (1e14, 0.0, 0.0)
+    eng.set_particles(P)
+    eng.configure("auta", precision="exact")
+    eng.compute_forces()
+    *_, fo, _ = oracle.sweep(P, mode="owner")
+    assert np.array_equal(eng.get_particles()["f"], fo)
+
+
+def test_exact_all_triplets_past_the_pair_table(eng):
+    """More particles than the table of pair lengths holds: against the FP64
+    path, at the bar of the all-triplets sweep of 2048 particles."""
+    n = 4100
+    P = jittered(n, 6)
+    eng.set_particles(P)
+    eng.configure("auta", precision="exact")
+    cnt = eng.compute_forces()
+    f = eng.get_particles()["f"]
+    eng.configure("auta", precision="fp64")
+    assert cnt == eng.compute_forces() == n * (n - 1) * (n - 2) // 6
+    f64 = eng.get_particles()["f"]
+    size = np.linalg.norm(f, axis=1)
+    floor = np.sqrt(np.mean(size ** 2))
+    assert np.all(np.linalg.norm(f64 - f, axis=1) <= 2e-11 * np.maximum(size, floor))

@@ -58,8 +58,8 @@ __device__ __forceinline__ double sqr_dist_periodic_min(double ax, double ay, do
 //
 // gfx950 has no FP64 divide or square-root instruction; the compiler expands
 // a / b into a Newton-Raphson sequence (reciprocal estimate, two refinements
-// y <- y + y (1 - b y), quotient q = a y, and the Markstein correction
-// q + y (a - b q), each step one FMA) wrapped in three range steps:
+// r <- r + r (1 - b r), quotient q = a r, and the Markstein correction
+// q + r (a - b q), each step one FMA) wrapped in three range steps:
 // v_div_scale scales an operand by a power of two when the quotient or the
 // reciprocal would leave the normal range or the numerator is near the
 // bottom of it, v_div_fmas undoes that scaling in the last FMA, and
@@ -67,28 +67,47 @@ __device__ __forceinline__ double sqr_dist_periodic_min(double ax, double ay, do
 // operands far inside the normal range (every caller here keeps numerators,
 // denominators and quotients within 2^-500 .. 2^500, or a zero numerator)
 // the scale step leaves both operands as they are, the last FMA is a plain
-// FMA, and the fixup returns the quotient unchanged.  div_rn_inrange is the
-// sequence without the three range steps: on such operands it yields the
-// bits of a / b in 8 instructions instead of 11.  The square root likewise:
-// sqrt(x) rescales x when it is tiny and passes +-0 and +inf through around
-// a Newton iteration on the reciprocal square-root estimate; for x within
-// 2^-500 .. 2^500 those steps are the identity and sqrt_rn_inrange is the
-// iteration alone (10 instructions instead of 17).  Both are checked bit for
-// bit against the compiler's IEEE expansions on the device
-// (tb3_selftest_fp64_inrange).
-__device__ __forceinline__ double div_rn_inrange(double a, double b)
+// FMA, and the fixup returns the quotient unchanged.
+//
+// div_rn_from leaves out those range steps and also the estimate and the
+// first refinement: the caller gives an approximation r of 1 / b that is
+// within 2^-46.  The refinement squares that error, so what goes into the
+// quotient is 1 / b to within half an ulp and 2^-92, and the rest is the
+// same: the bits of a / b in 5 instructions where the estimate (which issues
+// at a quarter of the FMA's rate) and two refinements take 8, four of them
+// for the estimate's slots.
+// Why the bits: what the last FMA rounds is off from a / b by
+// |a / b - q| |1 - b r|.  Near a midpoint m of two doubles q is half an ulp
+// away, so with b scaled to [1, 2) that is at most ulp(q) b 2^-55 (1 + 2^-38),
+// while a quotient that is no midpoint is at least ulp(q) 2^-53 / b away from
+// it: it falls on the right side for b^2 < 4 (1 - 2^-38).  Left are b within
+// 2^-38 of 2, b = 2 - t 2^-52, whose reciprocal is misrounded for odd
+// t < 128 only; over those, in exact rational arithmetic, the result is wrong
+// just for t = 1 (a mantissa of all ones) under a power of two.  Callers
+// whose numerator may be one send the denominators with an all-ones low word
+// (div_needs_ieee) to the IEEE division.
+//
+// The square root likewise: sqrt(x) rescales x when it is tiny and passes
+// +-0 and +inf through around a Newton iteration on the reciprocal
+// square-root estimate; for x within 2^-500 .. 2^500 those steps are the
+// identity and sqrt_rn_inrange is the iteration alone (10 instructions
+// instead of 17).  Its by-product h, half the reciprocal root, gives
+// 1 / sqrt(x) to within 2^-52 in two more, from whose powers the reciprocals
+// of the brackets' denominators are formed.
+// Both are checked bit for bit against the compiler's IEEE expansions on the
+// device (tb3_selftest_fp64_inrange).
+__device__ __forceinline__ unsigned low_word(double b) { return (unsigned)__double_as_longlong(b); }
+__device__ __forceinline__ bool div_needs_ieee(unsigned low) { return low == 0xffffffffu; }
+
+__device__ __forceinline__ double div_rn_from(double a, double b, double r)
 {
-    double r = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
     const double q = a * r;
     const double rem = __builtin_fma(-b, q, a);
     return __builtin_fma(rem, r, q);
 }
 
-__device__ __forceinline__ double sqrt_rn_inrange(double x)
+__device__ __forceinline__ double sqrt_rn_inrange(double x, double &inv)
 {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y;
@@ -99,53 +118,89 @@ __device__ __forceinline__ double sqrt_rn_inrange(double x)
     double d = __builtin_fma(-g, g, x);
     g = __builtin_fma(d, h, g);
     d = __builtin_fma(-g, g, x);
-    return __builtin_fma(d, h, g);
+    g = __builtin_fma(d, h, g);
+    const double r = h + h;
+    inv = __builtin_fma(r, __builtin_fma(-g, r, 1.0), r);
+    return g;
 }
 
-struct RefPowers {
-    double d1, d2, d3, d4, d5, d6;  // AxilrodTeller.cpp:33-51
+// A side's powers (AxilrodTeller.cpp:33-51) and, for the in-range sequences,
+// approximations of the reciprocals of those that the denominators take.
+struct RefSide {
+    double d1, d2, d3, d4, d5, d6;
+    double i1, i2;
 };
 
-__device__ __forceinline__ RefPowers ref_powers(double d1)
+template <bool INRANGE>
+__device__ __forceinline__ RefSide ref_powers(double d1, double i1)
 {
-    RefPowers p;
+    RefSide p;
     p.d1 = d1;
     p.d2 = p.d1 * d1;
     p.d3 = p.d2 * d1;
     p.d4 = p.d3 * d1;
     p.d5 = p.d4 * d1;
     p.d6 = p.d5 * d1;
+    if constexpr (INRANGE) {
+        p.i1 = i1;
+        p.i2 = i1 * i1;
+    }
     return p;
 }
 
-// IEEE division, or its in-range sequence when the caller has checked the
-// operands' range.
+// a / b: IEEE division, or the in-range sequence from r, the product of the
+// sides' reciprocal powers (rounded powers and products: within 40 ulp of
+// 1 / b), when the caller has checked the operands' range.
 template <bool INRANGE>
-__device__ __forceinline__ double ref_div(double a, double b)
+__device__ __forceinline__ double ref_div(double a, double b, double r)
 {
-    if constexpr (INRANGE) return div_rn_inrange(a, b);
+    if constexpr (INRANGE) return div_rn_from(a, b, r);
     else return a / b;
 }
 
 // One dVdR bracket (AxilrodTeller.cpp:68-81) for own side x and the two other
 // sides y, z in the order the source names them: dVdRa = (a; b, c),
 // dVdRb = (b; a, c), dVdRc = (c; b, a).  Left-to-right sums and products.
-template <bool INRANGE = false>
-__device__ __forceinline__ double ref_bracket(double nu, const RefPowers &x, const RefPowers &y,
-                                              const RefPowers &z)
+// `low` collects the largest low word of the denominators whose numerators
+// are powers of two (or may be: 3 nu), for div_needs_ieee.
+template <bool INRANGE>
+__device__ __forceinline__ double ref_bracket(double nu, const RefSide &x, const RefSide &y, const RefSide &z,
+                                              unsigned &low)
 {
-    double t = ref_div<INRANGE>(-8., x.d4 * y.d3 * z.d3);
-    t = t - ref_div<INRANGE>(1., y.d5 * z.d5);
-    t = t + ref_div<INRANGE>(5. * y.d1, x.d6 * z.d5);
-    t = t + ref_div<INRANGE>(5. * z.d1, x.d6 * y.d5);
-    t = t - ref_div<INRANGE>(1., x.d2 * y.d3 * z.d5);
-    t = t - ref_div<INRANGE>(1., x.d2 * y.d5 * z.d3);
-    t = t - ref_div<INRANGE>(3., x.d4 * y.d1 * z.d5);
-    t = t - ref_div<INRANGE>(3., x.d4 * y.d5 * z.d1);
-    t = t - ref_div<INRANGE>(5., x.d6 * y.d1 * z.d3);
-    t = t - ref_div<INRANGE>(5., x.d6 * y.d3 * z.d1);
-    t = t + ref_div<INRANGE>(6., x.d4 * y.d3 * z.d3);
-    return ref_div<INRANGE>(3. * nu, 8. * x.d1) * t;
+    // r1 = 1 / (x^4 y^3 z^3); the other denominators differ from it by even
+    // powers of the ratios of two sides
+    double a = 0, b = 0, ai = 0, bi = 0, r1 = 0, r3 = 0, r4 = 0, r5 = 0, r6 = 0;
+    if constexpr (INRANGE) {
+        a = x.d2 * y.i2;
+        b = x.d2 * z.i2;
+        ai = y.d2 * x.i2;
+        bi = z.d2 * x.i2;
+        const double yz = (y.i1 * z.i1) * (y.i2 * z.i2), x4 = x.i2 * x.i2;
+        r1 = x4 * yz;
+        r5 = r1 * b;
+        r6 = r1 * a;
+        r3 = (r5 * x4) * y.d3;
+        r4 = (r6 * x4) * z.d3;
+    }
+    const double b1 = x.d4 * y.d3 * z.d3, b2 = y.d5 * z.d5, b5 = x.d2 * y.d3 * z.d5, b6 = x.d2 * y.d5 * z.d3;
+    const double b0 = 8. * x.d1;
+    if constexpr (INRANGE) {
+        low = max(max(low, low_word(b1)), low_word(b2));
+        low = max(max(low, low_word(b5)), low_word(b6));
+        low = max(low, low_word(b0));
+    }
+    double t = ref_div<INRANGE>(-8., b1, r1);
+    t = t - ref_div<INRANGE>(1., b2, r5 * a);
+    t = t + ref_div<INRANGE>(5. * y.d1, x.d6 * z.d5, r3);
+    t = t + ref_div<INRANGE>(5. * z.d1, x.d6 * y.d5, r4);
+    t = t - ref_div<INRANGE>(1., b5, r5);
+    t = t - ref_div<INRANGE>(1., b6, r6);
+    t = t - ref_div<INRANGE>(3., x.d4 * y.d1 * z.d5, r5 * ai);
+    t = t - ref_div<INRANGE>(3., x.d4 * y.d5 * z.d1, r6 * bi);
+    t = t - ref_div<INRANGE>(5., x.d6 * y.d1 * z.d3, r1 * ai);
+    t = t - ref_div<INRANGE>(5., x.d6 * y.d3 * z.d1, r1 * bi);
+    t = t + ref_div<INRANGE>(6., b1, r1);
+    return ref_div<INRANGE>(3. * nu, b0, 0.125 * x.i1) * t;
 }
 
 // The range the in-range sequences need, per triplet: every squared side in
@@ -155,118 +210,85 @@ __device__ __forceinline__ double ref_bracket(double nu, const RefPowers &x, con
 // roots' arguments within 2^-80 .. 2^80; nu must be 0 or within 2^-200 ..
 // 2^200 (nu_inrange, checked once per launch), which keeps 3 nu / (8 d1)
 // within 2^-250 .. 2^250.
-__device__ __forceinline__ bool sides_inrange(double sa, double sb, double sc)
-{
-    constexpr double lo = 0x1p-80, hi = 0x1p80;
-    return sa >= lo && sa <= hi && sb >= lo && sb <= hi && sc >= lo && sc <= hi;
-}
-
 __host__ __device__ inline bool nu_inrange(double nu)
 {
     const double m = nu < 0 ? -nu : nu;
     return nu == 0.0 || (m >= 0x1p-200 && m <= 0x1p200);
 }
 
-// The sides of the triplet (AxilrodTeller.cpp:23-31, 53-63): the difference
-// vectors dXa = rj - ri, dXb = rk - ri, dXc = rk - rj and the squared norms
-// of a = rj - ri, b = ri - rk, c = rj - rk.  Negating a difference is exact,
-// so |b|^2 and |c|^2 from -dXb and -dXc are the reference's bits.
-struct RefSides {
-    double dXa, dYa, dZa, dXb, dYb, dZb, dXc, dYc, dZc;
-    double sa, sb, sc;
-};
-
-__device__ __forceinline__ RefSides ref_sides(double xi, double yi, double zi, double xj, double yj, double zj,
-                                              double xk, double yk, double zk)
-{
-    RefSides t;
-    t.dXa = xj - xi, t.dYa = yj - yi, t.dZa = zj - zi;
-    t.dXb = xk - xi, t.dYb = yk - yi, t.dZb = zk - zi;
-    t.dXc = xk - xj, t.dYc = yk - yj, t.dZc = zk - zj;
-    t.sa = (t.dXa * t.dXa + t.dYa * t.dYa) + t.dZa * t.dZa;
-    t.sb = (t.dXb * t.dXb + t.dYb * t.dYb) + t.dZb * t.dZb;
-    t.sc = (t.dXc * t.dXc + t.dYc * t.dYc) + t.dZc * t.dZc;
-    return t;
-}
-
-template <bool INRANGE>
-__device__ __forceinline__ double ref_sqrt(double x)
-{
-    if constexpr (INRANGE) return sqrt_rn_inrange(x);
-    else return __builtin_sqrt(x);
-}
-
-// The brackets dVdRa, dVdRb, dVdRc that role ROLE needs (-1: all three).
+// What AxilrodTeller::CalculateForces (AxilrodTeller.cpp:22-93) subtracts
+// from the force of one particle p of a triplet, whose others are e and o in
+// the triplet's order.  Written out for p as i (e = j, o = k; ROLE 0), as j
+// (e = i, o = k; ROLE 1) and as k (e = i, o = j; ROLE 2), the three
+// contributions have one form:
+//   (e - p) S + (o - p) T,
+// S and T being the brackets of the sides s = |e - p| and t = |o - p|; the
+// reference's negated differences and brackets come in pairs, and negation is
+// exact.  Only the order of a bracket's other two sides depends on p's place:
+// the third side m = |o - e| comes last in both for i, first in both for j,
+// and first in S, last in T for k.  Each operation is the reference's, so the
+// result is bit-identical; the third bracket, which p's force does not take,
+// is not evaluated.
 template <int ROLE, bool INRANGE>
-__device__ __forceinline__ void ref_brackets(const RefSides &t, double nu, double &A, double &B, double &C)
+__device__ __forceinline__ void ref_pair_brackets(const RefSide &s, const RefSide &t, const RefSide &m, double nu,
+                                                  double &S, double &T, unsigned &low)
 {
-    const RefPowers a = ref_powers(ref_sqrt<INRANGE>(t.sa));
-    const RefPowers b = ref_powers(ref_sqrt<INRANGE>(t.sb));
-    const RefPowers c = ref_powers(ref_sqrt<INRANGE>(t.sc));
-    A = B = C = 0.0;
-    if constexpr (ROLE != 2) A = ref_bracket<INRANGE>(nu, a, b, c);
-    if constexpr (ROLE != 1) B = ref_bracket<INRANGE>(nu, b, a, c);
-    if constexpr (ROLE != 0) C = ref_bracket<INRANGE>(nu, c, b, a);
+    if constexpr (ROLE == 0) S = ref_bracket<INRANGE>(nu, s, t, m, low);
+    else S = ref_bracket<INRANGE>(nu, s, m, t, low);
+    if constexpr (ROLE == 1) T = ref_bracket<INRANGE>(nu, t, m, s, low);
+    else T = ref_bracket<INRANGE>(nu, t, s, m, low);
 }
 
-// The brackets from the in-range sequences where the triplet's sides and nu
-// allow them (nu_ok = nu_inrange(nu), hoisted by the caller), else from the
-// IEEE expansions: the same bits either way.
-template <int ROLE>
-__device__ __forceinline__ void ref_brackets_any(const RefSides &t, double nu, bool nu_ok, double &A, double &B,
-                                                 double &C)
+// A squared side: |b|^2 and |-b|^2 are the same bits.
+__device__ __forceinline__ double ref_sqr(double dx, double dy, double dz) { return (dx * dx + dy * dy) + dz * dz; }
+
+// A side's length and its reciprocal, for the in-range sequences; zeros where
+// the square is out of their range.
+__device__ __forceinline__ double2 ref_root(double sq)
 {
-    if (nu_ok && sides_inrange(t.sa, t.sb, t.sc)) ref_brackets<ROLE, true>(t, nu, A, B, C);
-    else ref_brackets<ROLE, false>(t, nu, A, B, C);
+    double2 r = make_double2(0.0, 0.0);
+    if (sq >= 0x1p-80 && sq <= 0x1p80) r.x = sqrt_rn_inrange(sq, r.y);
+    return r;
 }
 
-// Contribution that AxilrodTeller::CalculateForces subtracts from the force
-// of the particle in role ROLE (0: i, 1: j, 2: k) of the triplet (i, j, k),
-// AxilrodTeller.cpp:83-93.  Only the two brackets that role needs are
-// evaluated; each is the same IEEE operation sequence as in the full call, so
-// the result is bit-identical to the reference's.
+// The contribution, given the three sides' ref_root.  The in-range sequences
+// run where the sides and nu allow them (nu_ok = nu_inrange(nu), hoisted by
+// the caller), the IEEE expansions elsewhere: the same bits either way.
 template <int ROLE>
-__device__ __forceinline__ void ref_contrib(double xi, double yi, double zi, double xj, double yj, double zj,
-                                            double xk, double yk, double zk, double nu, bool nu_ok, double &cx,
+__device__ __forceinline__ void ref_contrib(double xp, double yp, double zp, double xe, double ye, double ze,
+                                            double xo, double yo, double zo, double2 ss, double2 st, double2 sm,
+                                            double nu, bool nu_ok, double &cx, double &cy, double &cz)
+{
+    const double ex = xe - xp, ey = ye - yp, ez = ze - zp;
+    const double ox = xo - xp, oy = yo - yp, oz = zo - zp;
+    double S = 0.0, T = 0.0;
+    bool done = false;
+    if (nu_ok && ss.y != 0.0 && st.y != 0.0 && sm.y != 0.0) {
+        unsigned low = 0;
+        ref_pair_brackets<ROLE, true>(ref_powers<true>(ss.x, ss.y), ref_powers<true>(st.x, st.y),
+                                      ref_powers<true>(sm.x, sm.y), nu, S, T, low);
+        done = !div_needs_ieee(low);
+    }
+    if (!done) {
+        unsigned low;
+        auto side = [](double sq) { return ref_powers<false>(__builtin_sqrt(sq), 0.0); };
+        ref_pair_brackets<ROLE, false>(side(ref_sqr(ex, ey, ez)), side(ref_sqr(ox, oy, oz)),
+                                       side(ref_sqr(xo - xe, yo - ye, zo - ze)), nu, S, T, low);
+    }
+    cx = ex * S + ox * T;
+    cy = ey * S + oy * T;
+    cz = ez * S + oz * T;
+}
+
+// The same from the positions alone.
+template <int ROLE>
+__device__ __forceinline__ void ref_contrib(double xp, double yp, double zp, double xe, double ye, double ze,
+                                            double xo, double yo, double zo, double nu, bool nu_ok, double &cx,
                                             double &cy, double &cz)
 {
-    const RefSides t = ref_sides(xi, yi, zi, xj, yj, zj, xk, yk, zk);
-    double A, B, C;
-    ref_brackets_any<ROLE>(t, nu, nu_ok, A, B, C);
-    if constexpr (ROLE == 0) {
-        cx = t.dXa * A + t.dXb * B;
-        cy = t.dYa * A + t.dYb * B;
-        cz = t.dZa * A + t.dZb * B;
-    } else if constexpr (ROLE == 1) {
-        cx = t.dXa * (-A) + t.dXc * C;
-        cy = t.dYa * (-A) + t.dYc * C;
-        cz = t.dZa * (-A) + t.dZc * C;
-    } else {
-        cx = t.dXb * (-B) + t.dXc * (-C);
-        cy = t.dYb * (-B) + t.dYc * (-C);
-        cz = t.dZb * (-B) + t.dZc * (-C);
-    }
-}
-
-// All three contributions of one triplet from one evaluation of the three
-// brackets (AxilrodTeller.cpp:65-93): ci, cj, ck as the reference subtracts
-// them from i.f, j.f and k.f.
-__device__ __forceinline__ void ref_contrib_all(double xi, double yi, double zi, double xj, double yj, double zj,
-                                                double xk, double yk, double zk, double nu, bool nu_ok, double *ci,
-                                                double *cj, double *ck)
-{
-    const RefSides t = ref_sides(xi, yi, zi, xj, yj, zj, xk, yk, zk);
-    double A, B, C;
-    ref_brackets_any<-1>(t, nu, nu_ok, A, B, C);
-    ci[0] = t.dXa * A + t.dXb * B;
-    ci[1] = t.dYa * A + t.dYb * B;
-    ci[2] = t.dZa * A + t.dZb * B;
-    cj[0] = t.dXa * (-A) + t.dXc * C;
-    cj[1] = t.dYa * (-A) + t.dYc * C;
-    cj[2] = t.dZa * (-A) + t.dZc * C;
-    ck[0] = t.dXb * (-B) + t.dXc * (-C);
-    ck[1] = t.dYb * (-B) + t.dYc * (-C);
-    ck[2] = t.dZb * (-B) + t.dZc * (-C);
+    ref_contrib<ROLE>(xp, yp, zp, xe, ye, ze, xo, yo, zo, ref_root(ref_sqr(xe - xp, ye - yp, ze - zp)),
+                      ref_root(ref_sqr(xo - xp, yo - yp, zo - zp)), ref_root(ref_sqr(xo - xe, yo - ye, zo - ze)), nu,
+                      nu_ok, cx, cy, cz);
 }
 
 // ---------------------------------------------------------------------------

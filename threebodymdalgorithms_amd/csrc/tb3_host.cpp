@@ -87,6 +87,7 @@ struct Buffers {
     }
 };
 
+constexpr int PAIR_ROOTS_MAX = 4096;  // particles
 constexpr int MAX_LIST = 16384;  // longest neighbour list the LDS staging accepts
 
 // Working memory of tb3_energy_grad_dev_noalloc: one static array per GPU,
@@ -175,6 +176,10 @@ struct tb3_ctx {
     unsigned long long *triples = nullptr;
     long long ntriples = 0;
     long long triples_n = -1;
+
+    // pair lengths of the bit-exact all-triplets sweep (pair_roots)
+    double2 *pair_roots = nullptr;
+    int pair_roots_cap = 0;
 
     Status *d_status = nullptr;
     Status *h_status = nullptr;  // pinned
@@ -489,6 +494,23 @@ int next_pow2(int v)
     return p;
 }
 
+// The n x n table of pair lengths that the bit-exact all-triplets sweep reads
+// (16 bytes a pair, 256 MiB at the most).  Without it (more particles, or no
+// memory) the sweep computes every length where it needs it.
+void ensure_pair_roots(tb3_ctx *c, int n)
+{
+    if (n > PAIR_ROOTS_MAX || n <= c->pair_roots_cap) return;
+    dev_free(c->pair_roots);
+    c->pair_roots_cap = 0;
+    ++c->epoch;
+    if (hipMalloc((void **)&c->pair_roots, (size_t)n * n * sizeof(double2)) == hipSuccess) {
+        c->pair_roots_cap = n;
+    } else {
+        c->pair_roots = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
 // The force sweep proper on positions already in d (and, for the cutoff
 // algorithm, on a cell list already built for them).
 //   grad   : dE/dx (the reference's f) into d.fx/fy/fz
@@ -509,7 +531,7 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
     if (d.n >= 3) {
         if (exact && grad) {
             if (cut) launch_p3bca_exact(s, d, c->grid, cs, c->nu, c->list_cap, c->d_status);
-            else launch_auta_exact(s, d, c->nu, c->d_status);
+            else launch_auta_exact(s, d, c->nu, c->d_status, d.n <= c->pair_roots_cap ? c->pair_roots : nullptr);
         }
         if (fast_grad || energy) {
             const int slot = (exact && grad) ? 1 : 0;  // the exact pass owns count[0]
@@ -569,6 +591,7 @@ void launch_prepare(tb3_ctx *c, hipStream_t s, DeviceState &d, bool predict, dou
         launch_cells_build(s, d, predict ? 1 : 0, dt, dt * dt * 0.5, zero_f ? 1 : 0, c->grid, c->d_status,
                            c->scan_tmp);
     } else {
+        if (!cut && exact && grad && d.n >= 3 && !in_graph) ensure_pair_roots(c, d.n);
         if (predict) launch_predict(s, d, dt, dt * dt * 0.5);
         if (c->recording) HIPCHK(hipEventRecord(c->ev[1], s));
         if (zero_f) {
@@ -812,7 +835,10 @@ void run_steps_graph(tb3_ctx *c, int steps, double dt, const double *g, uint64_t
             ensure_grid_buffers(c, d.n);
             ensure_slot_buffers(c, d.n);
         }
-        if (!uses_cutoff(c) && d.n >= 3 && c->precision != TB3_FP64_EXACT) ensure_triples(c, d.n);
+        if (!uses_cutoff(c) && d.n >= 3) {
+            if (c->precision == TB3_FP64_EXACT) ensure_pair_roots(c, d.n);
+            else ensure_triples(c, d.n);
+        }
         capture_step_graph(c, dt, g);
         launch_begin_steps(s, c->d_status, c->d_counts,
                            c->graph_fused && c->graph_slots > 0 ? &c->grid : nullptr);
@@ -999,6 +1025,7 @@ tb3_status tb3_destroy(tb3_ctx *c)
     dev_free(c->grid.pad_rec);
     dev_free(c->scan_tmp);
     dev_free(c->triples);
+    dev_free(c->pair_roots);
     dev_free(c->d_status);
     dev_free(c->d_slots);
     dev_free(c->d_counts);

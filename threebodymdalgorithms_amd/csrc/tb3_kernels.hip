@@ -2091,120 +2091,167 @@ struct ExactShared {
     double cb[WAVE * 3];
 };
 
-struct ImplicitList {
-    int p;
-    __device__ int operator()(int t) const { return t < p ? t : t + 1; }
-};
-
-struct LdsList {
-    const int *sid;
-    __device__ int operator()(int t) const { return sid[t]; }
-};
-
-template <int ROLE, class List>
-__device__ void exact_role(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
-                           int p, const List &elem, int len, int split, bool use_cut, double c2, double Lx,
-                           double Ly, double Lz, double nu, ExactShared &sh, double &acc,
-                           unsigned long long &accepted)
-{
-    const int lane = lane_id();
-    const bool nu_ok = nu_inrange(nu);
-    const double xp = x[p], yp = y[p], zp = z[p];
-    int a0, a1, b1;
-    bool tri;
-    if constexpr (ROLE == 0) {
-        a0 = split; a1 = len; b1 = len; tri = true;
-    } else if constexpr (ROLE == 1) {
-        a0 = 0; a1 = split; b1 = len; tri = false;
-    } else {
-        a0 = 0; a1 = split; b1 = split; tri = true;
-    }
-    acc = 0.0;  // lanes 0, 1, 2 hold x, y, z
-    int head = 0, qn = 0;
-
-    auto flush = [&](int cnt) {
-        __syncthreads();
-        if (lane < cnt) {
-            const int s = (head + lane) & (RING - 1);
-            const int ea = sh.qa[s], eb = sh.qb[s];
-            const double xa = x[ea], ya = y[ea], za = z[ea];
-            const double xb = x[eb], yb = y[eb], zb = z[eb];
-            double cx, cy, cz;
-            if constexpr (ROLE == 0)
-                ref_contrib<0>(xp, yp, zp, xa, ya, za, xb, yb, zb, nu, nu_ok, cx, cy, cz);
-            else if constexpr (ROLE == 1)
-                ref_contrib<1>(xa, ya, za, xp, yp, zp, xb, yb, zb, nu, nu_ok, cx, cy, cz);
-            else
-                ref_contrib<2>(xa, ya, za, xb, yb, zb, xp, yp, zp, nu, nu_ok, cx, cy, cz);
-            sh.cb[lane * 3 + 0] = cx;
-            sh.cb[lane * 3 + 1] = cy;
-            sh.cb[lane * 3 + 2] = cz;
-        }
-        __syncthreads();
-        if (lane < 3) {
-            for (int t = 0; t < cnt; ++t) acc = acc - sh.cb[t * 3 + lane];
-        }
-        __syncthreads();
-        head = (head + cnt) & (RING - 1);
-        qn -= cnt;
-    };
-
-    for (int ia = a0; ia < a1; ++ia) {
-        const int ea = elem(ia);
-        const double xa = x[ea], ya = y[ea], za = z[ea];
-        const int bstart = tri ? ia + 1 : split;
-        for (int b = bstart; b < b1; b += WAVE) {
-            const int bl = b + lane;
-            bool ok = bl < b1;
-            int eb = 0;
-            if (ok) {
-                eb = elem(bl);
-                if (use_cut) ok = !(sqr_dist_periodic(xa, ya, za, x[eb], y[eb], z[eb], Lx, Ly, Lz) > c2);
-            }
-            const unsigned long long m = __ballot(ok);
-            if (ok) {
-                const int s = (head + qn + __popcll(m & __lanemask_lt())) & (RING - 1);
-                sh.qa[s] = ea;
-                sh.qb[s] = eb;
-            }
-            const int got = __popcll(m);
-            qn += got;
-            accepted += (unsigned long long)got;
-            if (qn >= WAVE) flush(WAVE);
-        }
-    }
-    if (qn > 0) flush(qn);
-}
-
-// NATA / AUTA (every triplet): wave w handles role w % 3 of particle w / 3
-// (role 2 in reverse so the longest streams of every role start first).
+// NATA / AUTA (every triplet).  A workgroup of W waves takes S consecutive
+// particles through their three role streams, whose lengths add up to
+// C(n - 1, 2) for every particle, so the workgroups' work is equal.  In a
+// round every stream's next 64 W / S items are evaluated by W / S waves into
+// LDS, and one wave folds all the streams' contributions in stream order, a
+// lane per stream and component.
+//
+// Bound by VALU issue: ~300 instructions per 64 items, two brackets of 12
+// correctly rounded quotients each most of it.  What was built around that:
+//  * the fold is serial (one subtraction after another) and uses 3 S lanes of
+//    a wave, so it is shared by S streams, falls to another wave every round,
+//    and runs up to AUTA_ROUNDS rounds behind the evaluation, ordered by
+//    counters in LDS instead of workgroup barriers, which made every wave
+//    wait for the one that folds (N = 2048: 46.7 against 49.0 ms);
+//  * lengths belong to pairs: k_pair_roots computes them once (16 n^2 bytes,
+//    for n up to 4096), and an item loads its three in place of three square
+//    roots and their differences (N = 2048: 49 against 56 ms);
+//  * one wave per stream (and a fold of 3 lanes after every 64 items) ended
+//    with the longest stream, 3 times the mean: N = 1000 14.6 -> 5.9 ms, N =
+//    2048 90 -> 46.7, N = 3000 233 -> 145 ms.
+// S = 2 below 700 particles, where S = 4 leaves CUs without a workgroup (N =
+// 400 0.81 against 1.17 ms, N = 1000 6.6 against 6.0).
 struct AutaExactDev {
     int n;
     const double *x, *y, *z;
     double nu;
     double *facc;
     Status *st;
+    const double2 *roots;  // n x n: every pair's ref_root, or null
 };
 
-__global__ __launch_bounds__(WAVE) void k_auta_exact(AutaExactDev a)
+// Every pair's length and reciprocal (ref_root).
+__global__ __launch_bounds__(256) void k_pair_roots(int n, const double *__restrict__ x, const double *__restrict__ y,
+                                                    const double *__restrict__ z, double2 *__restrict__ roots)
 {
-    __shared__ ExactShared sh;
-    const int w = blockIdx.x;
-    const int role = w % 3, q = w / 3;
-    if (q >= a.n) return;
-    const int lane = lane_id();
-    const int p = role == 2 ? a.n - 1 - q : q;
-    const ImplicitList list{p};
-    double acc = 0.0;
-    unsigned long long accepted = 0;
-    if (role == 0)
-        exact_role<0>(a.x, a.y, a.z, p, list, a.n - 1, p, false, 0, 0, 0, 0, a.nu, sh, acc, accepted);
-    else if (role == 1)
-        exact_role<1>(a.x, a.y, a.z, p, list, a.n - 1, p, false, 0, 0, 0, 0, a.nu, sh, acc, accepted);
-    else
-        exact_role<2>(a.x, a.y, a.z, p, list, a.n - 1, p, false, 0, 0, 0, 0, a.nu, sh, acc, accepted);
-    if (lane < 3) a.facc[(long long)(3 * role + lane) * a.n + p] = acc;
-    if (role == 0 && lane == 0) add_count(a.st, 0, accepted);
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+    if (j < n) roots[(long long)i * n + j] = ref_root(ref_sqr(x[j] - x[i], y[j] - y[i], z[j] - z[i]));
+}
+
+constexpr int AUTA_WAVES = 8;
+constexpr int AUTA_ROUNDS = 4;  // rounds a wave may run ahead of the fold
+
+template <int W, int S>
+struct AutaExactShared {
+    static constexpr int CH = WAVE * W / S;  // items of a stream per round
+    // rows padded so that the folding lanes' 16-byte reads meet no bank conflict
+    double cb[AUTA_ROUNDS][3 * S][CH + 2];
+    double acc[3 * S];
+    unsigned ready[AUTA_ROUNDS];  // waves that wrote a buffer, over all its uses
+    unsigned folded;              // rounds folded
+};
+
+// Spins until *p (LDS) has reached v.  Every wait here is for the writes or the
+// fold of an earlier round, by waves of the same workgroup.
+__device__ __forceinline__ void wait_at_least(unsigned *p, unsigned v)
+{
+    while (__hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < v) __builtin_amdgcn_s_sleep(1);
+}
+
+template <int ROLE, int W, int S, bool ROOTS>
+__device__ void auta_exact_role(const AutaExactDev &a, int p0, AutaExactShared<W, S> &sh)
+{
+    constexpr int CH = AutaExactShared<W, S>::CH;
+    const int tid = threadIdx.x, lane = lane_id(), wv = tid / WAVE, s = tid / CH, t = tid % CH;
+    const int n = a.n;
+    const bool nu_ok = nu_inrange(a.nu);
+    const int p = min(p0 + s, n - 1);
+    const double xp = a.x[p], yp = a.y[p], zp = a.z[p];
+    // rows e up to `rows`, partners o in (e, end) or, for role 1, in (p, end);
+    // this thread takes every CH-th item of the stream
+    const int rows = ROLE == 0 ? n - 1 : (ROLE == 1 ? p : p - 1), end = ROLE == 2 ? p : n;
+    int e = ROLE == 0 ? p + 1 : 0;
+    int o = (ROLE == 1 ? p : e) + 1 + t;
+    if (p0 + s >= n || end - (ROLE == 1 ? p : e) < 2) e = rows;
+    double xe = 0, ye = 0, ze = 0, xo = 0, yo = 0, zo = 0;
+    double2 re = {}, ro = {}, rm = {};
+    // carries o over into the next rows, then loads the item (e, o)
+    auto fetch = [&] {
+#pragma clang loop unroll(disable)
+        while (o >= end && e < rows) {
+            ++e;
+            o = o - end + (ROLE == 1 ? p : e) + 1;
+        }
+        if (e < rows) {
+            if constexpr (ROOTS) {
+                re = a.roots[(unsigned)(p * n + e)];
+                ro = a.roots[(unsigned)(p * n + o)];
+                rm = a.roots[(unsigned)(e * n + o)];
+            }
+            xe = a.x[e], ye = a.y[e], ze = a.z[e];
+            xo = a.x[o], yo = a.y[o], zo = a.z[o];
+        }
+    };
+    long long longest = 0;
+    for (int k = 0; k < S && p0 + k < n; ++k) {
+        const long long q = p0 + k, above = n - 1 - q;
+        const long long items = ROLE == 0 ? above * (above - 1) / 2 : (ROLE == 1 ? q * above : q * (q - 1) / 2);
+        longest = items > longest ? items : longest;
+    }
+    const long long rounds = (longest + CH - 1) / CH;
+    if (tid < 3 * S) sh.acc[tid] = 0.0;
+    if (tid < AUTA_ROUNDS) sh.ready[tid] = 0;
+    if (tid == 0) sh.folded = 0;
+    __syncthreads();
+    auto fold = [&](unsigned r) {
+        const int b = r % AUTA_ROUNDS;
+        wait_at_least(&sh.ready[b], W * (r / AUTA_ROUNDS + 1));
+        wait_at_least(&sh.folded, r);
+        if (lane < 3 * S) {
+            const double2 *c = reinterpret_cast<const double2 *>(sh.cb[b][lane]);
+            double acc = sh.acc[lane];
+#pragma unroll 8
+            for (int k = 0; k < CH / 2; ++k) {
+                const double2 v = c[k];
+                acc = acc - v.x;
+                acc = acc - v.y;
+            }
+            sh.acc[lane] = acc;
+        }
+        __hip_atomic_store(&sh.folded, r + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    fetch();
+    for (unsigned r = 0; r < rounds; ++r) {
+        double cx = 0.0, cy = 0.0, cz = 0.0;
+        if (e < rows) {
+            if constexpr (ROOTS)
+                ref_contrib<ROLE>(xp, yp, zp, xe, ye, ze, xo, yo, zo, re, ro, rm, a.nu, nu_ok, cx, cy, cz);
+            else
+                ref_contrib<ROLE>(xp, yp, zp, xe, ye, ze, xo, yo, zo, a.nu, nu_ok, cx, cy, cz);
+            o += CH;
+            fetch();
+        }
+        const int b = r % AUTA_ROUNDS;
+        if (r >= AUTA_ROUNDS) wait_at_least(&sh.folded, r - AUTA_ROUNDS + 1);
+        sh.cb[b][3 * s + 0][t] = cx;
+        sh.cb[b][3 * s + 1][t] = cy;
+        sh.cb[b][3 * s + 2][t] = cz;
+        if (lane == 0) __hip_atomic_fetch_add(&sh.ready[b], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (r > 0 && wv == (int)((r - 1) % W)) fold(r - 1);
+    }
+    if (rounds > 0 && wv == (int)((rounds - 1) % W)) fold((unsigned)rounds - 1);
+    __syncthreads();
+    if (tid < 3 * S) {
+        const int q = p0 + tid / 3;
+        if (q < n) a.facc[(long long)(3 * ROLE + tid % 3) * n + q] = sh.acc[tid];
+    }
+    __syncthreads();
+}
+
+template <int W, int S, bool ROOTS>
+__global__ __launch_bounds__(WAVE * W, 4) void k_auta_exact(AutaExactDev a)
+{
+    __shared__ __attribute__((aligned(16))) AutaExactShared<W, S> sh;
+    const int p0 = (int)blockIdx.x * S;
+    auta_exact_role<0, W, S, ROOTS>(a, p0, sh);
+    auta_exact_role<1, W, S, ROOTS>(a, p0, sh);
+    auta_exact_role<2, W, S, ROOTS>(a, p0, sh);
+    if ((int)threadIdx.x < S && p0 + (int)threadIdx.x < a.n) {
+        const unsigned long long above = (unsigned long long)(a.n - 1 - (p0 + (int)threadIdx.x));
+        add_count(a.st, 0, above ? above * (above - 1) / 2 : 0ull);
+    }
 }
 
 // The same role streams over an owner list staged in LDS (sorted ids and
@@ -2258,12 +2305,7 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
             const double xa = L.p[3 * ia], ya = L.p[3 * ia + 1], za = L.p[3 * ia + 2];
             const double xb = L.p[3 * ib], yb = L.p[3 * ib + 1], zb = L.p[3 * ib + 2];
             double cx, cy, cz;
-            if constexpr (ROLE == 0)
-                ref_contrib<0>(xp, yp, zp, xa, ya, za, xb, yb, zb, nu, nu_ok, cx, cy, cz);
-            else if constexpr (ROLE == 1)
-                ref_contrib<1>(xa, ya, za, xp, yp, zp, xb, yb, zb, nu, nu_ok, cx, cy, cz);
-            else
-                ref_contrib<2>(xa, ya, za, xb, yb, zb, xp, yp, zp, nu, nu_ok, cx, cy, cz);
+            ref_contrib<ROLE>(xp, yp, zp, xa, ya, za, xb, yb, zb, nu, nu_ok, cx, cy, cz);
             sh.cb[lane * 3 + 0] = cx;
             sh.cb[lane * 3 + 1] = cy;
             sh.cb[lane * 3 + 2] = cz;
@@ -2356,8 +2398,9 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
 // again.
 constexpr int EXACT_GATHER = 4;  // candidates per lane and round
 
-// 5 waves per SIMD (at most 96 VGPRs): 4% faster than the 101-VGPR build.
-__global__ __launch_bounds__(WAVE, 5) void k_p3bca_exact(CutDev a)
+// 4 waves per SIMD: within 96 VGPRs, for a fifth, the brackets' reciprocals
+// spill (7.1 ms against 7.0 per 10 steps of N = 32768).
+__global__ __launch_bounds__(WAVE, 4) void k_p3bca_exact(CutDev a)
 {
     extern __shared__ __attribute__((aligned(16))) int sid_ex[];
     __shared__ ExactShared sh;
@@ -2755,14 +2798,20 @@ __global__ void k_selftest_fp64(long long n, const double *__restrict__ a, const
     rs[i] = __builtin_amdgcn_rsq(a[i]);
 }
 
-// The in-range sequences of the bit-exact path, element-wise.
+// The in-range sequences of the bit-exact path, element-wise.  The division
+// starts from a reciprocal that is off by 2^-46 on purpose, either way.
 __global__ void k_selftest_fp64_inrange(long long n, const double *__restrict__ a, const double *__restrict__ b,
                                         double *__restrict__ sq, double *__restrict__ q)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    sq[i] = sqrt_rn_inrange(a[i]);
-    q[i] = div_rn_inrange(a[i], b[i]);
+    double inv;
+    sq[i] = sqrt_rn_inrange(a[i], inv);
+    double r = __builtin_amdgcn_rcp(b[i]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) r = __builtin_fma(r, __builtin_fma(-b[i], r, 1.0), r);
+    r *= i & 1 ? 1.0 + 0x1p-46 : 1.0 - 0x1p-46;
+    q[i] = div_needs_ieee(low_word(b[i])) ? a[i] / b[i] : div_rn_from(a[i], b[i], r);
 }
 
 GridDev grid_dev(const CellGrid &g)
@@ -3139,7 +3188,7 @@ void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     hipLaunchKernelGGL(k_p3bca_exact, dim3(owner_grid(d.n)), dim3(WAVE), shm, s, a);
 }
 
-void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *st)
+void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *st, double2 *roots)
 {
     if (d.n <= 0) return;
     AutaExactDev a;
@@ -3150,7 +3199,16 @@ void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *s
     a.nu = nu;
     a.facc = d.facc;
     a.st = st;
-    hipLaunchKernelGGL(k_auta_exact, dim3((unsigned)(3 * d.n)), dim3(WAVE), 0, s, a);
+    a.roots = roots;
+    const dim3 blk(AUTA_WAVES * WAVE), grid2(blocks_for(d.n, 2)), grid4(blocks_for(d.n, 4));
+    if (roots) {
+        hipLaunchKernelGGL(k_pair_roots, dim3(blocks_for(d.n, 256), (unsigned)d.n), dim3(256), 0, s, d.n, d.x, d.y, d.z,
+                           roots);
+        if (d.n < 700) hipLaunchKernelGGL((k_auta_exact<AUTA_WAVES, 2, true>), grid2, blk, 0, s, a);
+        else hipLaunchKernelGGL((k_auta_exact<AUTA_WAVES, 4, true>), grid4, blk, 0, s, a);
+    } else {
+        hipLaunchKernelGGL((k_auta_exact<AUTA_WAVES, 4, false>), grid4, blk, 0, s, a);
+    }
 }
 
 // The j per block: 8 halve what a block of 4 shares again, but take 127
