@@ -91,3 +91,34 @@ def test_exact_all_triplets_past_the_pair_table(eng):
     size = np.linalg.norm(f, axis=1)
     floor = np.sqrt(np.mean(size ** 2))
     assert np.all(np.linalg.norm(f64 - f, axis=1) <= 2e-11 * np.maximum(size, floor))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,cutoff", [(5, 2.0), (129, 2.0), (400, 2.0), (500, 2.0), (1100, 2.0), (1728, 2.5),
+                                      (3375, 2.0), (3375, 2.5), (8000, 2.0)])
+def test_cutoff_cell_shapes(eng, oracle, n, cutoff, precision):
+    """One to 343 cells, so that a cell's owners are split among 16 down to 3
+    workgroups, in the narrow and (cutoff 2.5, or everything in one cell) the
+    wide shape of the cell kernel."""
+    P = jittered(n, 2000 + n)
+    L = np.full(3, 0.8 * np.ceil(round(n ** (1 / 3), 9)))
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=cutoff, domain_L=L, precision=precision)
+    check(eng, oracle, P, precision, cutoff=cutoff, L=L)
+
+
+def test_cutoff_wide_shape_found_by_the_sweep(eng, oracle):
+    """A system whose mean density asks for the narrow shape but whose dense
+    half needs the wide one: the pass is repeated, and a run goes on in it."""
+    rng = np.random.default_rng(11)
+    P = jittered(8000, 12)
+    keep = (P[:, 0] < 8.0) | (rng.random(8000) < 0.2)
+    P = P[keep]
+    L = np.full(3, 16.0)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=2.5, domain_L=L, precision="fp64")
+    check(eng, oracle, P, "fp64", cutoff=2.5, L=L)
+    eng.set_particles(P)
+    counts = eng.run(3, 1e-4)
+    eng.set_particles(P)
+    assert [eng.step(1e-4)[1] for _ in range(3)] == [int(c) for c in counts]

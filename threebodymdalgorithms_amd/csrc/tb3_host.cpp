@@ -155,6 +155,7 @@ struct tb3_ctx {
     long long scan_tmp_cap = 0;
     int list_cap = 128;    // LDS neighbour-list capacity per wave (power of two)
     bool cells_ok = true;  // the cell-per-workgroup kernel staged every neighbourhood so far
+    bool wide_need = false;  // some owner needed its wide shape (else: where the density makes that likely)
     bool dense_on = false;  // the dense-owner kernel follows the cell kernel (once some owner needed it)
     // the slotted cell layout of replayed steps (CellGrid::pad_cap): slots
     // per cell asked for (-1: three times the mean cell count, 0: off), and
@@ -201,6 +202,7 @@ struct tb3_ctx {
     int graph_cap = -1;
     bool graph_cells_ok = false;
     bool graph_dense_on = false;
+    bool graph_wide = false;
     int graph_slots = 0;  // the slots per cell the capture used (0: contiguous layout)
     unsigned long long *d_counts = nullptr;
     unsigned long long *h_counts = nullptr;  // pinned, counts_cap entries
@@ -370,6 +372,7 @@ void configure_grid(tb3_ctx *c)
     if (!same && g.cell_work && g.ncell <= c->grid_cell_cap)
         HIPCHK(hipMemset(g.cell_work, 0, (size_t)g.ncell * sizeof(unsigned)));
     c->cells_ok = true;  // a new grid gets a new chance at the cell kernel
+    c->wide_need = false;
     c->dense_on = false;
     c->slots_failed = false;
     if (!same) ++c->epoch;
@@ -494,6 +497,71 @@ int next_pow2(int v)
     return p;
 }
 
+// Whether the cell kernel of one system should start in its wide shape: from
+// the mean density, the particles within the cutoff of a cell's box that are
+// forward of it (all neighbours on a grid with a 3-cell dimension), and the
+// longest list (an owner in the corner nearest the forward cells sees ~85% of
+// its cutoff sphere), with room for the fluctuations of a uniform system,
+// against what the narrow shape stages (256) and lists (96).  A neighbourhood
+// the wide shape could not stage either stays with the narrow one, which
+// hands its owners on.  Systems that are not uniform find out from the sweep
+// (grow_after_overflow).
+// Both sides: the wide shape costs a system that does not need it 7-15% of
+// its sweep (N = 32768 125 against 118 us, N = 1048576 3.5 against 3.0 ms), a
+// sweep that leaves a few owners to the dense-owner kernel 15-25 us.  So up to
+// WIDE_CELLS cells (sweeps of ~200 us) the room is for the largest cell, past
+// it for all but a few percent of the owners.  Where many owners need it:
+// 8000 particles, cutoff 2.5, 126 us against 192 with the narrow shape.
+constexpr int WIDE_CELLS = 3000;
+bool wide_expected(const CellGrid &g, double cutoff, long long n)
+{
+    if (g.nrep > 1 || n < 3) return false;
+    double w[3], area = 1.0, box = 1.0, vol = 1.0;
+    int ext = 0;
+    bool three = false;
+    for (int k = 0; k < 3; ++k) {
+        const double wk = g.L[k] / g.nc[k];
+        vol *= g.L[k];
+        box *= wk;
+        three = three || g.nc[k] == 3;
+        if (g.nc[k] > 1) w[ext++] = wk;
+        else area *= wk;  // a dimension of one cell is not extended by the cutoff
+    }
+    const double c = cutoff, pi = 3.14159265358979;
+    double reach = box;
+    if (ext == 1) reach = (w[0] + 2 * c) * area;
+    else if (ext == 2) reach = (w[0] * w[1] + 2 * c * (w[0] + w[1]) + pi * c * c) * area;
+    else if (ext == 3)
+        reach = box + 2 * c * (w[0] * w[1] + w[1] * w[2] + w[0] * w[2]) + pi * c * c * (w[0] + w[1] + w[2]) +
+                4.0 / 3.0 * pi * c * c * c;
+    const double density = (double)n / vol;
+    const double staged = density * (three ? reach : 0.5 * (box + reach));
+    const double list = 0.85 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n);
+    if (staged > 416.0) return false;
+    const bool few = g.ncell <= WIDE_CELLS;
+    const double zs = few ? std::sqrt(2.0 * std::log(std::max(g.ncell, 2))) + 0.3 : 2.0, zl = few ? 4.0 : 2.5;
+    return staged + zs * std::sqrt(staged) > 256.0 || list + zl * std::sqrt(list) > 96.0;
+}
+
+bool cells_wide(const tb3_ctx *c, long long n) { return c->wide_need || wide_expected(c->grid, c->cutoff, n); }
+
+// Workgroups per cell: a grid whose cells do not fill the GPU's workgroup
+// slots (4 or, wide, 2 per CU) splits each cell's owners among several, which
+// each stage the cell's neighbourhood: just more workgroups than slots, down
+// to 2 owners each, and up to 16 parts, past which the parts' atomics on a
+// cell's few particles cost more (1 cell of 400: 16 parts 32 us, 64 48, 200
+// 101).  Kernel times at cutoff 2, density 2, with 1 and this many parts: 1
+// cell 181 -> 24 us, 64 cells 71 -> 27, 216 54 -> 30, 343 66 -> 43, 512 98 ->
+// 61, 729 86 -> 66, 1000 93 -> 85.  Past the slots a second staging costs more
+// than it spreads (1728 cells, 2 parts: 117 -> 135).
+int cell_parts(const tb3_ctx *c, int ncell, long long n, bool wide)
+{
+    const int slots = c->ncu * (wide ? 2 : 4);
+    if (ncell > slots || ncell <= 0) return 1;
+    const long long own = (n + ncell - 1) / ncell;
+    return (int)std::max<long long>(1, std::min<long long>({slots / ncell + 1, (own + 1) / 2, 16}));
+}
+
 // The n x n table of pair lengths that the bit-exact all-triplets sweep reads
 // (16 bytes a pair, 256 MiB at the most).  Without it (more particles, or no
 // memory) the sweep computes every length where it needs it.
@@ -536,8 +604,10 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
         if (fast_grad || energy) {
             const int slot = (exact && grad) ? 1 : 0;  // the exact pass owns count[0]
             if (cut && c->cells_ok) {
+                const bool wide = cells_wide(c, d.n);
                 launch_p3bca_cells(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
-                                   energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, slotted ? 1 : 0);
+                                   energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0,
+                                   cell_parts(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0);
                 if (c->dense_on)
                     launch_p3bca_dense(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                        energy ? 1 : 0, c->d_owners, c->dense_grid, c->dense_waves);
@@ -605,14 +675,16 @@ void launch_prepare(tb3_ctx *c, hipStream_t s, DeviceState &d, bool predict, dou
 
 // Re-runs an overflowed cutoff sweep with a larger LDS list capacity.  The
 // update kernel skipped itself, so the state is just after the predictor.
-bool grow_after_overflow(tb3_ctx *c)
+bool grow_after_overflow(tb3_ctx *c, long long n)
 {
     if (!c->h_status->flags[2]) return false;
     // a neighbourhood too large for the cell kernel's staging: use the
     // per-owner kernel for this particle system from now on
     if (c->h_status->flags[3]) c->cells_ok = false;
     // owners that need the dense-owner kernel: launch it from now on
-    if (c->h_status->want_dense) c->dense_on = true;
+    // (or, where its wide shape is enough, that)
+    if (c->h_status->want_dense == 1 && c->grid.ncell <= WIDE_CELLS && !cells_wide(c, n)) c->wide_need = true;
+    else if (c->h_status->want_dense) c->dense_on = true;
     const int need = c->h_status->flags[1];
     if (need > c->list_cap) {
         if (need > MAX_LIST)
@@ -642,7 +714,7 @@ void finish_overflowed(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate
                        bool grad, bool energy)
 {
     const bool exact = c->precision == TB3_FP64_EXACT;
-    for (int retry = 0; grow_after_overflow(c); ++retry) {
+    for (int retry = 0; grow_after_overflow(c, d.n); ++retry) {
         if (retry >= 8) throw Fail(TB3_EHIP, "the cutoff sweep kept overflowing its LDS staging");
         launch_reset_status(s, c->d_status, 1);  // keeps the non-finite flag of the binning pass
         if (grad && !exact) {
@@ -736,7 +808,8 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
     const int slots = slotted_steps(c) ? c->grid.pad_cap : 0;
     if (c->step_exec && c->graph_epoch == c->epoch && c->graph_dt == dt && c->graph_g[0] == g[0] &&
         c->graph_g[1] == g[1] && c->graph_g[2] == g[2] && c->graph_cap == c->list_cap &&
-        c->graph_cells_ok == c->cells_ok && c->graph_dense_on == c->dense_on && c->graph_fused == fused &&
+        c->graph_cells_ok == c->cells_ok && c->graph_dense_on == c->dense_on &&
+        c->graph_wide == cells_wide(c, c->n) && c->graph_fused == fused &&
         c->graph_slots == slots)
         return;
     if (c->step_exec) {
@@ -790,6 +863,7 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
     c->graph_cap = c->list_cap;
     c->graph_cells_ok = c->cells_ok;
     c->graph_dense_on = c->dense_on;
+    c->graph_wide = cells_wide(c, c->n);
 }
 
 // The last pass's accepted-triplet count, or per-replica counts for a batch.
@@ -1560,7 +1634,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
         // buffers replaced by the scratch array: the dense-owner kernel once
         // an owner needs it, the per-owner kernel with a growing list
         // capacity once a neighbourhood is too large for the cell kernel
-        bool cells = true, dense = false;
+        bool cells = true, dense = false, wide = wide_expected(g, c->cutoff, n);
         int cap = c->list_cap;
         Status h;
         for (int attempt = 0;; ++attempt) {
@@ -1572,7 +1646,8 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             }
             if (n >= 3) {
                 if (cells) {
-                    launch_p3bca_cells(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, dense ? 1 : 0);
+                    launch_p3bca_cells(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, dense ? 1 : 0, wide ? 1 : 0,
+                                       cell_parts(c, ncell, n, wide));
                     if (dense)
                         launch_p3bca_dense(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, c->dense_grid,
                                            c->dense_waves);
@@ -1586,7 +1661,8 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             if (!h.flags[2]) break;
             if (attempt >= 8) throw Fail(TB3_EHIP, "the cutoff sweep kept overflowing its LDS staging");
             if (h.flags[3]) cells = false;
-            if (h.want_dense) dense = true;
+            if (h.want_dense == 1 && ncell <= WIDE_CELLS && !wide) wide = true;
+            else if (h.want_dense) dense = true;
             if (!cells && h.flags[1] > cap) {
                 if (h.flags[1] > MAX_LIST)
                     throw Fail(TB3_EUNSUPPORTED, "a particle has " + std::to_string(h.flags[1]) +

@@ -101,7 +101,8 @@ struct Status {
                                   // neighbourhood (re-run with the per-owner kernel)
     int dqueue[2];                // owner queue of the dense-owner kernel; returns to zero after each launch
     int dense_n;                  // owners the cell kernel handed to the dense-owner kernel
-    int want_dense;               // the cell kernel had owners for a dense-owner kernel that was not launched
+    int want_dense;               // the cell kernel had owners for a dense-owner kernel that was not launched:
+                                  // 1 if its wide shape would take them all, 2 or 3 otherwise
     Slots *slots;                 // partial sums of the sweep kernels
     // Replayed step graphs (tb3_run): a step whose sweep overflowed sets
     // halt; every later replay then leaves the state and the flags alone
@@ -193,16 +194,18 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
                        int cap, int mixed, int grad, Status *st, int count_slot, int want_energy);
 void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int cap, Status *st);
-// Fast cutoff sweep with one workgroup per cell.  With
-// dense_on, owners it cannot stage go to `owners` for launch_p3bca_dense,
-// which must follow on the same stream; without, such an owner sets
-// st->want_dense and st->flags[2] (the caller re-runs the pass with the
-// dense-owner kernel).  Non-finite positions set st->flags[2] and [3]; the
-// caller then re-runs the sweep with launch_p3bca_fast.
+// Fast cutoff sweep, `parts` workgroups per cell, in the narrow or the wide
+// shape (4 waves, 256 staged particles and lists of 96; 8 waves, 416 and
+// 144).  With dense_on, owners it cannot stage go to `owners` for
+// launch_p3bca_dense, which must follow on the same stream; without, such an
+// owner sets st->want_dense and st->flags[2] (the caller re-runs the pass in
+// the wide shape or with the dense-owner kernel).  Non-finite positions set
+// st->flags[2] and [3]; the caller then re-runs the sweep with
+// launch_p3bca_fast.
 // `slotted`: sweep the slotted layout (needs dense_on == 0).
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int slotted = 0);
+                        int wide, int parts, int slotted = 0);
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
 int p3bca_cells_blocks_per_cu();
 // The cell kernel hands owners whose neighbourhood does not fit its LDS

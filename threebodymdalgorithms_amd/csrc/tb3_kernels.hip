@@ -1327,10 +1327,11 @@ __global__ __launch_bounds__(WAVE) void k_p3bca_fast(CutDev a)
 // received any.  The owners of a neighbourhood larger than NBCAP, and an
 // owner whose list is longer than LCAP, are queued for the dense-owner
 // kernel below instead.
+//
+// Few cells leave most of the chip without a workgroup; the grid's y then
+// splits each cell's owners among `parts` workgroups (part k takes owners k,
+// k + parts, ...), each with its own staging.
 
-constexpr int CELL_WAVES = 4;
-constexpr int NBCAP = 256;
-constexpr int LCAP = 96;   // list positions fit in the 8-bit halves of a queue entry
 constexpr int RQ = 128;    // per-wave queue of passing pairs (>= 2 x 64)
 
 struct CellsDev {
@@ -1344,12 +1345,22 @@ struct CellsDev {
     SlotsDev sl;          // the slotted layout (cap > 0: staged from its slot records)
 };
 
+// The two shapes of the cell kernel: waves of a workgroup, staged particles
+// and entries of a wave's list (list positions fit in the 8-bit halves of a
+// queue entry).  16 waves per CU either way: 34 KB of LDS, 4 workgroups of a
+// CU, or 82 KB, 2 of them, for neighbourhoods that the narrow one would leave
+// to one 8-wave workgroup per owner (k_p3bca_dense).
+template <bool WIDE>
+struct CellShape {
+    static constexpr int W = WIDE ? 8 : 4, NB = WIDE ? 416 : 256, LC = WIDE ? 144 : 96;
+};
+
 // An owner that needs the dense-owner kernel when none follows this launch:
 // the pass fails (the update skips itself) and asks the host for a re-run
-// with the dense-owner kernel.
-__device__ __forceinline__ void want_dense_kernel(Status *st)
+// in the wide shape, where that fits it, or with the dense-owner kernel.
+__device__ __forceinline__ void want_dense_kernel(Status *st, bool wide_fits)
 {
-    atomicOr(&st->want_dense, 1);
+    atomicOr(&st->want_dense, wide_fits ? 1 : 2);
     atomicOr(&st->flags[2], 1);
 }
 
@@ -1467,9 +1478,11 @@ __device__ __forceinline__ int cell_for_block(int b, int ncell, const int *order
     return order[r * cap + k];
 }
 
-template <class T, bool GRAD, bool WANT_E>
-__global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
+template <class T, bool GRAD, bool WANT_E, bool WIDE>
+__global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(CellsDev a)
 {
+    constexpr int CELL_WAVES = CellShape<WIDE>::W, NBCAP = CellShape<WIDE>::NB, LCAP = CellShape<WIDE>::LC;
+    const int part = blockIdx.y, parts = gridDim.y;
     // one block per array family, so that the y, z and gradient arrays sit
     // at constant offsets from x and their addresses fold into the LDS
     // instructions' immediate offsets
@@ -1501,7 +1514,7 @@ __global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
     if (a.sl.cap > 0) {
         const unsigned e = a.sl.state[0];
         scnt = a.sl.cnt + (e & 1u) * a.ncell;
-        if (tid == 0) a.sl.cnt[((e + 1u) & 1u) * a.ncell + c] = 0;
+        if (tid == 0 && part == 0) a.sl.cnt[((e + 1u) & 1u) * a.ncell + c] = 0;
         if (A.st->pad_over) {
             if (tid == 0) atomicOr(&A.st->flags[2], 1);  // the update kernel skips itself
             return;
@@ -1639,9 +1652,10 @@ __global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
     if (total > NBCAP) {
         // hand every owner of c to the dense-owner kernel (which makes c a
         // light workgroup: it goes last in the next sweep's order)
+        if (part > 0) return;
         if (tid == 0) a.cell_work[c] = 1;
         if (!a.dense_on) {
-            if (tid == 0) want_dense_kernel(A.st);
+            if (tid == 0) want_dense_kernel(A.st, total <= CellShape<true>::NB);
             return;
         }
         if (tid == 0) s_next = atomicAdd(&A.st->dense_n, own);
@@ -1661,7 +1675,7 @@ __global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
         for (;;) {
             int i = 0;
             if (lane == 0) i = atomicAdd(&s_next, 1);
-            i = __builtin_amdgcn_readfirstlane(i);
+            i = part + parts * __builtin_amdgcn_readfirstlane(i);
             if (i >= own) break;
             const double xi = nx[i], yi = ny[i], zi = nz[i];
 
@@ -1695,7 +1709,7 @@ __global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
                 // too long for this wave's list: the dense-owner kernel takes i
                 if (lane == 0) {
                     if (a.dense_on) a.owners[atomicAdd(&A.st->dense_n, 1)] = sinfo[0] + i;
-                    else want_dense_kernel(A.st);
+                    else want_dense_kernel(A.st, len <= CellShape<true>::LC);
                 }
                 continue;
             }
@@ -1835,7 +1849,7 @@ __global__ __launch_bounds__(CELL_WAVES *WAVE, 4) void k_p3bca_cells(CellsDev a)
         atomicAdd(&s_work, (unsigned)cw);
     }
     __syncthreads();
-    if (tid == 0) a.cell_work[c] = max(s_work, 1u);
+    if (tid == 0 && part == 0) a.cell_work[c] = max(s_work * (unsigned)parts, 1u);
 }
 
 
@@ -3066,7 +3080,7 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
 
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int slotted)
+                        int wide, int parts, int slotted)
 {
     if (d.n <= 0) return;
     CellsDev a;
@@ -3082,8 +3096,12 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     a.cell_work = g.cell_work;
     a.sl = slots_dev(&g, slotted);
     // the 8 XCDs' runs at their capacity (the workgroups past a run's length exit at once)
-    const dim3 gr((unsigned)(8 * cell_run_cap(g.ncell))), blk(CELL_WAVES * WAVE);
-#define TB3_CELLS(T, G, E) hipLaunchKernelGGL((k_p3bca_cells<T, G, E>), gr, blk, 0, s, a)
+    const dim3 gr((unsigned)(8 * cell_run_cap(g.ncell)), (unsigned)parts);
+#define TB3_CELLS(T, G, E)                                                                                \
+    do {                                                                                                  \
+        if (wide) hipLaunchKernelGGL((k_p3bca_cells<T, G, E, true>), gr, dim3(CellShape<true>::W * WAVE), 0, s, a); \
+        else hipLaunchKernelGGL((k_p3bca_cells<T, G, E, false>), gr, dim3(CellShape<false>::W * WAVE), 0, s, a);    \
+    } while (0)
     if (mixed) {
         if (grad) {
             if (want_energy) TB3_CELLS(float, true, true);
@@ -3106,8 +3124,8 @@ int p3bca_cells_blocks_per_cu()
 {
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb,
-                                                     reinterpret_cast<const void *>(k_p3bca_cells<double, true, false>),
-                                                     CELL_WAVES * WAVE, 0) != hipSuccess || nb < 1)
+                                                     reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, false>),
+                                                     CellShape<false>::W * WAVE, 0) != hipSuccess || nb < 1)
         nb = 1;
     return nb;
 }
