@@ -122,3 +122,31 @@ def test_cutoff_wide_shape_found_by_the_sweep(eng, oracle):
     counts = eng.run(3, 1e-4)
     eng.set_particles(P)
     assert [eng.step(1e-4)[1] for _ in range(3)] == [int(c) for c in counts]
+
+
+def test_single_passes_share_the_slots(eng, oracle):
+    """Single passes leave the slot counts ready for the next one: sweeps of
+    changing particle counts, with steps, a run, a non-finite position and a
+    crowded cell (more particles than slots) between them, each against the
+    oracle's count of the same positions."""
+    L = np.full(3, 0.8 * 12)
+    eng.set_particles(jittered(1700, 30))
+    eng.configure("p3bca", cutoff=2.0, domain_L=L, precision="fp64")
+    rng = np.random.default_rng(31)
+    crowded = np.concatenate([jittered(1500, 32), rng.uniform(4.1, 4.9, (60, 3))])
+    lost = jittered(300, 33)
+    lost[7] = np.nan
+    for P in (jittered(1700, 30), jittered(800, 34), crowded, jittered(1728, 35), lost, jittered(900, 36), crowded):
+        eng.set_particles(P)
+        *_, co = oracle.sweep(P, cutoff=2.0, L=L, mode="owner")
+        assert eng.compute_forces() == co
+        assert eng.energy()[1] == co
+        f = eng.get_particles()["f"]
+        assert eng.energy_grad()[3] == co
+        if np.all(np.isfinite(P)):
+            S = oracle.force_scale(P, cutoff=2.0, L=L)
+            assert np.all(np.linalg.norm(eng.get_particles()["f"] - f, axis=1) <= 1e-12 * S)
+        eng.set_particles(P)
+        assert eng.step(0.0)[1] == co
+        if np.all(np.isfinite(P)):
+            assert list(eng.run(3, 0.0)) == [co] * 3

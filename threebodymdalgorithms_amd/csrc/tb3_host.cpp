@@ -151,6 +151,7 @@ struct tb3_ctx {
     // cell grid of the cutoff algorithm
     CellGrid grid;
     int grid_cell_cap = 0, grid_n_cap = 0;
+    unsigned char *cell_block = nullptr, *list_block = nullptr, *slot_block = nullptr;  // what its arrays are in
     long long *scan_tmp = nullptr;
     long long scan_tmp_cap = 0;
     int list_cap = 128;    // LDS neighbour-list capacity per wave (power of two)
@@ -165,6 +166,14 @@ struct tb3_ctx {
     bool slots_failed = false;
     long long slot_buf_cap = 0;  // slot entries allocated
     int slot_cnt_cap = 0;        // slotted count entries allocated (2 ncell)
+    // between single passes on the slotted layout: the counts of the next
+    // pass's parity are zero (its predecessor's sweep cleared them)
+    bool slots_clean = false;
+    int slots_parity = 0;
+    // a single pass failed on a full slot since tb3_configure: single passes
+    // stay off the layout, also with other particles (a clustered system fails
+    // every time)
+    bool slots_distrust = false;
     int dense_grid = 1;    // persistent grid of the dense-owner kernel (workgroups that fit the GPU)
     int dense_waves = 8;   // waves per owner in the dense-owner kernel (tuned: 4, 8 or 16)
     int ncu = 1;           // compute units of the device
@@ -183,7 +192,8 @@ struct tb3_ctx {
     int pair_roots_cap = 0;
 
     Status *d_status = nullptr;
-    Status *h_status = nullptr;  // pinned
+    Status *h_status = nullptr;  // pinned; a pass's last kernel writes to it
+    bool status_clean = false;   // the device's block is clear for the next pass
     Slots *d_slots = nullptr;
 
     // the replayed step graph of tb3_run, and what its capture baked in
@@ -375,6 +385,7 @@ void configure_grid(tb3_ctx *c)
     c->wide_need = false;
     c->dense_on = false;
     c->slots_failed = false;
+    c->slots_clean = false;
     if (!same) ++c->epoch;
 }
 
@@ -395,32 +406,65 @@ void replica_domains(tb3_ctx *c, const double *rows)
     }
 }
 
+// Carves consecutive arrays, 256-byte aligned, out of one allocation.
+struct Carver {
+    unsigned char *base;
+    size_t off = 0;
+    template <class T>
+    void take(T *&p, long long count)
+    {
+        p = reinterpret_cast<T *>(base + off);
+        off += ((size_t)std::max<long long>(count, 1) * sizeof(T) + 255) & ~(size_t)255;
+    }
+};
+
+// The per-cell arrays of the current grid, zeroed when allocated.
+void ensure_cell_buffers(tb3_ctx *c)
+{
+    CellGrid &g = c->grid;
+    if (g.ncell <= c->grid_cell_cap) return;
+    ++c->epoch;
+    auto carve = [&](unsigned char *base) {
+        Carver v{base};
+        v.take(g.cell_cnt, g.ncell);
+        v.take(g.cell_start, (long long)g.ncell + 1);
+        v.take(g.order, cell_order_len(g.ncell));
+        v.take(g.cell_work, g.ncell);
+        v.take(g.scatter_ticket, 1);
+        return v.off;
+    };
+    const size_t bytes = carve(nullptr);
+    c->grid_cell_cap = 0;
+    dev_alloc(c->cell_block, (long long)bytes);
+    HIPCHK(hipMemset(c->cell_block, 0, bytes));
+    carve(c->cell_block);
+    c->grid_cell_cap = g.ncell;
+}
+
+// Those, and what the contiguous cell list of n particles needs.
 void ensure_grid_buffers(tb3_ctx *c, int n)
 {
     CellGrid &g = c->grid;
-    if (g.ncell > c->grid_cell_cap) {
-        ++c->epoch;
-        dev_alloc(g.cell_cnt, g.ncell);
-        HIPCHK(hipMemset(g.cell_cnt, 0, (size_t)g.ncell * sizeof(int)));
-        dev_alloc(g.cell_start, (long long)g.ncell + 1);
-        dev_alloc(g.order, cell_order_len(g.ncell));
-        dev_alloc(g.cell_work, g.ncell);
-        HIPCHK(hipMemset(g.cell_work, 0, (size_t)g.ncell * sizeof(unsigned)));
-        dev_alloc(g.scatter_ticket, 1);
-        HIPCHK(hipMemset(g.scatter_ticket, 0, sizeof(unsigned)));
-        c->grid_cell_cap = g.ncell;
-    }
+    ensure_cell_buffers(c);
     if (n > c->grid_n_cap) {
         ++c->epoch;
-        dev_alloc(c->d_owners, n);
-        dev_alloc(g.cell_of, n);
-        dev_alloc(g.cell_rank, n);
-        dev_alloc(g.cell_idx, n);
-        dev_alloc(g.xs, n);
-        dev_alloc(g.ys, n);
-        dev_alloc(g.zs, n);
+        auto carve = [&](unsigned char *base) {
+            Carver v{base};
+            v.take(c->d_owners, n);
+            v.take(g.cell_of, n);
+            v.take(g.cell_rank, n);
+            v.take(g.cell_idx, n);
+            v.take(g.xs, n);
+            v.take(g.ys, n);
+            v.take(g.zs, n);
+            return v.off;
+        };
+        c->grid_n_cap = 0;
+        dev_alloc(c->list_block, (long long)carve(nullptr));
+        carve(c->list_block);
         c->grid_n_cap = n;
     }
+    if (cells_fused_scan(g)) return;
     const long long need = scan_tmp_elems(std::max<long long>(n, g.ncell));
     if (need > c->scan_tmp_cap) {
         ++c->epoch;
@@ -453,17 +497,21 @@ void ensure_slot_buffers(tb3_ctx *c, int n)
     g.pad_cap = slots_for(c, n);
     if (g.pad_cap == 0) return;
     const long long need = (long long)g.ncell * g.pad_cap;
-    if (need > c->slot_buf_cap) {
-        ++c->epoch;
-        dev_alloc(g.pad_rec, need);
-        c->slot_buf_cap = need;
-    }
-    if (2 * g.ncell > c->slot_cnt_cap) {
-        ++c->epoch;
-        dev_alloc(g.pad_cnt, 2LL * g.ncell);
-        dev_alloc(g.pad_state, 2);
-        c->slot_cnt_cap = 2 * g.ncell;
-    }
+    if (need <= c->slot_buf_cap && 2 * g.ncell <= c->slot_cnt_cap) return;
+    ++c->epoch;
+    c->slots_clean = false;
+    auto carve = [&](unsigned char *base) {
+        Carver v{base};
+        v.take(g.pad_rec, need);
+        v.take(g.pad_cnt, 2LL * g.ncell);
+        v.take(g.pad_state, 2);
+        return v.off;
+    };
+    c->slot_buf_cap = c->slot_cnt_cap = 0;
+    dev_alloc(c->slot_block, (long long)carve(nullptr));
+    carve(c->slot_block);
+    c->slot_buf_cap = need;
+    c->slot_cnt_cap = 2 * g.ncell;
 }
 
 void ensure_triples(tb3_ctx *c, long long n)
@@ -583,11 +631,10 @@ void ensure_pair_roots(tb3_ctx *c, int n)
 // algorithm, on a cell list already built for them).
 //   grad   : dE/dx (the reference's f) into d.fx/fy/fz
 //   energy : E into the status block
-// The sweep of a pass.  With `tail` it ends with the role sum (exact path)
-// and the status fold; an integrating pass leaves both to launch_tail.
-// `slotted`: the cell kernel sweeps the slotted layout (replayed steps).
-void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool energy, bool tail,
-                  bool slotted = false)
+// launch_tail ends the pass.  `slotted`: the cell kernel sweeps the slotted
+// layout, of the given epoch parity in a single pass.
+void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool energy, bool slotted = false,
+                  int parity = -1)
 {
     const bool cut = uses_cutoff(c);
     const bool exact = c->precision == TB3_FP64_EXACT;
@@ -607,7 +654,7 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
                 const bool wide = cells_wide(c, d.n);
                 launch_p3bca_cells(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                    energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0,
-                                   cell_parts(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0);
+                                   cell_parts(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0, parity);
                 if (c->dense_on)
                     launch_p3bca_dense(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                        energy ? 1 : 0, c->d_owners, c->dense_grid, c->dense_waves);
@@ -620,55 +667,64 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
         }
     }
     if (c->recording) HIPCHK(hipEventRecord(c->ev[3], s));
-    if (tail) {
-        if (exact && grad && d.n >= 3) launch_sum_roles(s, d);
-        launch_finalize(s, c->d_status);
-    }
     HIPCHK(hipGetLastError());
 }
 
-// The end of an integrating pass after launch_sweep(..., tail = false): one
-// kernel for the role sum, the status fold and the update (and, in a step
-// graph, the count record and the status clear for the next replay).
-void launch_tail(tb3_ctx *c, hipStream_t s, DeviceState &d, double dt, const double *g, bool grad, bool record,
-                 bool slotted = false)
+// What a single pass reads and writes beside the state: positions (n x 3
+// device rows, or null: those held), and where its energy and forces go
+// (device memory, or null).
+struct PassIo {
+    const double *rows = nullptr;
+    double *energy = nullptr;
+    double *forces = nullptr;
+};
+
+// The end of a pass after launch_sweep, one kernel: the role sum, the status
+// fold and, in an integrating pass, the update.  A single pass (io) also
+// writes its results and publishes the status to the host; in a step graph
+// (no io) the step's count is recorded and the status cleared for the next
+// replay.
+void launch_tail(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate, double dt, const double *g, bool grad,
+                 const PassIo *io, bool slotted = false, int parity = -1)
 {
-    const bool sum_roles = c->precision == TB3_FP64_EXACT && grad && d.n >= 3;
-    const bool cells = uses_cutoff(c) && d.n >= 3 && c->grid.order;
-    launch_update_fin(s, d, dt * 0.5, g, c->d_status, sum_roles ? 1 : 0, record ? 1 : 0, cells ? &c->grid : nullptr,
-                      slotted ? 1 : 0);
+    const int sum_roles = c->precision == TB3_FP64_EXACT && grad && d.n >= 3 ? 1 : 0;
+    // past 8192 cells one workgroup would take longer to cut the XCDs' runs
+    // than they gain (64 000 cells: 117 us, of a sweep that fills the chip 60
+    // times over)
+    const CellGrid *cells = uses_cutoff(c) && d.n >= 3 && c->grid.order && cells_fused_scan(c->grid) ? &c->grid
+                                                                                                     : nullptr;
+    if (integrate)
+        launch_update_fin(s, d, dt * 0.5, g, c->d_status, sum_roles, io ? 0 : 1, cells, slotted ? 1 : 0, parity,
+                          io ? c->h_status : nullptr);
+    else
+        launch_finish(s, d, c->d_status, c->h_status, io->energy, sum_roles, io->forces, cells, slotted ? 1 : 0,
+                      parity);
     HIPCHK(hipGetLastError());
 }
 
-// Prepares a sweep over d: resets the status block (not inside a step
-// graph, whose previous replay, or k_begin_steps, cleared it), runs the
-// predictor when asked (fused into the binning pass for the cutoff
-// algorithm), zeroes the force where the sweep accumulates atomically and
-// builds the cell list.
-void launch_prepare(tb3_ctx *c, hipStream_t s, DeviceState &d, bool predict, double dt, bool grad,
-                    bool in_graph = false)
+// Prepares a sweep over d: the positions, the predictor when asked, the clear
+// force where the sweep accumulates atomically and the cell list, contiguous
+// or slotted, with everything else fused into its binning.
+void launch_prepare(tb3_ctx *c, hipStream_t s, DeviceState &d, const double *rows, bool predict, double dt, bool grad,
+                    bool in_graph = false, bool slotted = false, int parity = -1)
 {
     const bool cut = uses_cutoff(c);
     const bool exact = c->precision == TB3_FP64_EXACT;
     const bool zero_f = grad && (!exact || d.n < 3);
-    if (!in_graph) launch_reset_status(s, c->d_status, 0);
     if (c->recording) HIPCHK(hipEventRecord(c->ev[0], s));
     if (cut && d.n >= 3) {
         // the predictor is fused into the binning pass: its time is counted
         // with the cell-list phase
-        ensure_grid_buffers(c, d.n);
+        if (!slotted) ensure_grid_buffers(c, d.n);
         if (c->recording) HIPCHK(hipEventRecord(c->ev[1], s));
-        launch_cells_build(s, d, predict ? 1 : 0, dt, dt * dt * 0.5, zero_f ? 1 : 0, c->grid, c->d_status,
-                           c->scan_tmp);
+        if (slotted)
+            launch_bin_slotted(s, d, rows, predict ? 1 : 0, dt, zero_f ? 1 : 0, c->grid, c->d_status, parity);
+        else
+            launch_cells_build(s, d, rows, predict ? 1 : 0, dt, zero_f ? 1 : 0, c->grid, c->d_status, c->scan_tmp);
     } else {
         if (!cut && exact && grad && d.n >= 3 && !in_graph) ensure_pair_roots(c, d.n);
-        if (predict) launch_predict(s, d, dt, dt * dt * 0.5);
+        launch_start(s, d, rows, predict ? 1 : 0, dt, zero_f ? 1 : 0);
         if (c->recording) HIPCHK(hipEventRecord(c->ev[1], s));
-        if (zero_f) {
-            launch_zero(s, d.fx, d.n);
-            launch_zero(s, d.fy, d.n);
-            launch_zero(s, d.fz, d.n);
-        }
     }
     HIPCHK(hipGetLastError());
 }
@@ -709,45 +765,84 @@ void accumulate_profile(tb3_ctx *c, unsigned long long triplets, const float *pr
 }
 
 // Completes a pass whose sweep overflowed (the status block is on the host):
-// grows the capacity or switches kernels, then sweeps and updates again.
+// grows the capacity or switches kernels, then sweeps and updates again.  A
+// pass on the slotted layout gets the contiguous cell list of its positions
+// first (the counters of the contiguous binning are at zero); a cell that
+// outgrew its slots turns that layout off.
 void finish_overflowed(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate, double dt, const double *g,
-                       bool grad, bool energy)
+                       bool grad, bool energy, const PassIo &io, bool was_slotted)
 {
     const bool exact = c->precision == TB3_FP64_EXACT;
+    if (was_slotted && c->h_status->flags[2]) {
+        if (c->h_status->pad_over) c->slots_failed = c->slots_distrust = true;
+        c->slots_clean = false;
+        ensure_grid_buffers(c, d.n);
+        // keeps the non-finite flag of the binning pass, clears the halt
+        // (the scatter kernel skips halted replays)
+        launch_reset_status(s, c->d_status, 1);
+        launch_cells_build(s, d, nullptr, 0, dt, 0, c->grid, c->d_status, c->scan_tmp);
+    }
     for (int retry = 0; grow_after_overflow(c, d.n); ++retry) {
         if (retry >= 8) throw Fail(TB3_EHIP, "the cutoff sweep kept overflowing its LDS staging");
-        launch_reset_status(s, c->d_status, 1);  // keeps the non-finite flag of the binning pass
-        if (grad && !exact) {
-            launch_zero(s, d.fx, d.n);
-            launch_zero(s, d.fy, d.n);
-            launch_zero(s, d.fz, d.n);
-        }
-        launch_sweep(c, s, d, grad, energy, !integrate);
-        if (integrate) launch_tail(c, s, d, dt, g, grad, false);
+        launch_reset_status(s, c->d_status, 1);
+        if (grad && !exact) launch_start(s, d, nullptr, 0, 0.0, 1);
+        launch_sweep(c, s, d, grad, energy);
+        launch_tail(c, s, d, integrate, dt, g, grad, &io);
         if (c->recording) HIPCHK(hipEventRecord(c->ev[4], s));
-        read_status(c, s);
+        HIPCHK(hipStreamSynchronize(s));
     }
+}
+
+// Whether a single pass over n particles runs on the slotted layout (then
+// with its buffers in place): as replayed steps do, its binning fills the
+// slots itself and no scatter kernel runs.
+bool slotted_pass(tb3_ctx *c, int n)
+{
+    if (!uses_cutoff(c) || n < 3 || !cells_fused_scan(c->grid) || !c->cells_ok || c->dense_on ||
+        c->slots_distrust)
+        return false;
+    ensure_slot_buffers(c, n);
+    if (c->grid.pad_cap == 0) return false;
+    ensure_cell_buffers(c);
+    return true;
 }
 
 // One pass over d: optional predictor, sweep, optional update.  Handles the
 // neighbour-list overflow protocol and returns the accepted-triplet count.
+// The host waits once, for the pass's last kernel, which has then written the
+// results and the status to their places.
 unsigned long long run_pass(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate, double dt, const double *g,
-                            bool grad, bool energy, bool record)
+                            bool grad, bool energy, bool record, const PassIo &io = PassIo())
 {
     c->recording = record && c->prof;
     struct Reset {
         tb3_ctx *c;
         ~Reset() { c->recording = false; }
     } reset{c};
-    launch_prepare(c, s, d, integrate, dt, grad);
-    launch_sweep(c, s, d, grad, energy, !integrate);
-    if (integrate) launch_tail(c, s, d, dt, g, grad, false);
+    const bool slotted = slotted_pass(c, d.n);
+    if (slotted && !c->slots_clean) {
+        launch_begin_steps(s, c->d_status, c->d_counts, &c->grid);
+        c->slots_parity = 0;
+    } else if (!c->status_clean) {
+        launch_reset_status(s, c->d_status, 0);
+    }
+    c->status_clean = false;
+    const int parity = slotted ? c->slots_parity : -1;
+    if (slotted) c->slots_clean = false;  // until this pass has gone through
+    launch_prepare(c, s, d, io.rows, integrate, dt, grad, false, slotted, parity);
+    launch_sweep(c, s, d, grad, energy, slotted, parity);
+    launch_tail(c, s, d, integrate, dt, g, grad, &io, slotted, parity);
     if (c->recording) HIPCHK(hipEventRecord(c->ev[4], s));
-    read_status(c, s);
+    HIPCHK(hipStreamSynchronize(s));
     float prep[2] = {0.0f, 0.0f};
     if (c->recording)
         for (int k = 0; k < 2; ++k) HIPCHK(hipEventElapsedTime(&prep[k], c->ev[k], c->ev[k + 1]));
-    finish_overflowed(c, s, d, integrate, dt, g, grad, energy);
+    if (slotted) {
+        c->slots_parity ^= 1;
+        c->slots_clean = true;
+    }
+    finish_overflowed(c, s, d, integrate, dt, g, grad, energy, io, slotted);
+    c->status_clean = c->nrep <= 1;
     if (c->recording) accumulate_profile(c, c->h_status->count[0], prep);
     return c->h_status->count[0];
 }
@@ -832,7 +927,7 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
         const bool slotted = slots > 0;  // then the binning fills the slots and no scatter runs
         auto mid = [&] {
             if (!slotted) launch_scatter_fused(s, d, c->grid, c->d_status);
-            launch_sweep(c, s, d, true, false, false, slotted);
+            launch_sweep(c, s, d, true, false, slotted);
             launch_update_bin(s, d, dt * 0.5, g, c->d_status, exact ? 1 : 0, dt, dt * dt * 0.5, exact ? 0 : 1,
                               c->grid, slotted ? 1 : 0);
         };
@@ -845,14 +940,14 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
             });
         c->step_exec = capture(s, [&] {
             if (!slotted) launch_scatter_fused(s, d, c->grid, c->d_status);
-            launch_sweep(c, s, d, true, false, false, slotted);
-            launch_tail(c, s, d, dt, g, true, true, slotted);
+            launch_sweep(c, s, d, true, false, slotted);
+            launch_tail(c, s, d, true, dt, g, true, nullptr, slotted);
         });
     } else {
         c->step_exec = capture(s, [&] {
-            launch_prepare(c, s, d, true, dt, true, true);
-            launch_sweep(c, s, d, true, false, false);
-            launch_tail(c, s, d, dt, g, true, true);
+            launch_prepare(c, s, d, nullptr, true, dt, true, true);
+            launch_sweep(c, s, d, true, false);
+            launch_tail(c, s, d, true, dt, g, true, nullptr);
         });
     }
     c->graph_fused = fused;
@@ -914,16 +1009,16 @@ void run_steps_graph(tb3_ctx *c, int steps, double dt, const double *g, uint64_t
             else ensure_triples(c, d.n);
         }
         capture_step_graph(c, dt, g);
+        c->status_clean = c->slots_clean = false;
         launch_begin_steps(s, c->d_status, c->d_counts,
                            c->graph_fused && c->graph_slots > 0 ? &c->grid : nullptr);
         if (c->graph_fused) {
             // the first step's predictor and binning; each step_exec_mid
             // replay ends with the next step's
             if (c->graph_slots > 0) {
-                launch_bin_slotted(s, d, dt, dt * dt * 0.5, 1, c->grid, c->d_status);
+                launch_bin_slotted(s, d, nullptr, 1, dt, 1, c->grid, c->d_status);
             } else {
-                launch_bin_ranked(s, d, 1, dt, dt * dt * 0.5, c->precision == TB3_FP64_EXACT ? 0 : 1, c->grid,
-                                  c->d_status);
+                launch_bin_ranked(s, d, 1, dt, c->precision == TB3_FP64_EXACT ? 0 : 1, c->grid, c->d_status);
             }
             int k = done;
             // the middle steps in batches of 16, 8, 4, 2, then one
@@ -949,19 +1044,7 @@ void run_steps_graph(tb3_ctx *c, int steps, double dt, const double *g, uint64_t
         if (done < steps) {
             // step `done` overflowed: its predictor ran, its update did not
             if (!c->h_status->flags[2]) throw Fail(TB3_EHIP, "replayed steps halted without an overflow");
-            if (c->graph_fused && c->graph_slots > 0) {
-                // that step was binned into the slots: the host's sweeps
-                // below need its contiguous cell list (the counters of the
-                // contiguous binning are at zero, untouched by the slotted
-                // steps), built once the halt is cleared (the scatter
-                // kernel skips halted replays; the status read above keeps
-                // what the host needs); a cell that outgrew its slots turns
-                // the layout off
-                if (c->h_status->pad_over) c->slots_failed = true;
-                launch_reset_status(s, c->d_status, 1);
-                launch_cells_build(s, d, 0, dt, dt * dt * 0.5, 0, c->grid, c->d_status, c->scan_tmp);
-            }
-            finish_overflowed(c, s, d, true, dt, g, true, false);
+            finish_overflowed(c, s, d, true, dt, g, true, false, PassIo(), c->graph_fused && c->graph_slots > 0);
             if (counts) step_counts(c, counts + (size_t)done * per);
             ++done;
         }
@@ -1083,27 +1166,15 @@ tb3_status tb3_destroy(tb3_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     c->state.release();
     c->scratch.release();
-    dev_free(c->grid.cell_of);
-    dev_free(c->grid.cell_cnt);
-    dev_free(c->grid.cell_start);
-    dev_free(c->grid.order);
-    dev_free(c->grid.cell_work);
-    dev_free(c->grid.cell_rank);
-    dev_free(c->grid.scatter_ticket);
-    dev_free(c->grid.cell_idx);
-    dev_free(c->grid.xs);
-    dev_free(c->grid.ys);
-    dev_free(c->grid.zs);
-    dev_free(c->grid.pad_cnt);
-    dev_free(c->grid.pad_state);
-    dev_free(c->grid.pad_rec);
+    dev_free(c->cell_block);
+    dev_free(c->list_block);
+    dev_free(c->slot_block);
     dev_free(c->scan_tmp);
     dev_free(c->triples);
     dev_free(c->pair_roots);
     dev_free(c->d_status);
     dev_free(c->d_slots);
     dev_free(c->d_counts);
-    dev_free(c->d_owners);
     dev_free(c->grid.p_off);
     dev_free(c->grid.c_off);
     dev_free(c->grid.rnc);
@@ -1147,6 +1218,7 @@ tb3_status tb3_configure(tb3_ctx *c, int algo, double nu, double cutoff, const d
         c->nu = nu;
         c->cutoff = cutoff;
         c->precision = precision;
+        c->slots_distrust = false;
         c->user_L = domain_L != nullptr;
         if (domain_L) {
             for (int k = 0; k < 3; ++k) {
@@ -1298,16 +1370,8 @@ tb3_status tb3_batch_energy(tb3_ctx *c, int32_t nrep, double *E, uint64_t *count
     tb3_status st = check_ready(c);
     if (st != TB3_OK) return st;
     return guarded(c, [&] {
-        c->scratch.ensure(c->n);
-        DeviceState sd = c->scratch.d;
-        const DeviceState &d = c->state.d;
-        if (c->n > 0) {
-            const size_t b = (size_t)c->n * sizeof(double);
-            HIPCHK(hipMemcpyAsync(sd.x, d.x, b, hipMemcpyDeviceToDevice, c->stream));
-            HIPCHK(hipMemcpyAsync(sd.y, d.y, b, hipMemcpyDeviceToDevice, c->stream));
-            HIPCHK(hipMemcpyAsync(sd.z, d.z, b, hipMemcpyDeviceToDevice, c->stream));
-        }
-        run_pass(c, c->stream, sd, false, 0.0, nullptr, false, true, false);
+        // an energy pass leaves positions and forces alone
+        run_pass(c, c->stream, c->state.d, false, 0.0, nullptr, false, true, false);
         if (nrep > 1) {
             HIPCHK(hipMemcpy(E, c->grid.rep_energy, (size_t)nrep * sizeof(double), hipMemcpyDeviceToHost));
         } else {
@@ -1328,20 +1392,11 @@ tb3_status tb3_compute_forces(tb3_ctx *c, uint64_t *n_triplets)
     });
 }
 
-// The energy of the held positions at the configured nu, from a pass over a
-// copy of the positions so that the held force stays as it is.
-static double energy_on_copy(tb3_ctx *c, unsigned long long *count)
+// The energy of the held positions at the configured nu (an energy pass
+// leaves positions and forces alone).
+static double held_energy(tb3_ctx *c, unsigned long long *count)
 {
-    c->scratch.ensure(c->n);
-    DeviceState sd = c->scratch.d;
-    const DeviceState &d = c->state.d;
-    if (c->n > 0) {
-        const size_t b = (size_t)c->n * sizeof(double);
-        HIPCHK(hipMemcpyAsync(sd.x, d.x, b, hipMemcpyDeviceToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(sd.y, d.y, b, hipMemcpyDeviceToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(sd.z, d.z, b, hipMemcpyDeviceToDevice, c->stream));
-    }
-    const unsigned long long cnt = run_pass(c, c->stream, sd, false, 0.0, nullptr, false, true, false);
+    const unsigned long long cnt = run_pass(c, c->stream, c->state.d, false, 0.0, nullptr, false, true, false);
     if (count) *count = cnt;
     return c->h_status->energy;
 }
@@ -1366,10 +1421,10 @@ tb3_status tb3_force_scale(tb3_ctx *c, double *scale)
         HIPCHK(hipMemcpyAsync(sd.z, d.z, b, hipMemcpyDeviceToDevice, s));
         // the per-owner kernel with the list capacity grown until no list overflows
         for (int attempt = 0;; ++attempt) {
-            launch_prepare(c, s, sd, false, 0.0, false);
-            launch_zero(s, sd.fx, sd.n);
-            launch_zero(s, sd.fy, sd.n);
-            launch_zero(s, sd.fz, sd.n);
+            c->status_clean = false;
+            launch_reset_status(s, c->d_status, 0);
+            launch_prepare(c, s, sd, nullptr, false, 0.0, false);
+            launch_start(s, sd, nullptr, 0, 0.0, 1);
             if (sd.n >= 3)
                 launch_p3bca_fast(s, sd, c->grid, cutoff_spec(c), c->nu, c->list_cap, 0, 2, c->d_status, 0, 0);
             launch_finalize(s, c->d_status);
@@ -1393,7 +1448,7 @@ tb3_status tb3_energy(tb3_ctx *c, double *E, uint64_t *n_triplets)
     if (st != TB3_OK) return st;
     return guarded(c, [&] {
         unsigned long long cnt = 0;
-        *E = energy_on_copy(c, &cnt);
+        *E = held_energy(c, &cnt);
         if (n_triplets) *n_triplets = cnt;
     });
 }
@@ -1405,14 +1460,17 @@ tb3_status tb3_energy_grad(tb3_ctx *c, double *E, double *dEdx, double *dEdnu, u
     if (st != TB3_OK) return st;
     return guarded(c, [&] {
         DeviceState &d = c->state.d;
-        const unsigned long long cnt = run_pass(c, c->stream, d, false, 0.0, nullptr, true, true, false);
+        PassIo io;
+        if (dEdx && c->n > 0) {
+            c->scratch.ensure(c->n);
+            io.forces = c->scratch.d.facc;
+        }
+        const unsigned long long cnt = run_pass(c, c->stream, d, false, 0.0, nullptr, true, true, false, io);
         const double e = c->h_status->energy;
         if (E) *E = e;
         if (n_triplets) *n_triplets = cnt;
-        if (dEdx && c->n > 0) {
-            c->scratch.ensure(c->n);
-            launch_rows_from_soa(c->stream, (int)c->n, d.fx, d.fy, d.fz, c->scratch.d.facc);
-            HIPCHK(hipMemcpyAsync(dEdx, c->scratch.d.facc, (size_t)c->n * 3 * sizeof(double), hipMemcpyDeviceToHost,
+        if (io.forces) {
+            HIPCHK(hipMemcpyAsync(dEdx, io.forces, (size_t)c->n * 3 * sizeof(double), hipMemcpyDeviceToHost,
                                   c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
         }
@@ -1425,7 +1483,7 @@ tb3_status tb3_energy_grad(tb3_ctx *c, double *E, double *dEdx, double *dEdnu, u
                 c->nu = 1.0;
                 double e1 = 0.0;
                 try {
-                    e1 = energy_on_copy(c, nullptr);
+                    e1 = held_energy(c, nullptr);
                 } catch (...) {
                     c->nu = 0.0;
                     throw;
@@ -1451,7 +1509,6 @@ static tb3_status dev_common(tb3_ctx *c, int64_t n, const double *d_pos, double 
         c->scratch.ensure(n);
         DeviceState sd = c->scratch.d;
         sd.n = (int)n;
-        if (n > 0) launch_soa_from_rows(s, (int)n, d_pos, sd.x, sd.y, sd.z);
         if (uses_cutoff(c) && !c->have_L && n > 0) {
             std::vector<double> rows((size_t)(3 * n));
             HIPCHK(hipMemcpyAsync(rows.data(), d_pos, rows.size() * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1462,20 +1519,19 @@ static tb3_status dev_common(tb3_ctx *c, int64_t n, const double *d_pos, double 
         }
         const double saved_nu = c->nu;
         c->nu = nu;
+        PassIo io;
+        io.rows = n > 0 ? d_pos : nullptr;
+        io.energy = d_E;
+        io.forces = grad && n > 0 ? d_dEdx : nullptr;
         try {
-            run_pass(c, s, sd, false, 0.0, nullptr, grad, true, true);
+            run_pass(c, s, sd, false, 0.0, nullptr, grad, true, true, io);
         } catch (...) {
             c->nu = saved_nu;
             throw;
         }
         c->nu = saved_nu;
-        HIPCHK(hipMemcpyAsync(d_E, &c->d_status->energy, sizeof(double), hipMemcpyDeviceToDevice, s));
-        if (grad && n > 0) launch_rows_from_soa(s, (int)n, sd.fx, sd.fy, sd.fz, d_dEdx);
-        HIPCHK(hipGetLastError());
-        // both reads above use the context's status block and scratch, which
-        // the context's next call (on its own stream) clears and reuses:
-        // they complete before the call returns
-        HIPCHK(hipStreamSynchronize(s));
+        // the pass wrote E and the forces, and has completed: the context's
+        // status block and scratch are its next call's
         if (n_triplets) *n_triplets = c->h_status->count[0];
     });
 }
@@ -1625,8 +1681,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
                            g.cell_work, g.scatter_ticket, ncell);
         HIPCHK(hipGetLastError());
         if (n >= 3) {
-            launch_soa_from_rows(s, (int)n, d_pos, d.x, d.y, d.z);
-            launch_cells_build(s, d, 0, 0.0, 0.0, 1, g, l.st, l.scan_tmp);
+            launch_cells_build(s, d, d_pos, 0, 0.0, 1, g, l.st, l.scan_tmp);
         }
         const CutoffSpec cs = cutoff_spec(c);
         const int mixed = c->precision == TB3_FP32_MIXED ? 1 : 0;

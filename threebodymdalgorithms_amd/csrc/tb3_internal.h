@@ -137,17 +137,27 @@ void launch_begin_steps(hipStream_t s, Status *st, unsigned long long *counts, C
 // Folds the slot partial sums into st->count / st->energy and clears the
 // slots; sets st->halt when the sweep overflowed (st->flags[2]).
 void launch_finalize(hipStream_t s, Status *st);
-void launch_predict(hipStream_t s, const DeviceState &d, double dt, double h);
+// The last kernel of a pass without an update: the fold, the energy to e and
+// the status to the host's copy (pinned; the device's block is then clear for
+// the next pass, unless the sweep overflowed or replicas' sums are still to be
+// read), the role sum of the exact path and the forces to rows (e and rows
+// may be null), and the cuts of `cells` as below.
+void launch_finish(hipStream_t s, const DeviceState &d, Status *st, Status *host, double *e, int sum_roles,
+                   double *rows, const CellGrid *cells, int slotted = 0, int parity = -1);
+// The start of a pass: positions from rows (n x 3, or null: those held),
+// predictor, force clear.  launch_start is that alone, for a pass without a
+// cell list; the binning launches below include it.
+void launch_start(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f);
 // The last kernel of an integrating pass: launch_finalize's fold, then
 // a = g - f/m, v += a dt/2 (f = b0 + (b1 + b2) first with sum_roles), the
 // update skipped entirely when st->flags[2] (overflow) is set.  With record
 // (inside a replayed step graph) a step that did not halt also appends its
 // count to st->counts and clears the status block for the next replay.
 // With `cells` (a cell list this pass swept), one more workgroup cuts the
-// next sweep's XCD runs from the per-cell work.
+// next sweep's XCD runs from the per-cell work.  With host (a single pass)
+// the status is published as by launch_finish.
 void launch_update_fin(hipStream_t s, const DeviceState &d, double hdt, const double g[3], Status *st, int sum_roles,
-                       int record, const CellGrid *cells, int slotted = 0);
-void launch_sum_roles(hipStream_t s, const DeviceState &d);
+                       int record, const CellGrid *cells, int slotted = 0, int parity = -1, Status *host = nullptr);
 void launch_zero(hipStream_t s, double *p, long long count);
 
 // Exclusive scan of `count` int32 values into `out` (count + 1 entries, the
@@ -159,27 +169,29 @@ void launch_scan_i32(hipStream_t s, const int *in, int *out, int count, long lon
 // bin (+ predict, + zero f) -> scan -> scatter.  Nothing downstream depends
 // on the order within a cell: the fast sweep accumulates through atomics and
 // the exact sweep sorts each owner's list by index.
-void launch_cells_build(hipStream_t s, const DeviceState &d, int predict, double dt, double h, int zero_f,
+void launch_cells_build(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
                         CellGrid &g, Status *st, long long *tmp);
 // The two halves of launch_cells_build for grids that scan inside the
 // scatter kernel (cells_fused_scan): the binning (+ predictor, + force clear)
 // and the scan-and-scatter, which does nothing in a halted step-graph replay.
 bool cells_fused_scan(const CellGrid &g);
-void launch_bin_ranked(hipStream_t s, const DeviceState &d, int predict, double dt, double h, int zero_f,
-                       CellGrid &g, Status *st);
+void launch_bin_ranked(hipStream_t s, const DeviceState &d, int predict, double dt, int zero_f, CellGrid &g,
+                       Status *st);
 void launch_scatter_fused(hipStream_t s, const DeviceState &d, CellGrid &g, Status *st);
 // A replayed step's end fused with the next step's start (cells_fused_scan
 // grids): launch_update_fin's work with record, then the next step's
 // predictor, force clear (zero_f) and binning.
 void launch_update_bin(hipStream_t s, const DeviceState &d, double hdt, const double g3[3], Status *st,
                        int sum_roles, double dt, double h, int zero_f, CellGrid &g, int slotted = 0);
-// The slotted layout (CellGrid::pad_cap): launch_bin_slotted is a run's
-// first predictor (+ force clear) and binning into the slots, with the cell
-// order of the first sweep (after launch_begin_steps with the grid).
+// The slotted layout (CellGrid::pad_cap): launch_bin_slotted is the start of a
+// run or of a single pass and its binning into the slots, with the cell
+// order of the sweep (after launch_begin_steps with the grid).
 // launch_update_bin and launch_update_fin with `slotted` read and fill the
 // slotted counts instead (and order the next sweep's cells themselves).
-void launch_bin_slotted(hipStream_t s, const DeviceState &d, double dt, double h, int zero_f, CellGrid &g,
-                        Status *st);
+// `parity`: of the epoch, in single passes; -1 in a run, whose kernels keep
+// the epoch on the device.
+void launch_bin_slotted(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
+                        CellGrid &g, Status *st, int parity = -1);
 
 // Cutoff sweeps (P3BCA).  One wave per particle builds that particle's
 // neighbour list in LDS (capacity `cap`) from the cell list; a list longer
@@ -205,7 +217,7 @@ void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, 
 // `slotted`: sweep the slotted layout (needs dense_on == 0).
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, int parts, int slotted = 0);
+                        int wide, int parts, int slotted = 0, int parity = -1);
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
 int p3bca_cells_blocks_per_cu();
 // The cell kernel hands owners whose neighbourhood does not fit its LDS

@@ -208,6 +208,29 @@ __device__ void fold_slots(Status *st)
     }
 }
 
+// A folded status block to the host's copy (pinned memory, which the kernel's
+// end makes visible), where the host waits for the pass's last kernel alone
+// instead of a copy behind it; then, unless the pass is to be repeated or the
+// per-replica sums are still to be read, the block cleared for the next pass.
+__device__ __forceinline__ void publish_status(Status *st, Status *host, int t, int nt)
+{
+    __syncthreads();  // the fold
+    const bool over = st->flags[2] != 0;
+    if (t == 0) {
+        host->count[0] = st->count[0];
+        host->count[1] = st->count[1];
+        host->energy = st->energy;
+        for (int k = 0; k < 4; ++k) host->flags[k] = st->flags[k];
+        host->want_dense = st->want_dense;
+        host->pad_over = st->pad_over;
+    }
+    __syncthreads();
+    if (!over && st->nrep <= 1) {
+        clear_status(st, false, t, nt);
+        if (t == 0) st->halt = 0;
+    }
+}
+
 __global__ __launch_bounds__(NSLOT) void k_finalize(Status *st) { fold_slots(st); }
 
 // Particle::UpdatePredictorStage (utility/structs.hpp:40-55):
@@ -217,19 +240,52 @@ __device__ __forceinline__ double predicted(double x, double v, double aX, doubl
     return x + v * dt + aX * h;
 }
 
-__device__ __forceinline__ void predict_one(const DeviceState &d, int p, double dt, double h)
+// Particle p's position at the start of a pass: read from the caller's rows
+// (n x 3, kept in the state's arrays) or the state, moved by the predictor.
+struct PassStart {
+    const double *rows;  // or null
+    int predict;
+    double dt, h;
+    int zero_f;  // clear the force for a sweep that adds to it
+};
+
+__device__ __forceinline__ void start_particle(const DeviceState &d, const PassStart &a, int p, bool predict,
+                                               double &px, double &py, double &pz)
 {
-    const double aX = d.ax[p];
-    d.x[p] = predicted(d.x[p], d.vx[p], aX, dt, h);
-    d.y[p] = predicted(d.y[p], d.vy[p], aX, dt, h);
-    d.z[p] = predicted(d.z[p], d.vz[p], aX, dt, h);
+    if (a.rows) {
+        px = a.rows[3 * (long long)p + 0];
+        py = a.rows[3 * (long long)p + 1];
+        pz = a.rows[3 * (long long)p + 2];
+    } else {
+        px = d.x[p];
+        py = d.y[p];
+        pz = d.z[p];
+    }
+    if (predict) {
+        const double aX = d.ax[p];
+        px = predicted(px, d.vx[p], aX, a.dt, a.h);
+        py = predicted(py, d.vy[p], aX, a.dt, a.h);
+        pz = predicted(pz, d.vz[p], aX, a.dt, a.h);
+    }
+    if (predict || a.rows) {
+        d.x[p] = px;
+        d.y[p] = py;
+        d.z[p] = pz;
+    }
+    if (a.zero_f) {
+        d.fx[p] = 0.0;
+        d.fy[p] = 0.0;
+        d.fz[p] = 0.0;
+    }
 }
 
-__global__ void k_predict(DeviceState d, double dt, double h)
+// The start of a pass without a cell list.
+__global__ void k_start(DeviceState d, PassStart a)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= d.n) return;
-    predict_one(d, p, dt, h);
+    double px, py, pz;
+    start_particle(d, a, p, a.predict != 0, px, py, pz);
 }
 
 // The dispatch order of the cell kernel (see cell_run_cap), for it to start
@@ -367,6 +423,9 @@ struct SlotsDev {
     int *cnt;         // 2 ncell counts, by epoch parity
     unsigned *state;  // [0] epoch, [1] finished workgroups of a binning pass
     double4 *rec;     // ncell cap slots: x, y, z, and the particle index's bits in w
+    int parity;       // of the epoch, in single passes (the host counts them); -1: read the epoch from state
+
+    __device__ __forceinline__ unsigned epoch() const { return parity >= 0 ? (unsigned)parity : state[0]; }
 };
 
 // Particle p (position px, py, pz) into a slot of cell c, counted in cnt; a
@@ -395,6 +454,63 @@ __device__ __forceinline__ void slots_ticket(const SlotsDev &sl, unsigned e)
     if (threadIdx.x == 0 && atomicInc(&sl.state[1], gridDim.x - 1) == gridDim.x - 1) sl.state[0] = e + 1;
 }
 
+// The workgroup that cuts the next sweep's XCD runs from this sweep's
+// per-cell work (and cell counts, contiguous or slotted).
+__device__ void cuts_workgroup(int ncell, const int *__restrict__ cell_start, const unsigned *__restrict__ cell_work,
+                               int *__restrict__ order, const SlotsDev &sl)
+{
+    __shared__ float fpart[4];
+    __shared__ int cut[9];
+    int *out = order + 8 * cell_run_cap(ncell) + 8;
+    if (sl.cap > 0) {
+        const int *cur = sl.cnt + (sl.epoch() & 1u) * ncell;
+        compute_cuts(ncell, [&](int c) { return min(cur[c], sl.cap); }, cell_work, out, fpart, cut);
+    } else {
+        compute_cuts(ncell, [&](int c) { return cell_start[c + 1] - cell_start[c]; }, cell_work, out, fpart, cut);
+    }
+}
+
+// The last kernel of a pass without an update: workgroup 0 folds the status,
+// stores the energy (e, may be null) and publishes the status, the next
+// (with a cell list, ncell > 0) cuts the XCD runs of the next sweep, the
+// others take the particles' role sums (exact path; SumUpParticles,
+// Algorithm.cpp:245-249) and forces to rows (may be null).
+__global__ __launch_bounds__(NSLOT) void k_finish(DeviceState d, Status *st, Status *host, double *e, int sum_roles,
+                                                  double *rows, int ncell, const int *__restrict__ cell_start,
+                                                  const unsigned *__restrict__ cell_work, int *__restrict__ order,
+                                                  SlotsDev sl)
+{
+    if (blockIdx.x == 0) {
+        fold_slots(st);
+        if (threadIdx.x == 0 && e) *e = st->energy;
+        publish_status(st, host, threadIdx.x, NSLOT);
+        return;
+    }
+    const int extra = ncell > 0 ? 2 : 1;
+    if ((int)blockIdx.x < extra) {
+        cuts_workgroup(ncell, cell_start, cell_work, order, sl);
+        return;
+    }
+    const int p = ((int)blockIdx.x - extra) * NSLOT + threadIdx.x;
+    if (p >= d.n) return;
+    double fx, fy, fz;
+    if (sum_roles) {
+        const long long n = d.n;
+        d.fx[p] = fx = d.facc[0 * n + p] + (d.facc[3 * n + p] + d.facc[6 * n + p]);
+        d.fy[p] = fy = d.facc[1 * n + p] + (d.facc[4 * n + p] + d.facc[7 * n + p]);
+        d.fz[p] = fz = d.facc[2 * n + p] + (d.facc[5 * n + p] + d.facc[8 * n + p]);
+    } else {
+        fx = d.fx[p];
+        fy = d.fy[p];
+        fz = d.fz[p];
+    }
+    if (rows) {
+        rows[3 * (long long)p + 0] = fx;
+        rows[3 * (long long)p + 1] = fy;
+        rows[3 * (long long)p + 2] = fz;
+    }
+}
+
 // The last kernel of an integrating pass.  Workgroup 0 first folds the
 // sweep's slot sums into the status block (k_finalize); with `record` (a
 // replayed step graph) it then appends the step's count and, unless the
@@ -409,7 +525,7 @@ __global__ __launch_bounds__(NSLOT) void k_update_fin(DeviceState d, double hdt,
                                                      Status *st, int sum_roles, int record, int ncell,
                                                      const int *__restrict__ cell_start,
                                                      const unsigned *__restrict__ cell_work, int *__restrict__ order,
-                                                     SlotsDev sl)
+                                                     SlotsDev sl, Status *host)
 {
     // The particles' workgroups, then (with a cell list, ncell > 0) one that
     // cuts the next sweep's XCD runs from this sweep's per-cell work (and
@@ -430,19 +546,11 @@ __global__ __launch_bounds__(NSLOT) void k_update_fin(DeviceState d, double hdt,
             clear_status(st, false, t, NSLOT);
             if (t == 0) st->nstep = ns + 1;
         }
+        if (host) publish_status(st, host, threadIdx.x, NSLOT);
         return;
     }
     if (x == 0) {
-        __shared__ float fpart[4];
-        __shared__ int cut[9];
-        int *out = order + 8 * cell_run_cap(ncell) + 8;
-        if (sl.cap > 0) {
-            const int *cur = sl.cnt + (sl.state[0] & 1u) * ncell;
-            compute_cuts(ncell, [&](int c) { return min(cur[c], sl.cap); }, cell_work, out, fpart, cut);
-        } else {
-            compute_cuts(ncell, [&](int c) { return cell_start[c + 1] - cell_start[c]; }, cell_work, out, fpart,
-                         cut);
-        }
+        cuts_workgroup(ncell, cell_start, cell_work, order, sl);
         return;
     }
     // The fold's clear happens only when flags[2] is already zero, so every
@@ -472,17 +580,6 @@ __global__ __launch_bounds__(NSLOT) void k_update_fin(DeviceState d, double hdt,
     d.ax[p] = a0;
     d.ay[p] = a1;
     d.az[p] = a2;
-}
-
-// Algorithm::SumUpParticles (Algorithm.cpp:245-249): f = b0 + (b1 + b2).
-__global__ void k_sum_roles(DeviceState d)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= d.n) return;
-    const long long n = d.n;
-    d.fx[p] = d.facc[0 * n + p] + (d.facc[3 * n + p] + d.facc[6 * n + p]);
-    d.fy[p] = d.facc[1 * n + p] + (d.facc[4 * n + p] + d.facc[7 * n + p]);
-    d.fz[p] = d.facc[2 * n + p] + (d.facc[5 * n + p] + d.facc[8 * n + p]);
 }
 
 __global__ void k_zero(double *p, long long count)
@@ -650,27 +747,14 @@ __device__ __forceinline__ void cell_of_pos(const SysGrid &g, double x, double y
 }
 
 template <bool RANK>
-__global__ void k_bin(DeviceState d, int predict, double dt, double h, int zero_f, GridDev g,
-                      int *__restrict__ cell_of, int *__restrict__ cell_cnt, int *__restrict__ cell_rank, Status *st)
+__global__ void k_bin(DeviceState d, PassStart a, GridDev g, int *__restrict__ cell_of, int *__restrict__ cell_cnt,
+                      int *__restrict__ cell_rank, Status *st)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= d.n) return;
-    // the predicted position stays in registers for the binning below
-    double px = d.x[p], py = d.y[p], pz = d.z[p];
-    if (predict && !st->halt) {
-        const double aX = d.ax[p];
-        px = predicted(px, d.vx[p], aX, dt, h);
-        py = predicted(py, d.vy[p], aX, dt, h);
-        pz = predicted(pz, d.vz[p], aX, dt, h);
-        d.x[p] = px;
-        d.y[p] = py;
-        d.z[p] = pz;
-    }
-    if (zero_f) {
-        d.fx[p] = 0.0;
-        d.fy[p] = 0.0;
-        d.fz[p] = 0.0;
-    }
+    // the position stays in registers for the binning below
+    double px, py, pz;
+    start_particle(d, a, p, a.predict && !st->halt, px, py, pz);
     if (!finite3(px, py, pz)) atomicOr(&st->flags[0], 1);
     const SysGrid sg = grid_of_particle(g, p);
     int cx, cy, cz;
@@ -700,13 +784,14 @@ __global__ __launch_bounds__(256) void k_begin_steps_slotted(Status *st, unsigne
     }
 }
 
-// The first step of a slotted run: predictor, force clear and binning of
-// k_bin<true>, into the slots of the current epoch; 8 more workgroups order
-// the first sweep's cells from the cuts the last integrating pass stored
-// (the counts fill beside them, so cells never swept weigh alike).
-__global__ __launch_bounds__(256) void k_bin_slotted(DeviceState d, double dt, double h, int zero_f, GridDev g,
-                                                     SlotsDev sl, Status *st, int ncell,
-                                                     const unsigned *__restrict__ cell_work, int *__restrict__ order)
+// The first step of a slotted run, or a single pass on the slotted layout:
+// the start of a pass and the binning of k_bin<true>, into the slots of the
+// current epoch; 8 more workgroups order the sweep's cells from the cuts the
+// last integrating pass stored (the counts fill beside them, so cells never
+// swept weigh alike).
+__global__ __launch_bounds__(256) void k_bin_slotted(DeviceState d, PassStart a, GridDev g, SlotsDev sl, Status *st,
+                                                     int ncell, const unsigned *__restrict__ cell_work,
+                                                     int *__restrict__ order)
 {
     const int nbin = (int)gridDim.x - 8;
     if ((int)blockIdx.x >= nbin) {
@@ -720,24 +805,14 @@ __global__ __launch_bounds__(256) void k_bin_slotted(DeviceState d, double dt, d
     }
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= d.n) return;
-    const double aX = d.ax[p];
-    const double px = predicted(d.x[p], d.vx[p], aX, dt, h);
-    const double py = predicted(d.y[p], d.vy[p], aX, dt, h);
-    const double pz = predicted(d.z[p], d.vz[p], aX, dt, h);
-    d.x[p] = px;
-    d.y[p] = py;
-    d.z[p] = pz;
-    if (zero_f) {
-        d.fx[p] = 0.0;
-        d.fy[p] = 0.0;
-        d.fz[p] = 0.0;
-    }
+    double px, py, pz;
+    start_particle(d, a, p, a.predict != 0, px, py, pz);
     if (!finite3(px, py, pz)) atomicOr(&st->flags[0], 1);
     const SysGrid sg = grid_of_particle(g, p);
     int cx, cy, cz;
     cell_of_pos(sg, px, py, pz, cx, cy, cz);
     const int c = sg.cbase + (cz * sg.nc[1] + cy) * sg.nc[0] + cx;
-    bin_slotted(sl, sl.cnt + (sl.state[0] & 1u) * ncell, c, p, px, py, pz, st);
+    bin_slotted(sl, sl.cnt + (sl.epoch() & 1u) * ncell, c, p, px, py, pz, st);
 }
 
 // One particle of k_update_bin: update, predictor, force clear, binning
@@ -1512,7 +1587,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     // on the contiguous layout.
     const int *scnt = nullptr;
     if (a.sl.cap > 0) {
-        const unsigned e = a.sl.state[0];
+        const unsigned e = a.sl.epoch();
         scnt = a.sl.cnt + (e & 1u) * a.ncell;
         if (tid == 0 && part == 0) a.sl.cnt[((e + 1u) & 1u) * a.ncell + c] = 0;
         if (A.st->pad_over) {
@@ -2875,9 +2950,10 @@ CutDev cut_dev(const DeviceState &d, const CellGrid &g, const CutoffSpec &c, dou
 }
 
 // The slotted layout's device view (cap 0 when off).
-SlotsDev slots_dev(const CellGrid *g, int on)
+SlotsDev slots_dev(const CellGrid *g, int on, int parity = -1)
 {
     SlotsDev v{};
+    v.parity = parity;
     if (on && g && g->pad_cap > 0) {
         v.cap = g->pad_cap;
         v.cnt = g->pad_cnt;
@@ -2932,14 +3008,29 @@ void launch_begin_steps(hipStream_t s, Status *st, unsigned long long *counts, C
 
 void launch_finalize(hipStream_t s, Status *st) { hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NSLOT), 0, s, st); }
 
-void launch_predict(hipStream_t s, const DeviceState &d, double dt, double h)
+void launch_finish(hipStream_t s, const DeviceState &d, Status *st, Status *host, double *e, int sum_roles,
+                   double *rows, const CellGrid *cells, int slotted, int parity)
 {
-    if (d.n <= 0) return;
-    hipLaunchKernelGGL(k_predict, dim3(blocks_for(d.n, 256)), dim3(256), 0, s, d, dt, h);
+    const unsigned nb = 1 + (cells ? 1 : 0) + ((sum_roles || rows) && d.n > 0 ? blocks_for(d.n, NSLOT) : 0);
+    hipLaunchKernelGGL(k_finish, dim3(nb), dim3(NSLOT), 0, s, d, st, host, e, sum_roles, rows,
+                       cells ? cells->ncell : 0, cells ? cells->cell_start : nullptr,
+                       cells ? cells->cell_work : nullptr, cells ? cells->order : nullptr,
+                       slots_dev(cells, slotted && cells, parity));
+}
+
+static PassStart pass_start(const double *rows, int predict, double dt, int zero_f)
+{
+    return PassStart{rows, predict, dt, dt * dt * 0.5, zero_f};
+}
+
+void launch_start(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f)
+{
+    if (d.n <= 0 || !(rows || predict || zero_f)) return;
+    hipLaunchKernelGGL(k_start, dim3(blocks_for(d.n, 256)), dim3(256), 0, s, d, pass_start(rows, predict, dt, zero_f));
 }
 
 void launch_update_fin(hipStream_t s, const DeviceState &d, double hdt, const double g[3], Status *st, int sum_roles,
-                       int record, const CellGrid *cells, int slotted)
+                       int record, const CellGrid *cells, int slotted, int parity, Status *host)
 {
     // the particles' workgroups, then (with a cell list) one that cuts the
     // next sweep's XCD runs, and one that folds the status
@@ -2947,13 +3038,7 @@ void launch_update_fin(hipStream_t s, const DeviceState &d, double hdt, const do
     hipLaunchKernelGGL(k_update_fin, dim3(nb), dim3(NSLOT), 0, s, d, hdt, g[0], g[1], g[2], st, sum_roles, record,
                        cells ? cells->ncell : 0, cells ? cells->cell_start : nullptr,
                        cells ? cells->cell_work : nullptr, cells ? cells->order : nullptr,
-                       slots_dev(cells, slotted && cells));
-}
-
-void launch_sum_roles(hipStream_t s, const DeviceState &d)
-{
-    if (d.n <= 0) return;
-    hipLaunchKernelGGL(k_sum_roles, dim3(blocks_for(d.n, 256)), dim3(256), 0, s, d);
+                       slots_dev(cells, slotted && cells, parity), host);
 }
 
 void launch_zero(hipStream_t s, double *p, long long count)
@@ -2981,12 +3066,12 @@ void launch_scan_i32(hipStream_t s, const int *in, int *out, int count, long lon
 
 bool cells_fused_scan(const CellGrid &g) { return g.ncell <= FUSED_SCAN_CELLS; }
 
-void launch_bin_ranked(hipStream_t s, const DeviceState &d, int predict, double dt, double h, int zero_f,
-                       CellGrid &g, Status *st)
+void launch_bin_ranked(hipStream_t s, const DeviceState &d, int predict, double dt, int zero_f, CellGrid &g,
+                       Status *st)
 {
     if (d.n <= 0) return;
-    hipLaunchKernelGGL(k_bin<true>, dim3(blocks_for(d.n, 256)), dim3(256), 0, s, d, predict, dt, h, zero_f,
-                       grid_dev(g), g.cell_of, g.cell_cnt, g.cell_rank, st);
+    hipLaunchKernelGGL(k_bin<true>, dim3(blocks_for(d.n, 256)), dim3(256), 0, s, d,
+                       pass_start(nullptr, predict, dt, zero_f), grid_dev(g), g.cell_of, g.cell_cnt, g.cell_rank, st);
 }
 
 void launch_scatter_fused(hipStream_t s, const DeviceState &d, CellGrid &g, Status *st)
@@ -3009,31 +3094,29 @@ void launch_update_bin(hipStream_t s, const DeviceState &d, double hdt, const do
                        g.cell_work, g.order, slots_dev(&g, slotted));
 }
 
-void launch_bin_slotted(hipStream_t s, const DeviceState &d, double dt, double h, int zero_f, CellGrid &g,
-                        Status *st)
+void launch_bin_slotted(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
+                        CellGrid &g, Status *st, int parity)
 {
     // the particles' workgroups, then 8 that order the first sweep's cells
     const unsigned nb = (d.n > 0 ? blocks_for(d.n, 256) : 0) + 8;
-    hipLaunchKernelGGL(k_bin_slotted, dim3(nb), dim3(256), 0, s, d, dt, h, zero_f, grid_dev(g), slots_dev(&g, 1),
-                       st, g.ncell, g.cell_work, g.order);
+    hipLaunchKernelGGL(k_bin_slotted, dim3(nb), dim3(256), 0, s, d, pass_start(rows, predict, dt, zero_f), grid_dev(g),
+                       slots_dev(&g, 1, parity), st, g.ncell, g.cell_work, g.order);
 }
 
-void launch_cells_build(hipStream_t s, const DeviceState &d, int predict, double dt, double h, int zero_f,
+void launch_cells_build(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
                         CellGrid &g, Status *st, long long *tmp)
 {
     const int n = d.n;
+    const PassStart a = pass_start(rows, predict, dt, zero_f);
     if (n > 0 && g.ncell <= FUSED_SCAN_CELLS) {
-        hipLaunchKernelGGL(k_bin<true>, dim3(blocks_for(n, 256)), dim3(256), 0, s, d, predict, dt, h, zero_f,
-                           grid_dev(g), g.cell_of, g.cell_cnt, g.cell_rank, st);
-        const int nsc = blocks_for(n, 256);
-        hipLaunchKernelGGL(k_cell_scatter_fused, dim3(nsc + 8), dim3(256), 0, s, n, d.x, d.y, d.z, g.cell_of,
-                           g.cell_rank, g.cell_cnt, g.cell_start, g.cell_idx, g.xs, g.ys, g.zs, g.ncell, g.order,
-                           g.cell_work, g.scatter_ticket, nsc, st);
+        hipLaunchKernelGGL(k_bin<true>, dim3(blocks_for(n, 256)), dim3(256), 0, s, d, a, grid_dev(g), g.cell_of,
+                           g.cell_cnt, g.cell_rank, st);
+        launch_scatter_fused(s, d, g, st);
         return;
     }
     if (n > 0)
-        hipLaunchKernelGGL(k_bin<false>, dim3(blocks_for(n, 256)), dim3(256), 0, s, d, predict, dt, h, zero_f,
-                           grid_dev(g), g.cell_of, g.cell_cnt, nullptr, st);
+        hipLaunchKernelGGL(k_bin<false>, dim3(blocks_for(n, 256)), dim3(256), 0, s, d, a, grid_dev(g), g.cell_of,
+                           g.cell_cnt, nullptr, st);
     launch_scan_i32(s, g.cell_cnt, g.cell_start, g.ncell, tmp);
     if (n > 0)
         hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, d.x, d.y, d.z, g.cell_of,
@@ -3080,7 +3163,7 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
 
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, int parts, int slotted)
+                        int wide, int parts, int slotted, int parity)
 {
     if (d.n <= 0) return;
     CellsDev a;
@@ -3094,7 +3177,7 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     a.owners = owners;
     a.order = g.order;
     a.cell_work = g.cell_work;
-    a.sl = slots_dev(&g, slotted);
+    a.sl = slots_dev(&g, slotted, parity);
     // the 8 XCDs' runs at their capacity (the workgroups past a run's length exit at once)
     const dim3 gr((unsigned)(8 * cell_run_cap(g.ncell)), (unsigned)parts);
 #define TB3_CELLS(T, G, E)                                                                                \
