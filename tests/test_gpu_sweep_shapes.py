@@ -150,3 +150,19 @@ def test_single_passes_share_the_slots(eng, oracle):
         assert eng.step(0.0)[1] == co
         if np.all(np.isfinite(P)):
             assert list(eng.run(3, 0.0)) == [co] * 3
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [300, 520, 900])
+def test_dense_owner_lists(eng, oracle, n, precision):
+    """Lists of the dense-owner kernel of one up to 15 blocks of r, even and
+    odd lengths: n sites of a grid with spacing 0.8 scaled by 0.3, so that
+    (almost) all are within the cutoff of each other, in a box of 5 cells
+    that leaves the pair tests plain, and in one whose periodic images count."""
+    P = 0.3 * jittered(n, 3000 + n)
+    for box, shift in ((20.0, 10.0), (6.6, 5.8)):
+        Q = P + shift
+        L = np.full(3, box)
+        eng.set_particles(Q)
+        eng.configure("p3bca", cutoff=2.0, domain_L=L, precision=precision)
+        check(eng, oracle, Q, precision, cutoff=2.0, L=L)

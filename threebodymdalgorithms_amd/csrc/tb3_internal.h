@@ -221,14 +221,13 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
 int p3bca_cells_blocks_per_cu();
 // The cell kernel hands owners whose neighbourhood does not fit its LDS
-// staging to this kernel (one owner per workgroup, lists of up to
-// p3bca_dense_cap() particles); owners beyond that set st->flags[2] and [3]
+// staging to this kernel (one owner per workgroup, lists of up to 1440
+// particles); owners beyond that set st->flags[2] and [3]
 // like the cell kernel's own overflow.  `owners` holds n ints.  Call
 // p3bca_dense_setup once per device before the first launch (it sets the
 // kernel's LDS limit, which a captured graph cannot).
 // `waves` (4, 8 or 16) is the workgroup size per owner in waves.
 void p3bca_dense_setup();
-int p3bca_dense_cap();
 bool p3bca_dense_waves_ok(int waves);
 int p3bca_dense_blocks_per_cu(int waves);
 void launch_p3bca_dense(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,

@@ -1936,12 +1936,25 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
 // kernel would have used (its own cell's later slots, then the forward
 // neighbour cells, within the cutoff), gathered from the cell-ordered
 // positions into LDS by all waves; the list's unordered pairs are then split
-// over the workgroup's lanes in folded order and evaluated in place as in
-// the cell kernel.  A list longer than DCAP raises the overflow flags (the
-// host then re-runs the sweep with the per-owner kernel).
-
-constexpr int DCAP = 1440;  // two workgroups of 4 or 8 waves (one of 16) fit a CU's 160 KB of LDS
-
+// over the workgroup's waves in folded order, pair (r, (r + o) mod len) for
+// o = 1 .. len / 2, tested, queued where they pass and evaluated 64 at a time
+// as in the cell kernel.  A list longer than DCAP raises the overflow flags
+// (the host then re-runs the sweep with the per-owner kernel).
+//
+// Bound by LDS (busy 70% of the time, most of it the six FP64 atomics of a
+// triplet) beside 53% VALU issue; before, by waiting (59% VALU).  So
+//  * the chain of round trips from a ticket to its owner's cells, which every
+//    wave waited for, is walked by one wave for the next owner while the
+//    others are at this one's pairs (claimed from a counter, so that nobody
+//    waits for that wave);
+//  * a wave takes a block of up to 64 consecutive r and a range of o: r stays
+//    in registers, a test reads one position instead of two, and takes the
+//    plain form where the list is compact (17 instructions instead of 35).
+// Kernel times: 48 Gaussian replicas of up to 2048 particles 1615 -> 1490 us,
+// 64 of up to 4096 8.2 -> 7.2 ms, 20000 particles at density 2.2 and cutoff
+// 2.7 (lists of 91) 511 -> 470 us.  Evaluating every tested pair in place
+// with the coefficients masked (half of them pass) has no LDS conflicts but
+// 25% more VALU work: 1550, 7.2, 507.
 struct DenseDev {
     CutDev c;
     const double *xs, *ys, *zs;
@@ -1950,18 +1963,25 @@ struct DenseDev {
     int *queue;  // [0] next owner ticket, [1] finished workgroups (both return to 0)
 };
 
+constexpr int DCAP = 1440;  // two workgroups of 4 or 8 waves (one of 16) fit a CU's 160 KB of LDS
+
 size_t dense_lds() { return (size_t)DCAP * (6 * sizeof(double) + sizeof(int)); }
 
 template <class T, bool GRAD, int DW>
-__global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
+__global__ __launch_bounds__(DW *WAVE, 4) void k_p3bca_dense(DenseDev a)
 {
     extern __shared__ double dsm[];
     double *qx = dsm, *qy = qx + DCAP, *qz = qy + DCAP;
     double *hx = qz + DCAP, *hy = hx + DCAP, *hz = hy + DCAP;
     int *qid = reinterpret_cast<int *>(hz + DCAP);
-    __shared__ int cst[32], cpre[33], sinfo[4];
-    __shared__ int s_item, s_len;
-    __shared__ double s_gi[3];
+    // the owner in hand and, fetched while its pairs are walked, the next
+    struct Owner {
+        int item, slot, p, rep;
+        int cst[32], cpre[33], info[4];
+        double L[3];
+    };
+    __shared__ Owner own[2];
+    __shared__ int s_len, s_far, s_unit;
     __shared__ unsigned dring[DW][RQ];
 
     const CutDev &A = a.c;
@@ -1972,39 +1992,57 @@ __global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
     const int nowners = A.st->halt ? 0 : A.st->dense_n;  // written by the cell kernel before this launch
     if (nowners == 0) return;                            // the common case: no queue traffic at all
     double esum = 0.0;
-    unsigned cnt = 0;
+    unsigned cnt = 0;  // this wave's triplets, in every lane
     bool overflow = false;
 
-    for (;;) {
-        if (tid == 0) s_item = atomicAdd(&a.queue[0], 1);
-        __syncthreads();
-        const int item = s_item;
-        if (item >= nowners) break;
-        const int slot = a.owners[item];
-        const int p = A.cell_idx[slot];
-        const int c = a.cell_of[p];
-        const SysGrid sg = grid_of_cell(A.g, c);
-        const double Lx = sg.L[0], Ly = sg.L[1], Lz = sg.L[2];
-        if (wv == 0) stage_cells(A, sg, c, cst, cpre, sinfo);
-        if (tid == 0) {
-            s_len = 0;
-            s_gi[0] = s_gi[1] = s_gi[2] = 0.0;
+    // wave 0: the next ticket, and its owner's cells (a chain of dependent
+    // memory round trips, a fifth of an owner's time when every wave waited
+    // for it)
+    auto fetch = [&](Owner &w) {
+        int item = 0;
+        if (lane == 0) item = atomicAdd(&a.queue[0], 1);
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item < nowners) {
+            const int slot = a.owners[item];
+            const int p = A.cell_idx[slot];
+            const int c = a.cell_of[p];
+            const SysGrid sg = grid_of_cell(A.g, c);
+            stage_cells(A, sg, c, w.cst, w.cpre, w.info);
+            if (lane == 0) {
+                w.slot = slot;
+                w.p = p;
+                w.rep = sg.r;
+                for (int k = 0; k < 3; ++k) w.L[k] = sg.L[k];
+            }
         }
+        if (lane == 0) w.item = item;
+    };
+    if (wv == 0) fetch(own[0]);
+    if (tid == 0) s_len = s_far = s_unit = 0;
+
+    for (int b = 0;; b ^= 1) {
         __syncthreads();
-        const int i = slot - sinfo[0], nk = sinfo[2], total = sinfo[3];
+        const Owner &w = own[b];
+        if (w.item >= nowners) break;
+        const double Lx = w.L[0], Ly = w.L[1], Lz = w.L[2];
+        const int slot = w.slot, i = slot - w.info[0], nk = w.info[2], total = w.info[3];
         const double xi = a.xs[slot], yi = a.ys[slot], zi = a.zs[slot];
 
-        // the owner's forward list
+        // the owner's forward list; when all of it lies within 0.24 L of the
+        // owner in every dimension, any two entries differ by less than L / 2
+        // and the pair tests take the plain form
+        bool far = false;
         for (int t0 = i + 1; t0 < total; t0 += NT) {
             const int t = t0 + tid;
             bool ok = t < total;
             double xt = 0.0, yt = 0.0, zt = 0.0;
             int st = 0;
             if (ok) {
-                st = staged_slot(cst, cpre, nk, t);
+                st = staged_slot(w.cst, w.cpre, nk, t);
                 xt = a.xs[st];
                 yt = a.ys[st];
                 zt = a.zs[st];
+                st = A.cell_idx[st];
                 ok = !(sqr_dist_periodic_min(xi, yi, zi, xt, yt, zt, Lx, Ly, Lz) > c2);
             }
             const unsigned long long m = __ballot(ok);
@@ -2013,29 +2051,26 @@ __global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
             base = __shfl(base, 0);
             const int pos = base + lane_prefix(m);
             if (ok && pos < DCAP) {
+                far = far || !(__builtin_fabs(xt - xi) <= 0.24 * Lx && __builtin_fabs(yt - yi) <= 0.24 * Ly &&
+                               __builtin_fabs(zt - zi) <= 0.24 * Lz);
                 qx[pos] = xt;
                 qy[pos] = yt;
                 qz[pos] = zt;
                 hx[pos] = 0.0;
                 hy[pos] = 0.0;
                 hz[pos] = 0.0;
-                qid[pos] = A.cell_idx[st];
+                qid[pos] = st;
             }
         }
+        if (far) s_far = 1;
         __syncthreads();
         const int len = s_len;
-        if (len > DCAP) {
-            overflow = true;
-            __syncthreads();
-            continue;
-        }
+        const bool periodic = s_far != 0, fits = len <= DCAP;
+        if (!fits) overflow = true;
+        if (wv == 0) fetch(own[b ^ 1]);
 
-        // the list's unordered pairs, folded, split over the workgroup's
-        // lanes; each wave queues its passing pairs and evaluates them 64 at
-        // a time (as the cell kernel does)
-        double gix = 0.0, giy = 0.0, giz = 0.0;
-        const int npairs = len * (len - 1) / 2;
-        if (npairs > 0) {
+        auto pairs = [&](auto per) {
+            constexpr bool PER = decltype(per)::value;
             unsigned *rq = dring[wv];
             int head = 0, qw = 0;
             auto flush = [&](int nq) {
@@ -2055,9 +2090,6 @@ __global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
                     T et;
                     at_coeffs_from64<T, GRAD>(u64, v64, w64, nu, K, cu, cv, cw, et);
                     if (GRAD) {
-                        gix = __builtin_fma(-cu, djx, __builtin_fma(-cv, dkx, gix));
-                        giy = __builtin_fma(-cu, djy, __builtin_fma(-cv, dky, giy));
-                        giz = __builtin_fma(-cu, djz, __builtin_fma(-cv, dkz, giz));
                         // the j and k terms share the products cw * e: (-cw) e = -(cw e) exactly
                         const double tx = cw * ex, ty = cw * ey, tz = cw * ez;
                         lds_add(&hx[r], __builtin_fma(cu, djx, -tx));
@@ -2068,73 +2100,80 @@ __global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
                         lds_add(&hz[kk], __builtin_fma(cv, dkz, tz));
                     }
                     esum += (double)et;
-                    ++cnt;
                 }
                 wave_sync();
+                cnt += (unsigned)nq;
                 head = (head + nq) & (RQ - 1);
                 qw -= nq;
             };
-            const int qn = NT / len, rn = NT - qn * len;
-            int o = tid / len;
-            int r = tid - o * len;
-            ++o;
-            for (int t0 = 0; t0 < npairs; t0 += NT) {
-                bool ok = false;
-                int kk = 0;
-                if (t0 + tid < npairs) {
-                    kk = r + o;
-                    kk = kk >= len ? kk - len : kk;
-                    ok = !(sqr_dist_periodic_min(qx[r], qy[r], qz[r], qx[kk], qy[kk], qz[kk], Lx, Ly, Lz) > c2);
-                }
-                const unsigned long long m = __ballot(ok);
-                if (ok) rq[(head + qw + lane_prefix(m)) & (RQ - 1)] = (unsigned)r | ((unsigned)kk << 16);
-                qw += __popcll(m);
-                if (qw >= WAVE) flush(WAVE);
-                r += rn;
-                o += qn;
-                if (r >= len) {
-                    r -= len;
-                    ++o;
+            const int H = len >> 1;                       // for even len, o = H takes half of the r
+            const int nb = (len + WAVE - 1) / WAVE, bw = (len + nb - 1) / nb;
+            const int nch = min(H, (4 * DW + nb - 1) / nb), och = (H + nch - 1) / nch;
+            for (;;) {
+                int unit = 0;
+                if (lane == 0) unit = atomicAdd(&s_unit, 1);
+                unit = __builtin_amdgcn_readfirstlane(unit);
+                if (unit >= nb * nch) break;
+                const int r0 = unit % nb * bw + lane;
+                const int o0 = 1 + unit / nb * och, o1 = min(o0 + och, H + 1);
+                const bool live = lane < bw && r0 < len;
+                const int r = live ? r0 : 0;
+                const double xr = qx[r], yr = qy[r], zr = qz[r];
+                int kk = r + o0;
+                kk = kk >= len ? kk - len : kk;
+                for (int o = o0; o < o1; ++o) {
+                    bool ok = live && !(cut_sq<PER>(xr, yr, zr, qx[kk], qy[kk], qz[kk], Lx, Ly, Lz) > c2);
+                    if (2 * o == len) ok = ok && r < H;
+                    const unsigned long long m = __ballot(ok);
+                    if (ok) rq[(head + qw + lane_prefix(m)) & (RQ - 1)] = (unsigned)r | ((unsigned)kk << 16);
+                    qw += __popcll(m);
+                    if (qw >= WAVE) flush(WAVE);
+                    ++kk;
+                    kk = kk == len ? 0 : kk;
                 }
             }
             if (qw > 0) flush(qw);
-        }
-        if (GRAD) {
-            gix = wave_total(gix);
-            giy = wave_total(giy);
-            giz = wave_total(giz);
-            if (lane == 0) {
-                lds_add(&s_gi[0], gix);
-                lds_add(&s_gi[1], giy);
-                lds_add(&s_gi[2], giz);
-            }
+        };
+        if (fits && len > 1) {
+            if (periodic) pairs(std::true_type{});
+            else pairs(std::false_type{});
         }
         __syncthreads();
-        if (GRAD) {
+        if (tid == 0) s_len = s_far = s_unit = 0;
+        if (GRAD && fits) {
+            // the owner's gradient is minus the list's sum
+            double gix = 0.0, giy = 0.0, giz = 0.0;
             for (int t = tid; t < len; t += NT) {
                 const int q = qid[t];
-                unsafeAtomicAdd(&A.fx[q], hx[t]);
-                unsafeAtomicAdd(&A.fy[q], hy[t]);
-                unsafeAtomicAdd(&A.fz[q], hz[t]);
+                const double gx = hx[t], gy = hy[t], gz = hz[t];
+                unsafeAtomicAdd(&A.fx[q], gx);
+                unsafeAtomicAdd(&A.fy[q], gy);
+                unsafeAtomicAdd(&A.fz[q], gz);
+                gix -= gx;
+                giy -= gy;
+                giz -= gz;
             }
-            if (tid == 0) {
-                unsafeAtomicAdd(&A.fx[p], s_gi[0]);
-                unsafeAtomicAdd(&A.fy[p], s_gi[1]);
-                unsafeAtomicAdd(&A.fz[p], s_gi[2]);
+            if (wv * WAVE < len) {
+                gix = wave_total(gix);
+                giy = wave_total(giy);
+                giz = wave_total(giz);
+                if (lane == 0) {
+                    unsafeAtomicAdd(&A.fx[w.p], gix);
+                    unsafeAtomicAdd(&A.fy[w.p], giy);
+                    unsafeAtomicAdd(&A.fz[w.p], giz);
+                }
             }
         }
         if (A.g.nrep > 1) {
-            const unsigned long long cc = wave_sum_u64(cnt);
             const double ee = A.want_energy ? wave_sum(esum) : 0.0;
             if (lane == 0) {
                 if (A.want_energy) add_energy(A.st, ee);
-                add_count(A.st, A.count_slot, cc);
-                add_rep(A, sg.r, cc, ee);
+                add_count(A.st, A.count_slot, cnt);
+                add_rep(A, w.rep, cnt, ee);
             }
             cnt = 0;
             esum = 0.0;
         }
-        __syncthreads();
     }
 
     if (overflow && tid == 0) {
@@ -2142,10 +2181,9 @@ __global__ __launch_bounds__(DW *WAVE) void k_p3bca_dense(DenseDev a)
         atomicOr(&A.st->flags[3], 1);
     }
     if (A.want_energy) esum = wave_sum(esum);
-    const unsigned long long cw = wave_sum_u64(cnt);
     if (lane == 0) {
         if (A.want_energy) add_energy(A.st, esum);
-        add_count(A.st, A.count_slot, cw);
+        add_count(A.st, A.count_slot, cnt);
     }
     __syncthreads();
     if (tid == 0) {
@@ -3214,8 +3252,9 @@ int p3bca_cells_blocks_per_cu()
 }
 
 template <int DW>
-void dense_setup_waves(size_t shm)
+void dense_setup_waves()
 {
+    const size_t shm = dense_lds();
     allow_lds(k_p3bca_dense<double, true, DW>, shm);
     allow_lds(k_p3bca_dense<double, false, DW>, shm);
     allow_lds(k_p3bca_dense<float, true, DW>, shm);
@@ -3224,13 +3263,10 @@ void dense_setup_waves(size_t shm)
 
 void p3bca_dense_setup()
 {
-    const size_t shm = dense_lds();
-    dense_setup_waves<4>(shm);
-    dense_setup_waves<8>(shm);
-    dense_setup_waves<16>(shm);
+    dense_setup_waves<4>();
+    dense_setup_waves<8>();
+    dense_setup_waves<16>();
 }
-
-int p3bca_dense_cap() { return DCAP; }
 
 bool p3bca_dense_waves_ok(int waves) { return waves == 4 || waves == 8 || waves == 16; }
 
