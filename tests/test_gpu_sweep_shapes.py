@@ -166,3 +166,18 @@ def test_dense_owner_lists(eng, oracle, n, precision):
         eng.set_particles(Q)
         eng.configure("p3bca", cutoff=2.0, domain_L=L, precision=precision)
         check(eng, oracle, Q, precision, cutoff=2.0, L=L)
+
+
+@pytest.mark.parametrize("n,spacing", [(4, 0.8), (30, 0.8), (300, 0.8), (700, 0.5), (1400, 0.34), (1400, 0.27)])
+def test_exact_cutoff_list_lengths(eng, oracle, n, spacing):
+    """Bit for bit with lists of a few entries up to past 1024, where they
+    stop holding the sides to the owner (33, 65, 130, 270, ~800, ~1300
+    neighbours), so that every sort and both forms of the list run."""
+    P = jittered(n, 4000 + n, spacing=spacing, sd=0.06 * spacing)
+    L = np.full(3, 12.0)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=2.0, domain_L=L, precision="exact")
+    cnt = eng.compute_forces()
+    *_, fo, co = oracle.sweep(P, cutoff=2.0, L=L, mode="owner")
+    assert cnt == co
+    assert np.array_equal(eng.get_particles()["f"], fo)

@@ -2214,8 +2214,8 @@ __global__ __launch_bounds__(DW *WAVE, 4) void k_p3bca_dense(DenseDev a)
 // algorithm, implicit (every other particle) otherwise.
 
 struct ExactShared {
-    int qa[RING], qb[RING];
-    double cb[WAVE * 3];
+    int q[RING];              // accepted pairs: list positions, 16 bits each
+    double cb[3][WAVE + 2];   // x, y, z contributions of 64 items; rows padded against bank conflicts
 };
 
 // NATA / AUTA (every triplet).  A workgroup of W waves takes S consecutive
@@ -2390,10 +2390,14 @@ __global__ __launch_bounds__(WAVE * W, 4) void k_auta_exact(AutaExactDev a)
 // pairs enter the queue in item order, which is the stream order, so the
 // fold below adds the contributions exactly as the nested loops did.
 struct StagedList {
-    const double *p;  // entry t at p[3t], p[3t + 1], p[3t + 2] (x, y, z side by side: two LDS reads)
+    const double *p;        // entry t at p[3t], p[3t + 1], p[3t + 2] (x, y, z side by side: two LDS reads)
+    const double2 *root;    // ROOTS: the entry's side to the owner (ref_root)
 };
 
-template <int ROLE>
+// ROOTS: an item's two sides to the owner are read from the list instead of
+// computed from the positions for each of the ~31 triplets that an entry of
+// an average list is in.
+template <int ROLE, bool ROOTS>
 __device__ void exact_role_staged(const StagedList &L, double xp, double yp, double zp, int len, int split,
                                   bool plain, double c2, double Lx, double Ly, double Lz, double nu, ExactShared &sh,
                                   double &acc, unsigned long long &accepted)
@@ -2415,31 +2419,45 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
         m = split;
         m2 = 0;
     }
-    // Item numbers and row starts fit an int (lists hold at most 5851
-    // entries: 160 KB of LDS).  Up to 2048 entries (64 KB) they and
-    // (2m - 1)^2 stay below 2^24, exact in FP32, so the row estimates below
-    // are off by less than 0.001; on longer lists the correction loops may
-    // run more than once.
+    // Item numbers and row starts fit an int, and their factors 24 bits
+    // (lists hold at most 5851 entries: 160 KB of LDS).  Up to 2048 entries
+    // (64 KB) they and (2m - 1)^2 stay below 2^24, exact in FP32, so the row
+    // estimates below are off by less than 0.001 and one step either way
+    // corrects them; on longer lists the correction is a loop.
     const int nitems = ROLE == 1 ? m * m2 : m * (m - 1) / 2;
     acc = 0.0;  // lanes 0, 1, 2 hold x, y, z
     int head = 0, qn = 0;
 
     auto flush = [&](int cnt) {
         __syncthreads();
+        double cx = 0.0, cy = 0.0, cz = 0.0;
         if (lane < cnt) {
-            const int q = (head + lane) & (RING - 1);
-            const int ia = sh.qa[q] & 0xffff, ib = sh.qa[q] >> 16;
-            const double xa = L.p[3 * ia], ya = L.p[3 * ia + 1], za = L.p[3 * ia + 2];
-            const double xb = L.p[3 * ib], yb = L.p[3 * ib + 1], zb = L.p[3 * ib + 2];
-            double cx, cy, cz;
-            ref_contrib<ROLE>(xp, yp, zp, xa, ya, za, xb, yb, zb, nu, nu_ok, cx, cy, cz);
-            sh.cb[lane * 3 + 0] = cx;
-            sh.cb[lane * 3 + 1] = cy;
-            sh.cb[lane * 3 + 2] = cz;
+            const int q = sh.q[(head + lane) & (RING - 1)];
+            const int ia = q & 0xffff, ib = q >> 16;
+            const double *pa = L.p + ((ia << 1) + ia), *pb = L.p + ((ib << 1) + ib);
+            const double xa = pa[0], ya = pa[1], za = pa[2];
+            const double xb = pb[0], yb = pb[1], zb = pb[2];
+            if constexpr (ROOTS)
+                ref_contrib<ROLE>(xp, yp, zp, xa, ya, za, xb, yb, zb, L.root[ia], L.root[ib],
+                                  ref_root(ref_sqr(xb - xa, yb - ya, zb - za)), nu, nu_ok, cx, cy, cz);
+            else
+                ref_contrib<ROLE>(xp, yp, zp, xa, ya, za, xb, yb, zb, nu, nu_ok, cx, cy, cz);
         }
+        // lanes past the count add zeros, which change no accumulator
+        sh.cb[0][lane] = cx;
+        sh.cb[1][lane] = cy;
+        sh.cb[2][lane] = cz;
         __syncthreads();
         if (lane < 3) {
-            for (int t = 0; t < cnt; ++t) acc = acc - sh.cb[t * 3 + lane];
+            const double2 *c = reinterpret_cast<const double2 *>(sh.cb[lane]);
+            for (int t = 0; t < cnt; t += 16) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const double2 v = c[t / 2 + k];
+                    acc = acc - v.x;
+                    acc = acc - v.y;
+                }
+            }
         }
         __syncthreads();
         head = (head + cnt) & (RING - 1);
@@ -2448,46 +2466,55 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
 
     const float twom1 = (float)(2 * m - 1), disc0 = (float)((2 * m - 1) * (2 * m - 1));
     const float inv_m2 = m2 > 0 ? 1.0f / (float)m2 : 0.0f;
+    const bool long_list = len > 2048;
     for (int t0 = 0; t0 < nitems; t0 += WAVE) {
         const int t = t0 + lane;
         bool ok = t < nitems;
         int ia = 0, ib = 0;
         if (ok) {
-            // the row from an FP32 estimate (within one of the true row),
-            // then corrected with exact integer comparisons
-            // (the loops below correct the estimate exactly, whatever its
-            // error; they are kept as loops, not unrolled: they rarely run)
+            // the row from an FP32 estimate, corrected with integers
             if constexpr (ROLE == 1) {
                 int ra = (int)((float)t * inv_m2);
-                int rem = t - ra * m2;
-#pragma clang loop unroll(disable)
-                while (rem < 0) {
-                    --ra;
-                    rem += m2;
-                }
-#pragma clang loop unroll(disable)
-                while (rem >= m2) {
-                    ++ra;
-                    rem -= m2;
+                int rem = t - __mul24(ra, m2);
+                if (long_list) {
+                    while (rem < 0) {
+                        --ra;
+                        rem += m2;
+                    }
+                    while (rem >= m2) {
+                        ++ra;
+                        rem -= m2;
+                    }
+                } else {
+                    const int down = rem < 0 ? 1 : 0, up = rem >= m2 ? 1 : 0;
+                    ra += up - down;
+                    rem += down ? m2 : (up ? -m2 : 0);
                 }
                 ia = ra;
                 ib = split + rem;
             } else {
-                // largest row a with a (2m - a - 1) / 2 <= t
+                // largest row a with a (2m - a - 1) / 2 <= t; row a holds m - a - 1 items
                 const float disc = disc0 - 8.0f * (float)t;
                 int ra = (int)((twom1 - __builtin_amdgcn_sqrtf(disc)) * 0.5f);
                 ra = ra < 0 ? 0 : (ra > m - 2 ? m - 2 : ra);
-                auto start = [&](int r) { return r * (2 * m - r - 1) / 2; };
-                int st = start(ra);
-#pragma clang loop unroll(disable)
-                while (ra > 0 && st > t) st = start(--ra);
-#pragma clang loop unroll(disable)
-                while (ra < m - 2 && start(ra + 1) <= t) st = start(++ra);
+                int st = __mul24(ra, 2 * m - ra - 1) >> 1;
+                if (long_list) {
+                    while (ra > 0 && st > t) st -= m - ra--;
+                    while (ra < m - 2 && st + (m - ra - 1) <= t) st += m - ra++ - 1;
+                } else {
+                    if (st > t) st -= m - ra--;
+                    const int nx = st + (m - ra - 1);
+                    if (nx <= t) {
+                        st = nx;
+                        ++ra;
+                    }
+                }
                 ia = s0 + ra;
                 ib = ia + 1 + (t - st);
             }
-            const double ax = L.p[3 * ia], ay = L.p[3 * ia + 1], az = L.p[3 * ia + 2];
-            const double bx = L.p[3 * ib], by = L.p[3 * ib + 1], bz = L.p[3 * ib + 2];
+            const double *pa = L.p + ((ia << 1) + ia), *pb = L.p + ((ib << 1) + ib);
+            const double ax = pa[0], ay = pa[1], az = pa[2];
+            const double bx = pb[0], by = pb[1], bz = pb[2];
             double d2;
             if (plain) {
                 // the periodic form's bits whenever every |difference| is
@@ -2502,7 +2529,7 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
         const unsigned long long mk = __ballot(ok);
         if (ok) {
             const int q = (head + qn + lane_prefix(mk)) & (RING - 1);
-            sh.qa[q] = ia | (ib << 16);  // list indices are below 2^16
+            sh.q[q] = ia | (ib << 16);  // list indices are below 2^15
         }
         const int got = __popcll(mk);
         qn += got;
@@ -2523,14 +2550,23 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
 // (each entry's rank is the number of smaller ids), carrying their positions
 // along; longer ones take a bitonic sort of the ids and read the positions
 // again.
+//
+// Bound by VALU issue (88% busy): of an owner's ~9200 instructions at N =
+// 32768 and cutoff 2 (67 neighbours, 1044 triplets in 3 x 6 batches of 64)
+// two thirds are the batches' ~270 each, then the 35 rounds of pair tests and
+// the fold (one subtraction per triplet and component).  The lists hold each
+// entry's side to the owner, items are decoded without 32-bit products (a
+// quarter of the rate), and the sort ranks as many entries per lane as the
+// list needs: 10 steps 7.5 -> 6.4 ms with the quotients of at_math.h.
 constexpr int EXACT_GATHER = 4;  // candidates per lane and round
 
 // 4 waves per SIMD: within 96 VGPRs, for a fifth, the brackets' reciprocals
-// spill (7.1 ms against 7.0 per 10 steps of N = 32768).
+// spill (6.9 ms against 6.6 per 10 steps of N = 32768).
+template <bool ROOTS>
 __global__ __launch_bounds__(WAVE, 4) void k_p3bca_exact(CutDev a)
 {
     extern __shared__ __attribute__((aligned(16))) int sid_ex[];
-    __shared__ ExactShared sh;
+    __shared__ __attribute__((aligned(16))) ExactShared sh;
     __shared__ int sh_start[32], sh_pre[32];
     // a halted step-graph replay leaves the step to the host
     if (a.st->halt) return;
@@ -2542,6 +2578,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_p3bca_exact(CutDev a)
     const double xp = a.xs[slot], yp = a.ys[slot], zp = a.zs[slot];
     const SysGrid sg = grid_of_particle(a.g, p);
     double *sp = reinterpret_cast<double *>(sid_ex + cap);  // 3 cap doubles: x, y, z of entry t at 3t
+    double2 *root = reinterpret_cast<double2 *>(sp + 3 * cap);  // ROOTS: cap
 
     const Candidates cand = gather_candidates(a, sg, xp, yp, zp, sh_start, sh_pre);
     int len = 0;
@@ -2610,40 +2647,47 @@ __global__ __launch_bounds__(WAVE, 4) void k_p3bca_exact(CutDev a)
         // (the capacity is a power of two of at least 64, so it has room).
         if (lane < ((4 - (len & 3)) & 3)) sid_ex[len + lane] = INT_MAX;
         __syncthreads();
-        int id[EXACT_GATHER], rk[EXACT_GATHER];
-        double ex[EXACT_GATHER], ey[EXACT_GATHER], ez[EXACT_GATHER];
+        auto rank_sort = [&](auto per_lane) {
+            constexpr int NH = decltype(per_lane)::value;  // entries per lane
+            int id[NH], rk[NH];
+            double ex[NH], ey[NH], ez[NH];
 #pragma unroll
-        for (int h = 0; h < EXACT_GATHER; ++h) {
-            const int t = h * WAVE + lane;
-            id[h] = INT_MAX;
-            rk[h] = 0;
-            ex[h] = ey[h] = ez[h] = 0.0;
-            if (t < len) {
-                id[h] = sid_ex[t];
-                ex[h] = sp[3 * t];
-                ey[h] = sp[3 * t + 1];
-                ez[h] = sp[3 * t + 2];
-                note_far(ex[h], ey[h], ez[h]);
-                below += id[h] < p ? 1 : 0;
+            for (int h = 0; h < NH; ++h) {
+                const int t = h * WAVE + lane;
+                id[h] = INT_MAX;
+                rk[h] = 0;
+                ex[h] = ey[h] = ez[h] = 0.0;
+                if (t < len) {
+                    id[h] = sid_ex[t];
+                    ex[h] = sp[3 * t];
+                    ey[h] = sp[3 * t + 1];
+                    ez[h] = sp[3 * t + 2];
+                    note_far(ex[h], ey[h], ez[h]);
+                    below += id[h] < p ? 1 : 0;
+                }
             }
-        }
-        const int4 *ids4 = reinterpret_cast<const int4 *>(sid_ex);
-        for (int j = 0; j < (len + 3) >> 2; ++j) {
-            const int4 v = ids4[j];
+            const int4 *ids4 = reinterpret_cast<const int4 *>(sid_ex);
+            for (int j = 0; j < (len + 3) >> 2; ++j) {
+                const int4 v = ids4[j];
 #pragma unroll
-            for (int h = 0; h < EXACT_GATHER; ++h)
-                rk[h] += (v.x < id[h] ? 1 : 0) + (v.y < id[h] ? 1 : 0) + (v.z < id[h] ? 1 : 0) + (v.w < id[h] ? 1 : 0);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int h = 0; h < EXACT_GATHER; ++h) {
-            if (h * WAVE + lane < len) {
-                sid_ex[rk[h]] = id[h];
-                sp[3 * rk[h]] = ex[h];
-                sp[3 * rk[h] + 1] = ey[h];
-                sp[3 * rk[h] + 2] = ez[h];
+                for (int h = 0; h < NH; ++h)
+                    rk[h] += (v.x < id[h] ? 1 : 0) + (v.y < id[h] ? 1 : 0) + (v.z < id[h] ? 1 : 0) +
+                             (v.w < id[h] ? 1 : 0);
             }
-        }
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                if (h * WAVE + lane < len) {
+                    sid_ex[rk[h]] = id[h];
+                    sp[3 * rk[h]] = ex[h];
+                    sp[3 * rk[h] + 1] = ey[h];
+                    sp[3 * rk[h] + 2] = ez[h];
+                }
+            }
+        };
+        if (len <= WAVE) rank_sort(std::integral_constant<int, 1>{});
+        else if (len <= 2 * WAVE) rank_sort(std::integral_constant<int, 2>{});
+        else rank_sort(std::integral_constant<int, EXACT_GATHER>{});
     } else {
         // bitonic sort of sid_ex[0, P), padded with INT_MAX, then the
         // positions read again in sorted order
@@ -2681,14 +2725,19 @@ __global__ __launch_bounds__(WAVE, 4) void k_p3bca_exact(CutDev a)
     const int split = below;
     const bool plain = __ballot(far) == 0;
     __syncthreads();
-    const StagedList list{sp};
+    if constexpr (ROOTS) {
+        for (int t = lane; t < len; t += WAVE)
+            root[t] = ref_root(ref_sqr(sp[3 * t] - xp, sp[3 * t + 1] - yp, sp[3 * t + 2] - zp));
+        __syncthreads();
+    }
+    const StagedList list{sp, root};
     double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
     unsigned long long accepted = 0, unused = 0;
-    exact_role_staged<0>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc0,
+    exact_role_staged<0, ROOTS>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc0,
                          accepted);
-    exact_role_staged<1>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc1,
+    exact_role_staged<1, ROOTS>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc1,
                          unused);
-    exact_role_staged<2>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc2,
+    exact_role_staged<2, ROOTS>(list, xp, yp, zp, len, split, plain, a.c2, sg.L[0], sg.L[1], sg.L[2], a.nu, sh, acc2,
                          unused);
     if (lane < 3) {
         a.facc[(long long)lane * a.n + p] = acc0;
@@ -3013,8 +3062,15 @@ size_t p3bca_fast_lds(int cap)
     return (size_t)cap * (6 * sizeof(double) + sizeof(int)) + RING * sizeof(unsigned) + 64 * sizeof(int);
 }
 
-// sorted ids, then (8-byte aligned, cap is a multiple of 64) the positions
-size_t p3bca_exact_lds(int cap) { return (size_t)cap * (sizeof(int) + 3 * sizeof(double)); }
+// The exact sweep's lists hold roots where that leaves them under 64 KB.
+static bool exact_roots(int cap) { return cap <= 1024; }
+
+// sorted ids, then (16-byte aligned, cap is a multiple of 64) the positions
+// and the roots
+size_t p3bca_exact_lds(int cap)
+{
+    return (size_t)cap * (sizeof(int) + 3 * sizeof(double) + (exact_roots(cap) ? sizeof(double2) : 0));
+}
 
 void launch_soa_from_rows(hipStream_t s, int n, const double *rows, double *x, double *y, double *z)
 {
@@ -3321,8 +3377,13 @@ void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     if (d.n <= 0) return;
     const CutDev a = cut_dev(d, g, c, nu, cap, st, 0);
     const size_t shm = p3bca_exact_lds(cap);
-    allow_lds(k_p3bca_exact, shm);
-    hipLaunchKernelGGL(k_p3bca_exact, dim3(owner_grid(d.n)), dim3(WAVE), shm, s, a);
+    const dim3 grid(owner_grid(d.n)), blk(WAVE);
+    if (exact_roots(cap)) {
+        hipLaunchKernelGGL(k_p3bca_exact<true>, grid, blk, shm, s, a);
+    } else {
+        allow_lds(k_p3bca_exact<false>, shm);
+        hipLaunchKernelGGL(k_p3bca_exact<false>, grid, blk, shm, s, a);
+    }
 }
 
 void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *st, double2 *roots)
