@@ -181,3 +181,15 @@ def test_exact_cutoff_list_lengths(eng, oracle, n, spacing):
     *_, fo, co = oracle.sweep(P, cutoff=2.0, L=L, mode="owner")
     assert cnt == co
     assert np.array_equal(eng.get_particles()["f"], fo)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [4913, 5832, 9261, 12167])
+def test_cutoff_heaviest_cells_split(eng, oracle, n, precision):
+    """1331 to 2744 cells, a sixteenth of them split among two workgroups,
+    and 3375, none of them."""
+    P = jittered(n, 5000 + n, sd=0.1)
+    L = np.full(3, 0.8 * round(n ** (1 / 3)))
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=1.2, domain_L=L, precision=precision)
+    check(eng, oracle, P, precision, cutoff=1.2, L=L)

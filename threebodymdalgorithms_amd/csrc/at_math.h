@@ -314,21 +314,6 @@ __device__ __forceinline__ float rsqrt_f32(float x)
     return __builtin_fmaf(0.5f * y, r, y);
 }
 
-template <class T>
-__device__ __forceinline__ T fma_t(T a, T b, T c);
-template <>
-__device__ __forceinline__ double fma_t<double>(double a, double b, double c)
-{
-    return __builtin_fma(a, b, c);
-}
-template <>
-__device__ __forceinline__ float fma_t<float>(float a, float b, float c)
-{
-    return __builtin_fmaf(a, b, c);
-}
-__device__ __forceinline__ double rsqrt_t(double x) { return rsqrt_f64(x); }
-__device__ __forceinline__ float rsqrt_t(float x) { return rsqrt_f32(x); }
-
 // Mixed-precision form: u, v, w arrive in FP64 and A = u+v-w, B = u-v+w,
 // C = -u+v+w are formed in FP64 before rounding to FP32, because for
 // elongated triangles (two long sides of nearly equal length) the difference
@@ -391,41 +376,12 @@ __device__ __forceinline__ void at_coeffs_mixed(double u64, double v64, double w
     }
 }
 
-// Dispatch on the per-triplet type: FP64 throughout, or the mixed form; the
-// gradient coefficients come back in FP64 either way.
-template <class T, bool NEED_W>
-__device__ __forceinline__ void at_coeffs_from64(double u, double v, double w, T nu, T K, double &cu, double &cv,
-                                                 double &cw, T &e);
-
-// Gradient coefficients of one triplet in the squared-distance form.
-// Returns eu = 2 dE/du, ev = 2 dE/dv, ew = 2 dE/dw and the energy e, so that
+// Gradient coefficients of one triplet in the squared-distance form, in FP64
+// with s = (u v w)^-1/2 given; s = 0 (u, v, w finite) gives zero coefficients
+// and energy.  Returns eu = 2 dE/du, ev = 2 dE/dv, ew = 2 dE/dw and the energy
+// e, so that
 //   dE/dxi = -(eu dij + ev dik), dE/dxj = eu dij - ew djk, dE/dxk = ev dik + ew djk
 // with dij = xj - xi, dik = xk - xi, djk = xk - xj.
-template <class T, bool NEED_W>
-__device__ __forceinline__ void at_coeffs(T u, T v, T w, T nu, T K, T &eu, T &ev, T &ew, T &e)
-{
-    const T uv = u * v;
-    const T s = rsqrt_t(uv * w);
-    const T s2 = s * s;
-    const T A = (u + v) - w;
-    const T B = (u - v) + w;
-    const T C = (v - u) + w;
-    const T X = B * C, Y = A * C, Z = A * B;
-    const T Q = (A * X) * s2;
-    const T R = fma_t<T>(T(-2.5) * K, Q, T(-1.5) * nu);
-    const T S = (X + Y) + Z;
-    const T KS = K * S;
-    const T m2K = T(-2) * K;
-    const T c2s5 = T(2) * (s2 * s2 * s);
-    eu = c2s5 * fma_t<T>(R, v * w, fma_t<T>(m2K, Z, KS));
-    ev = c2s5 * fma_t<T>(R, u * w, fma_t<T>(m2K, Y, KS));
-    if constexpr (NEED_W) ew = c2s5 * fma_t<T>(R, uv, fma_t<T>(m2K, X, KS));
-    else ew = T(0);
-    e = (s2 * s) * fma_t<T>(K, Q, nu);
-}
-
-// at_coeffs in FP64 with s = (u v w)^-1/2 given; s = 0 (u, v, w finite) gives
-// zero coefficients and energy.
 template <bool WANT_E>
 __device__ __forceinline__ void at_coeffs_roots(double u, double v, double w, double s, double nu, double K,
                                                 double &eu, double &ev, double &ew, double &e)
@@ -449,11 +405,13 @@ __device__ __forceinline__ void at_coeffs_roots(double u, double v, double w, do
     e = WANT_E ? s3 * __builtin_fma(K, Q, nu) : 0.0;
 }
 
+// Dispatch on the per-triplet type: FP64 throughout, or the mixed form; the
+// gradient coefficients come back in FP64 either way.
 template <class T, bool NEED_W>
 __device__ __forceinline__ void at_coeffs_from64(double u, double v, double w, T nu, T K, double &cu, double &cv,
                                                  double &cw, T &e)
 {
-    if constexpr (sizeof(T) == 8) at_coeffs<double, NEED_W>(u, v, w, nu, K, cu, cv, cw, e);
+    if constexpr (sizeof(T) == 8) at_coeffs_roots<true>(u, v, w, rsqrt_f64(u * v * w), nu, K, cu, cv, cw, e);
     else at_coeffs_mixed(u, v, w, nu, K, cu, cv, cw, e, NEED_W);
 }
 

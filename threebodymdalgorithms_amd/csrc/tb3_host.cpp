@@ -594,20 +594,24 @@ bool wide_expected(const CellGrid &g, double cutoff, long long n)
 bool cells_wide(const tb3_ctx *c, long long n) { return c->wide_need || wide_expected(c->grid, c->cutoff, n); }
 
 // Workgroups per cell: a grid whose cells do not fill the GPU's workgroup
-// slots (4 or, wide, 2 per CU) splits each cell's owners among several, which
+// slots (5 or, wide, 2 per CU) splits each cell's owners among several, which
 // each stage the cell's neighbourhood: just more workgroups than slots, down
 // to 2 owners each, and up to 16 parts, past which the parts' atomics on a
 // cell's few particles cost more (1 cell of 400: 16 parts 32 us, 64 48, 200
 // 101).  Kernel times at cutoff 2, density 2, with 1 and this many parts: 1
 // cell 181 -> 24 us, 64 cells 71 -> 27, 216 54 -> 30, 343 66 -> 43, 512 98 ->
 // 61, 729 86 -> 66, 1000 93 -> 85.  Past the slots a second staging costs more
-// than it spreads (1728 cells, 2 parts: 117 -> 135).
-int cell_parts(const tb3_ctx *c, int ncell, long long n, bool wide)
+// than it spreads (1728 cells, 2 parts: 117 -> 135), except for the heaviest
+// cells, which would be the last to end: with a sixteenth of the cells in 2
+// parts, 1728 cells of 16 take 103 us instead of 114, of 19 116 instead of
+// 119; from 2.5 times the slots it makes no difference.
+CellSplit cell_split(const tb3_ctx *c, int ncell, long long n, bool wide)
 {
-    const int slots = c->ncu * (wide ? 2 : 4);
-    if (ncell > slots || ncell <= 0) return 1;
+    const int slots = c->ncu * (wide ? 2 : 5);
+    if (ncell <= 0 || ncell > slots * 5 / 2) return {0, 1};
+    if (ncell > slots) return {(ncell + 127) / 128, 2};
     const long long own = (n + ncell - 1) / ncell;
-    return (int)std::max<long long>(1, std::min<long long>({slots / ncell + 1, (own + 1) / 2, 16}));
+    return {ncell, (int)std::max<long long>(1, std::min<long long>({slots / ncell + 1, (own + 1) / 2, 16}))};
 }
 
 // The n x n table of pair lengths that the bit-exact all-triplets sweep reads
@@ -654,7 +658,7 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
                 const bool wide = cells_wide(c, d.n);
                 launch_p3bca_cells(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                    energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0,
-                                   cell_parts(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0, parity);
+                                   cell_split(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0, parity);
                 if (c->dense_on)
                     launch_p3bca_dense(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                        energy ? 1 : 0, c->d_owners, c->dense_grid, c->dense_waves);
@@ -1702,7 +1706,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             if (n >= 3) {
                 if (cells) {
                     launch_p3bca_cells(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, dense ? 1 : 0, wide ? 1 : 0,
-                                       cell_parts(c, ncell, n, wide));
+                                       cell_split(c, ncell, n, wide));
                     if (dense)
                         launch_p3bca_dense(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, c->dense_grid,
                                            c->dense_waves);

@@ -206,7 +206,11 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
                        int cap, int mixed, int grad, Status *st, int count_slot, int want_energy);
 void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int cap, Status *st);
-// Fast cutoff sweep, `parts` workgroups per cell, in the narrow or the wide
+// The first `head` cells of each XCD's run are split among `parts` workgroups.
+struct CellSplit {
+    int head, parts;
+};
+// Fast cutoff sweep, one workgroup per cell or `split`, in the narrow or the wide
 // shape (4 waves, 256 staged particles and lists of 96; 8 waves, 416 and
 // 144).  With dense_on, owners it cannot stage go to `owners` for
 // launch_p3bca_dense, which must follow on the same stream; without, such an
@@ -217,7 +221,7 @@ void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, 
 // `slotted`: sweep the slotted layout (needs dense_on == 0).
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, int parts, int slotted = 0, int parity = -1);
+                        int wide, CellSplit split, int slotted = 0, int parity = -1);
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
 int p3bca_cells_blocks_per_cu();
 // The cell kernel hands owners whose neighbourhood does not fit its LDS

@@ -1403,11 +1403,17 @@ __global__ __launch_bounds__(WAVE) void k_p3bca_fast(CutDev a)
 // owner whose list is longer than LCAP, are queued for the dense-owner
 // kernel below instead.
 //
-// Few cells leave most of the chip without a workgroup; the grid's y then
-// splits each cell's owners among `parts` workgroups (part k takes owners k,
-// k + parts, ...), each with its own staging.
-
-constexpr int RQ = 128;    // per-wave queue of passing pairs (>= 2 x 64)
+// Where cells are few, or the heaviest would outlast the rest, the owners of
+// the first `head` cells of each XCD's run are split among `parts` workgroups
+// (part k takes owners k, k + parts, ...), each with its own staging.
+//
+// Bound by VALU issue (70% at N = 1048576) beside LDS, with latencies between
+// them: a fifth wave per SIMD, which is what keeps the workgroup's LDS within
+// 32000 bytes (the queue holds one batch, the particles' numbers wait in
+// registers), takes N = 1048576 at cutoff 2 from 2810 to 2680 us and 25001 in
+// FP32-mixed from 108 to 94; three rows of 5 waves per workgroup instead,
+// 3485.  Of the 2680, 300 are staging, 440 the owners' lists, 690 the tests of
+// pairs and 1260 the evaluations.
 
 struct CellsDev {
     CutDev c;
@@ -1418,13 +1424,14 @@ struct CellsDev {
     const int *order;  // each XCD's run of cells, heaviest first (k_cell_scatter)
     unsigned *cell_work;  // each cell's accepted triplets, the next sweep's dispatch key
     SlotsDev sl;          // the slotted layout (cap > 0: staged from its slot records)
+    int head, parts;      // the first cells of each XCD's run, each split among this many workgroups
 };
 
 // The two shapes of the cell kernel: waves of a workgroup, staged particles
 // and entries of a wave's list (list positions fit in the 8-bit halves of a
-// queue entry).  16 waves per CU either way: 34 KB of LDS, 4 workgroups of a
-// CU, or 82 KB, 2 of them, for neighbourhoods that the narrow one would leave
-// to one 8-wave workgroup per owner (k_p3bca_dense).
+// queue entry).  20 waves per CU in 5 workgroups with 32 KB of LDS each, or 16
+// in 2 with 79 KB, for neighbourhoods that the narrow one would leave to one
+// 8-wave workgroup per owner (k_p3bca_dense).
 template <bool WIDE>
 struct CellShape {
     static constexpr int W = WIDE ? 8 : 4, NB = WIDE ? 416 : 256, LC = WIDE ? 144 : 96;
@@ -1515,6 +1522,19 @@ __device__ void stage_cells(const CutDev &A, const SysGrid &sg, int c, int *cst,
     }
 }
 
+// The geometry of cell c along dimension k for the staging's box test: its
+// cell coordinate, the cells per length, 1 / cells, and the cell width.
+__device__ __forceinline__ void cell_geometry(const SysGrid &sg, int c, int k, double *geo)
+{
+    const int lc = c - sg.cbase;
+    const int n = k == 0 ? sg.nc[0] : (k == 1 ? sg.nc[1] : sg.nc[2]);
+    const double L = k == 0 ? sg.L[0] : (k == 1 ? sg.L[1] : sg.L[2]);
+    geo[4 * k + 0] = (double)(k == 0 ? lc % sg.nc[0] : (k == 1 ? lc / sg.nc[0] % sg.nc[1] : lc / (sg.nc[0] * sg.nc[1])));
+    geo[4 * k + 1] = (double)n / L;
+    geo[4 * k + 2] = 1.0 / (double)n;
+    geo[4 * k + 3] = L / (double)n;
+}
+
 // Squared distance for the cutoff test.  PER: the periodic form
 // min(t, L - t) per component (Algorithm.cpp's cutoff test).  !PER: the plain
 // difference, which gives the same bits whenever every |difference| is below
@@ -1544,11 +1564,21 @@ __device__ __forceinline__ int staged_slot(const int *cst, const int *cpre, int 
 // Cell for workgroup b, or -1: workgroups are dispatched round-robin over
 // the 8 XCDs (b % 8), so each XCD gets a contiguous run of cells, whose
 // neighbourhoods overlap in its own L2, of about an eighth of the work, and
-// takes them heaviest first (order_runs).
-__device__ __forceinline__ int cell_for_block(int b, int ncell, const int *order)
+// takes them heaviest first (order_runs).  The first `head` cells of a run
+// are each split among `parts` workgroups.
+__device__ __forceinline__ int cell_for_block(int b, int ncell, const int *order, int head, int &part, int &parts)
 {
     const int cap = cell_run_cap(ncell);
-    const int r = b & 7, k = b >> 3;
+    const int r = b & 7;
+    int k = b >> 3;
+    if (k < head * parts) {
+        part = k % parts;
+        k /= parts;
+    } else {
+        k -= head * (parts - 1);
+        part = 0;
+        parts = 1;
+    }
     if (k >= cap || k >= order[8 * cap + r]) return -1;
     return order[r * cap + k];
 }
@@ -1557,23 +1587,24 @@ template <class T, bool GRAD, bool WANT_E, bool WIDE>
 __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(CellsDev a)
 {
     constexpr int CELL_WAVES = CellShape<WIDE>::W, NBCAP = CellShape<WIDE>::NB, LCAP = CellShape<WIDE>::LC;
-    const int part = blockIdx.y, parts = gridDim.y;
+    using StagedIndex = typename std::conditional<(NBCAP > 256), unsigned short, unsigned char>::type;
+    static_assert(NBCAP <= CELL_WAVES * WAVE && LCAP >= WAVE && LCAP <= 256, "one staged particle per thread");
     // one block per array family, so that the y, z and gradient arrays sit
     // at constant offsets from x and their addresses fold into the LDS
     // instructions' immediate offsets
     __shared__ double stg[6][NBCAP];
     double *nx = stg[0], *ny = stg[1], *nz = stg[2];
     double *gxs = stg[3], *gys = stg[4], *gzs = stg[5];
-    __shared__ int nid[NBCAP];
-    __shared__ unsigned short wl[CELL_WAVES][LCAP];
+    __shared__ StagedIndex wl[CELL_WAVES][LCAP];
     __shared__ double wls[CELL_WAVES][6][LCAP];
-    __shared__ unsigned short ring[CELL_WAVES][RQ];
+    __shared__ unsigned short ring[CELL_WAVES][WAVE];
     __shared__ int cst[32], cpre[33], sinfo[4];
     __shared__ int s_next, s_far, s_wcnt[2][CELL_WAVES];
     __shared__ unsigned s_work;
 
     const CutDev &A = a.c;
-    const int c = cell_for_block(blockIdx.x, a.ncell, a.order);
+    int part, parts = a.parts;
+    const int c = cell_for_block(blockIdx.x, a.ncell, a.order, a.head, part, parts);
     if (c < 0) return;
     const int tid = threadIdx.x, lane = lane_id(), wv = tid / WAVE;
     // A halted step-graph replay leaves the step to the host.  Non-finite
@@ -1615,7 +1646,9 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     // workgroups' arithmetic (C1 sweep 120.7 -> 117.5 us; the same priority
     // for the evaluations made it 130 us, for the owners' list builds 121 us).
     __builtin_amdgcn_s_setprio(3);
+    double *geo = wls[0][1];  // until wave 0's first list
     if (wv == 0) stage_cells(A, sg, c, cst, cpre, sinfo, scnt, a.sl.cap);
+    if (wv == 1 && lane < 3) cell_geometry(sg, c, lane, geo);
     __syncthreads();
     const int cand = sinfo[3], own = sinfo[1], nk = sinfo[2];
 
@@ -1636,25 +1669,21 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     }
     int total = 0;
     {
-        const int lc = c - sg.cbase;
-        const double ccx = (double)(lc % sg.nc[0]), ccy = (double)((lc / sg.nc[0]) % sg.nc[1]),
-                     ccz = (double)(lc / (sg.nc[0] * sg.nc[1]));
-        const double wx = Lx / sg.nc[0], wy = Ly / sg.nc[1], wz = Lz / sg.nc[2];
-        const double ix = 1.0 / wx, iy = 1.0 / wy, iz = 1.0 / wz;
-        const double mx = sg.lo[0] + (ccx + 0.5) * wx, my = sg.lo[1] + (ccy + 0.5) * wy,
-                     mz = sg.lo[2] + (ccz + 0.5) * wz;
+        const double ccx = geo[0], ccy = geo[4], ccz = geo[8], ix = geo[1], iy = geo[5], iz = geo[9];
         const double reach2 = c2 * (1.0 + 1e-6);
-        auto gap = [](double d, double L, double w) {
-            d -= L * __builtin_rint(d / L);
-            const double g = __builtin_fabs(d) - 0.5 * w;
-            return g > 0.0 ? g : 0.0;
+        // periodic distance from c's box along dimension k, from the unwrapped
+        // cell coordinate u of a position relative to c's
+        auto gap = [&](double u, int k) {
+            double d = u - 0.5;
+            d = __builtin_fma(-(double)sg.nc[k], __builtin_rint(d * geo[4 * k + 2]), d);
+            return __builtin_fmax(__builtin_fabs(d) - 0.5, 0.0) * geo[4 * k + 3];
         };
         // two candidates per thread and round (a cell's neighbourhood has
         // ~265 on average), with every load issued before the first use
         bool far = false;
         constexpr int NT = CELL_WAVES * WAVE;
         for (int t0 = 0; t0 < cand; t0 += 2 * NT) {
-            bool keep[2];
+            bool keep[2], out[2];
             double x[2], y[2], z[2];
             int q[2];
 #pragma unroll
@@ -1682,10 +1711,14 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int t = t0 + h * NT + tid;
+                out[h] = false;
                 if (t < cand) {
-                    const double gx = gap(x[h] - mx, Lx, wx), gy = gap(y[h] - my, Ly, wy),
-                                 gz = gap(z[h] - mz, Lz, wz);
+                    const double ux = __builtin_fma(x[h] - sg.lo[0], ix, -ccx),
+                                 uy = __builtin_fma(y[h] - sg.lo[1], iy, -ccy),
+                                 uz = __builtin_fma(z[h] - sg.lo[2], iz, -ccz);
+                    const double gx = gap(ux, 0), gy = gap(uy, 1), gz = gap(uz, 2);
                     keep[h] = t < own || gx * gx + gy * gy + gz * gz <= reach2;
+                    out[h] = !(ux >= -1.01 && ux < 2.01 && uy >= -1.01 && uy < 2.01 && uz >= -1.01 && uz < 2.01);
                 }
             }
             const unsigned long long m0 = __ballot(keep[0]), m1 = __ballot(keep[1]);
@@ -1711,13 +1744,11 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                     nx[p] = x[h];
                     ny[p] = y[h];
                     nz[p] = z[h];
-                    nid[p] = q[h];
+                    wls[p / WAVE][0][p % WAVE] = __longlong_as_double(q[h]);
                     gxs[p] = 0.0;
                     gys[p] = 0.0;
                     gzs[p] = 0.0;
-                    const double ux = (x[h] - sg.lo[0]) * ix - ccx, uy = (y[h] - sg.lo[1]) * iy - ccy,
-                                 uz = (z[h] - sg.lo[2]) * iz - ccz;
-                    far = far || !(ux >= -1.01 && ux < 2.01 && uy >= -1.01 && uy < 2.01 && uz >= -1.01 && uz < 2.01);
+                    far = far || out[h];
                 }
             }
             __syncthreads();  // s_wcnt is reused
@@ -1739,10 +1770,13 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
         return;
     }
     __syncthreads();
+    // staged particle tid's number waits in a register for the end; its wave's
+    // list, not yet in use, brought it
+    const int my_id = tid < total ? (int)__double_as_longlong(wls[wv][0][lane]) : 0;
 
     // 3. owners of cell c, claimed one at a time by the waves; the cutoff
     // tests take the plain form unless the staging found a far particle
-    unsigned short *list = wl[wv];
+    StagedIndex *list = wl[wv];
     double *qx = wls[wv][0], *qy = wls[wv][1], *qz = wls[wv][2];
     double *hx = wls[wv][3], *hy = wls[wv][4], *hz = wls[wv][5];
     auto owners = [&](auto per) {
@@ -1770,7 +1804,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                 const unsigned long long m = __ballot(ok);
                 const int pos = len + lane_prefix(m);
                 if (ok && pos < LCAP) {
-                    list[pos] = (unsigned short)t;
+                    list[pos] = (StagedIndex)t;
                     qx[pos] = xt;
                     qy[pos] = yt;
                     qz[pos] = zt;
@@ -1803,11 +1837,11 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
             const int npairs = len * (len - 1) / 2;
             if (npairs > 0) {
                 unsigned short *rq = ring[wv];
-                int head = 0, qn = 0;
+                int qn = 0;
                 auto flush = [&](int nq) {
                     wave_sync();
                     if (lane < nq) {
-                        const unsigned e = rq[(head + lane) & (RQ - 1)];
+                        const unsigned e = rq[lane];
                         const int r = (int)(e & 0xffu), kk = (int)(e >> 8);
                         const double xj = qx[r], yj = qy[r], zj = qz[r];
                         const double xk = qx[kk], yk = qy[kk], zk = qz[kk];
@@ -1834,8 +1868,6 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                         ++cnt;
                     }
                     wave_sync();
-                    head = (head + nq) & (RQ - 1);
-                    qn -= nq;
                 };
                 // 64 / len and lane / len from one FP32 reciprocal: for
                 // len <= LCAP the fraction of (k + 0.5) / len stays 0.5 / len
@@ -1851,9 +1883,14 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                     kk = live ? kk : r;  // lanes past the last item read their own entry
                     const bool ok = live && !(cut_sq<PER>(qx[r], qy[r], qz[r], qx[kk], qy[kk], qz[kk], Lx, Ly, Lz) > c2);
                     const unsigned long long m = __ballot(ok);
-                    if (ok) rq[(head + qn + lane_prefix(m)) & (RQ - 1)] = (unsigned short)(r | (kk << 8));
+                    const int at = qn + lane_prefix(m);
+                    if (ok && at < WAVE) rq[at] = (unsigned short)(r | (kk << 8));
                     qn += __popcll(m);
-                    if (qn >= WAVE) flush(WAVE);
+                    if (qn >= WAVE) {
+                        flush(WAVE);
+                        if (ok && at >= WAVE) rq[at - WAVE] = (unsigned short)(r | (kk << 8));
+                        qn -= WAVE;
+                    }
                     r += r64;
                     o += q64;
                     if (r >= len) {
@@ -1905,9 +1942,9 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     // cells) hold exact zeros and are skipped: f starts at +0.0, and adding
     // +-0.0 to it never changes it.
     if (GRAD) {
-        for (int t = tid; t < total; t += CELL_WAVES * WAVE) {
-            const int q = nid[t];
-            const double gx = gxs[t], gy = gys[t], gz = gzs[t];
+        if (tid < total) {
+            const int q = my_id;
+            const double gx = gxs[tid], gy = gys[tid], gz = gzs[tid];
             if (gx != 0.0 || gy != 0.0 || gz != 0.0) {
                 unsafeAtomicAdd(&A.fx[q], gx);
                 unsafeAtomicAdd(&A.fy[q], gy);
@@ -1955,6 +1992,8 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
 // 2.7 (lists of 91) 511 -> 470 us.  Evaluating every tested pair in place
 // with the coefficients masked (half of them pass) has no LDS conflicts but
 // 25% more VALU work: 1550, 7.2, 507.
+constexpr int RQ = 128;    // a wave's queue of passing pairs (>= 2 x 64)
+
 struct DenseDev {
     CutDev c;
     const double *xs, *ys, *zs;
@@ -3257,7 +3296,7 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
 
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, int parts, int slotted, int parity)
+                        int wide, CellSplit split, int slotted, int parity)
 {
     if (d.n <= 0) return;
     CellsDev a;
@@ -3273,7 +3312,10 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     a.cell_work = g.cell_work;
     a.sl = slots_dev(&g, slotted, parity);
     // the 8 XCDs' runs at their capacity (the workgroups past a run's length exit at once)
-    const dim3 gr((unsigned)(8 * cell_run_cap(g.ncell)), (unsigned)parts);
+    const int cap = cell_run_cap(g.ncell);
+    a.parts = split.parts;
+    a.head = split.parts > 1 ? min(split.head, cap) : 0;
+    const dim3 gr((unsigned)(8 * (cap + (a.parts - 1) * a.head)));
 #define TB3_CELLS(T, G, E)                                                                                \
     do {                                                                                                  \
         if (wide) hipLaunchKernelGGL((k_p3bca_cells<T, G, E, true>), gr, dim3(CellShape<true>::W * WAVE), 0, s, a); \
