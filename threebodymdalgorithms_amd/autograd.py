@@ -36,7 +36,7 @@ class _Energy(torch.autograd.Function):
         _check_pos(pos)
         pos_c = pos.detach().contiguous()
         nu_v = float(nu)
-        E = torch.zeros((), dtype=torch.float64, device=pos.device)
+        E = torch.empty((), dtype=torch.float64, device=pos.device)
         grad = None
         if ctx.needs_input_grad[0]:
             # one sweep gives E and dE/dx together; backward only scales it
@@ -48,7 +48,8 @@ class _Energy(torch.autograd.Function):
         ctx.engine = engine
         ctx.nu_v = nu_v
         ctx.has_grad = grad is not None
-        ctx.save_for_backward(pos_c, E.detach().clone(), grad if grad is not None else E.new_zeros(()))
+        # dE/dnu comes from E, kept apart from the output that the caller may change
+        ctx.save_for_backward(pos_c, E.detach().clone() if ctx.needs_input_grad[1] else None, grad)
         return E
 
     @staticmethod
@@ -58,17 +59,19 @@ class _Energy(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             if not ctx.has_grad:
                 grad = torch.empty_like(pos_c)
-                E2 = torch.zeros((), dtype=torch.float64, device=pos_c.device)
+                E2 = torch.empty((), dtype=torch.float64, device=pos_c.device)
                 ctx.engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), ctx.nu_v, E2.data_ptr(),
                                            grad.data_ptr(), _stream_handle(pos_c.device))
             g_pos = grad * gE
         g_nu = None
         if ctx.needs_input_grad[1]:
             # E is linear in nu: dE/dnu is the energy at nu = 1
-            if ctx.nu_v != 0.0:
+            if ctx.nu_v == 1.0:
+                g_nu = E * gE  # E / 1 is E
+            elif ctx.nu_v != 0.0:
                 g_nu = (E / ctx.nu_v) * gE
             else:
-                E1 = torch.zeros((), dtype=torch.float64, device=pos_c.device)
+                E1 = torch.empty((), dtype=torch.float64, device=pos_c.device)
                 ctx.engine.energy_dev(pos_c.shape[0], pos_c.data_ptr(), 1.0, E1.data_ptr(),
                                       _stream_handle(pos_c.device))
                 g_nu = E1 * gE
@@ -81,7 +84,7 @@ class _Forces(torch.autograd.Function):
         _check_pos(pos)
         pos_c = pos.detach().contiguous()
         nu_v = float(nu)
-        E = torch.zeros((), dtype=torch.float64, device=pos.device)
+        E = torch.empty((), dtype=torch.float64, device=pos.device)
         grad = torch.empty_like(pos_c)
         engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), grad.data_ptr(),
                                _stream_handle(pos.device))
@@ -101,7 +104,7 @@ class _Forces(torch.autograd.Function):
             if ctx.nu_v != 0.0:
                 g_nu = (gF * grad).sum() / ctx.nu_v
             else:
-                E1 = torch.zeros((), dtype=torch.float64, device=pos_c.device)
+                E1 = torch.empty((), dtype=torch.float64, device=pos_c.device)
                 grad1 = torch.empty_like(pos_c)
                 ctx.engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), 1.0, E1.data_ptr(), grad1.data_ptr(),
                                            _stream_handle(pos_c.device))
@@ -112,12 +115,12 @@ class _Forces(torch.autograd.Function):
 def at_energy(pos, nu, engine: Engine):
     """Total Axilrod-Teller energy of `pos` (differentiable in pos and nu)."""
     if not isinstance(nu, torch.Tensor):
-        nu = torch.tensor(float(nu), dtype=torch.float64, device=pos.device)
+        nu = torch.tensor(float(nu), dtype=torch.float64)  # on the host, where its value is read
     return _Energy.apply(pos, nu, engine)
 
 
 def at_forces(pos, nu, engine: Engine):
     """dE/dx at `pos` (the reference's f), differentiable in nu."""
     if not isinstance(nu, torch.Tensor):
-        nu = torch.tensor(float(nu), dtype=torch.float64, device=pos.device)
+        nu = torch.tensor(float(nu), dtype=torch.float64)  # on the host, where its value is read
     return _Forces.apply(pos, nu, engine)
