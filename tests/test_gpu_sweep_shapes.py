@@ -193,3 +193,16 @@ def test_cutoff_heaviest_cells_split(eng, oracle, n, precision):
     eng.set_particles(P)
     eng.configure("p3bca", cutoff=1.2, domain_L=L, precision=precision)
     check(eng, oracle, P, precision, cutoff=1.2, L=L)
+
+
+@pytest.mark.parametrize("n", [300, 800, 1500])
+def test_cutoff_uneven_cells(eng, oracle, n):
+    """A cloud in a box of 1728 cells, most of them empty: the few that hold it
+    are split by their work, estimated in the first pass and measured in the
+    next ones, and (n = 1500) hand owners on, one by one and cell by cell."""
+    P = np.random.default_rng(n).normal(12.0, 2.0, (n, 3))
+    L = np.full(3, 24.5)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=2.0, domain_L=L, precision="fp64")
+    for _ in range(3):
+        check(eng, oracle, P, "fp64", cutoff=2.0, L=L)

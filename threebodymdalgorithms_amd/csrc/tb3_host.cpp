@@ -95,8 +95,11 @@ constexpr int MAX_LIST = 16384;  // longest neighbour list the LDS staging accep
 // code `scratch` names a host-side stand-in, never the device memory: its
 // device address comes from hipGetSymbolAddress, once per device (at
 // tb3_create, with that device current), and only that address is used.
+// What the entries of split cells take is on top of the size that calls are
+// measured against.
 constexpr size_t NOALLOC_BYTES = TB3_NOALLOC_SCRATCH_BYTES;
-__device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
+constexpr size_t NOALLOC_SPLIT_BYTES = 8 * CELL_SPLIT_MAX * sizeof(int) + 256;
+__device__ __align__(256) unsigned char scratch[NOALLOC_BYTES + NOALLOC_SPLIT_BYTES];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mutex;
@@ -418,10 +421,17 @@ struct Carver {
     }
 };
 
-// The per-cell arrays of the current grid, zeroed when allocated.
-void ensure_cell_buffers(tb3_ctx *c)
+bool cells_wide(const tb3_ctx *c, long long n);
+
+// Workgroups of the cell kernel that an XCD holds at once (5 or, wide, 2 per CU).
+int xcd_slots(const tb3_ctx *c, bool wide) { return std::max(1, c->ncu / 8 * (wide ? 2 : 5)); }
+
+// The per-cell arrays of the current grid, zeroed when allocated, and the
+// workgroup slots that its cells fill.
+void ensure_cell_buffers(tb3_ctx *c, int n)
 {
     CellGrid &g = c->grid;
+    g.xcd_slots = xcd_slots(c, cells_wide(c, n));
     if (g.ncell <= c->grid_cell_cap) return;
     ++c->epoch;
     auto carve = [&](unsigned char *base) {
@@ -445,7 +455,7 @@ void ensure_cell_buffers(tb3_ctx *c)
 void ensure_grid_buffers(tb3_ctx *c, int n)
 {
     CellGrid &g = c->grid;
-    ensure_cell_buffers(c);
+    ensure_cell_buffers(c, n);
     if (n > c->grid_n_cap) {
         ++c->epoch;
         auto carve = [&](unsigned char *base) {
@@ -548,18 +558,20 @@ int next_pow2(int v)
 // Whether the cell kernel of one system should start in its wide shape: from
 // the mean density, the particles within the cutoff of a cell's box that are
 // forward of it (all neighbours on a grid with a 3-cell dimension), and the
-// longest list (an owner in the corner nearest the forward cells sees ~85% of
+// longest list (an owner in the corner nearest the forward cells sees ~80% of
 // its cutoff sphere), with room for the fluctuations of a uniform system,
 // against what the narrow shape stages (256) and lists (96).  A neighbourhood
 // the wide shape could not stage either stays with the narrow one, which
 // hands its owners on.  Systems that are not uniform find out from the sweep
 // (grow_after_overflow).
 // Both sides: the wide shape costs a system that does not need it 7-15% of
-// its sweep (N = 32768 125 against 118 us, N = 1048576 3.5 against 3.0 ms), a
-// sweep that leaves a few owners to the dense-owner kernel 15-25 us.  So up to
-// WIDE_CELLS cells (sweeps of ~200 us) the room is for the largest cell, past
-// it for all but a few percent of the owners.  Where many owners need it:
-// 8000 particles, cutoff 2.5, 126 us against 192 with the narrow shape.
+// its sweep (N = 131072 434 against 377 us), a sweep that leaves a few owners
+// to the dense-owner kernel 15-25 us.  So up to WIDE_CELLS cells (sweeps of
+// ~200 us) the room is for the largest cell, past it for all but a few percent
+// of the owners.  Where many owners need it: 8000 particles, cutoff 2.5, 109 us
+// against 192 with the narrow shape; 4000 at cutoff 2.7 110 against 145.  Past
+// 460 staged on average most cells would be handed on in either: 20000 at
+// cutoff 2.75 510 us in both.
 constexpr int WIDE_CELLS = 3000;
 bool wide_expected(const CellGrid &g, double cutoff, long long n)
 {
@@ -584,35 +596,14 @@ bool wide_expected(const CellGrid &g, double cutoff, long long n)
                 4.0 / 3.0 * pi * c * c * c;
     const double density = (double)n / vol;
     const double staged = density * (three ? reach : 0.5 * (box + reach));
-    const double list = 0.85 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n);
-    if (staged > 416.0) return false;
+    const double list = 0.8 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n);
+    if (staged > 460.0) return false;
     const bool few = g.ncell <= WIDE_CELLS;
     const double zs = few ? std::sqrt(2.0 * std::log(std::max(g.ncell, 2))) + 0.3 : 2.0, zl = few ? 4.0 : 2.5;
     return staged + zs * std::sqrt(staged) > 256.0 || list + zl * std::sqrt(list) > 96.0;
 }
 
 bool cells_wide(const tb3_ctx *c, long long n) { return c->wide_need || wide_expected(c->grid, c->cutoff, n); }
-
-// Workgroups per cell: a grid whose cells do not fill the GPU's workgroup
-// slots (5 or, wide, 2 per CU) splits each cell's owners among several, which
-// each stage the cell's neighbourhood: just more workgroups than slots, down
-// to 2 owners each, and up to 16 parts, past which the parts' atomics on a
-// cell's few particles cost more (1 cell of 400: 16 parts 32 us, 64 48, 200
-// 101).  Kernel times at cutoff 2, density 2, with 1 and this many parts: 1
-// cell 181 -> 24 us, 64 cells 71 -> 27, 216 54 -> 30, 343 66 -> 43, 512 98 ->
-// 61, 729 86 -> 66, 1000 93 -> 85.  Past the slots a second staging costs more
-// than it spreads (1728 cells, 2 parts: 117 -> 135), except for the heaviest
-// cells, which would be the last to end: with a sixteenth of the cells in 2
-// parts, 1728 cells of 16 take 103 us instead of 114, of 19 116 instead of
-// 119; from 2.5 times the slots it makes no difference.
-CellSplit cell_split(const tb3_ctx *c, int ncell, long long n, bool wide)
-{
-    const int slots = c->ncu * (wide ? 2 : 5);
-    if (ncell <= 0 || ncell > slots * 5 / 2) return {0, 1};
-    if (ncell > slots) return {(ncell + 127) / 128, 2};
-    const long long own = (n + ncell - 1) / ncell;
-    return {ncell, (int)std::max<long long>(1, std::min<long long>({slots / ncell + 1, (own + 1) / 2, 16}))};
-}
 
 // The n x n table of pair lengths that the bit-exact all-triplets sweep reads
 // (16 bytes a pair, 256 MiB at the most).  Without it (more particles, or no
@@ -657,8 +648,8 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
             if (cut && c->cells_ok) {
                 const bool wide = cells_wide(c, d.n);
                 launch_p3bca_cells(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
-                                   energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0,
-                                   cell_split(c, c->grid.ncell, d.n, wide), slotted ? 1 : 0, parity);
+                                   energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0, slotted ? 1 : 0,
+                                   parity);
                 if (c->dense_on)
                     launch_p3bca_dense(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                        energy ? 1 : 0, c->d_owners, c->dense_grid, c->dense_waves);
@@ -742,9 +733,15 @@ bool grow_after_overflow(tb3_ctx *c, long long n)
     // per-owner kernel for this particle system from now on
     if (c->h_status->flags[3]) c->cells_ok = false;
     // owners that need the dense-owner kernel: launch it from now on
-    // (or, where its wide shape is enough, that)
-    if (c->h_status->want_dense == 1 && c->grid.ncell <= WIDE_CELLS && !cells_wide(c, n)) c->wide_need = true;
-    else if (c->h_status->want_dense) c->dense_on = true;
+    // (or, where the cell kernel's wide shape is enough, that).  Replicas that
+    // need it take both: their densities lie wide apart (48 clouds of up to
+    // 2048: 1.50 ms in both kernels, with the narrow shape 1.66)
+    if (c->h_status->want_dense == 1 && c->grid.ncell <= WIDE_CELLS && !cells_wide(c, n)) {
+        c->wide_need = true;
+    } else if (c->h_status->want_dense) {
+        c->dense_on = true;
+        if (c->nrep > 1) c->wide_need = true;
+    }
     const int need = c->h_status->flags[1];
     if (need > c->list_cap) {
         if (need > MAX_LIST)
@@ -807,7 +804,7 @@ bool slotted_pass(tb3_ctx *c, int n)
         return false;
     ensure_slot_buffers(c, n);
     if (c->grid.pad_cap == 0) return false;
-    ensure_cell_buffers(c);
+    ensure_cell_buffers(c, n);
     return true;
 }
 
@@ -1600,7 +1597,8 @@ struct NoallocLayout {
     long long *scan_tmp;
 };
 
-size_t noalloc_layout(unsigned char *base, long long n, int ncell, NoallocLayout *L)
+// `order_len` ints for the cells' order.
+size_t noalloc_layout(unsigned char *base, long long n, int ncell, NoallocLayout *L, long long order_len)
 {
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -1630,7 +1628,7 @@ size_t noalloc_layout(unsigned char *base, long long n, int ncell, NoallocLayout
     l.g.zs = reinterpret_cast<double *>(take(dn));
     l.g.cell_cnt = reinterpret_cast<int *>(take(cn));
     l.g.cell_start = reinterpret_cast<int *>(take(cn + sizeof(int)));
-    l.g.order = reinterpret_cast<int *>(take((size_t)cell_order_len(std::max(ncell, 1)) * sizeof(int)));
+    l.g.order = reinterpret_cast<int *>(take((size_t)order_len * sizeof(int)));
     l.g.cell_work = reinterpret_cast<unsigned *>(take(cn));
     l.g.scatter_ticket = reinterpret_cast<unsigned *>(take(sizeof(unsigned)));
     l.scan_tmp = reinterpret_cast<long long *>(
@@ -1666,11 +1664,13 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
         int nc[3];
         grid_shape(c, c->L, nc);
         const int ncell = nc[0] * nc[1] * nc[2];
-        const size_t need = noalloc_layout(base, n, ncell, &l);
+        const size_t need = noalloc_layout(base, n, ncell, nullptr, 8LL * cell_run_max(ncell) + 35);
         if (need > NOALLOC_BYTES)
             throw Fail(TB3_EINVAL, "the allocation-free call needs " + std::to_string(need) + " bytes of scratch "
                                    "for " + std::to_string(n) + " particles in " + std::to_string(ncell) +
                                    " cells; the scratch array holds " + std::to_string(NOALLOC_BYTES));
+        noalloc_layout(base, n, ncell, &l, cell_order_len(ncell));
+        l.g.xcd_slots = xcd_slots(c, false);
         CellGrid &g = l.g;
         for (int k = 0; k < 3; ++k) {
             g.nc[k] = nc[k];
@@ -1705,8 +1705,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             }
             if (n >= 3) {
                 if (cells) {
-                    launch_p3bca_cells(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, dense ? 1 : 0, wide ? 1 : 0,
-                                       cell_split(c, ncell, n, wide));
+                    launch_p3bca_cells(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, dense ? 1 : 0, wide ? 1 : 0);
                     if (dense)
                         launch_p3bca_dense(s, d, g, cs, nu, mixed, 1, l.st, 0, 1, l.owners, c->dense_grid,
                                            c->dense_waves);

@@ -23,16 +23,31 @@ struct DeviceState {
 // hold every particle within the periodic cutoff.
 // The cell kernel's dispatch order: one contiguous run of cells per XCD, the
 // runs cut to about equal work (so their lengths vary around ncell / 8),
-// each sorted heaviest first.  `order` holds 8 runs of cell_run_cap(ncell)
-// entries, then the 8 run lengths, then the 9 cuts (run r is cells
+// each sorted heaviest first, a heavy cell in several parts (order_runs).
+// `order` holds 8 runs of cell_run_cap(ncell) entries (the cell, in grids of
+// up to CELL_SPLIT_CELLS with its part in bits 16-23 and parts - 1 above), then the 8 run lengths, then the 9 cuts (run r is cells
 // [cut r, cut r+1)) that the last integrating pass's update computed, then
 // two more sets of 9 that replays on the slotted layout alternate between.
-__host__ __device__ inline int cell_run_cap(int ncell)
+constexpr int CELL_SPLIT_CELLS = 8192;  // the largest grids that split cells
+constexpr int CELL_SLOTS_MAX = 160;     // workgroup slots of an XCD that the parts are counted for
+// Entries a run may have beyond one per cell: a part of every cell per slot and
+// cell (up to half as many again where the cuts are uneven), and the extra ones
+// of heavy cells.
+constexpr int CELL_SPLIT_MAX = 2 * CELL_SLOTS_MAX + CELL_SLOTS_MAX;
+__host__ __device__ inline int cell_run_max(int ncell)
 {
     const int run = (ncell + 7) / 8;
     return run + (run + 1) / 2;
 }
-__host__ __device__ inline long long cell_order_len(int ncell) { return 8LL * cell_run_cap(ncell) + 35; }
+__host__ __device__ inline int cell_run_cap(int ncell)
+{
+    return cell_run_max(ncell) + (ncell <= CELL_SPLIT_CELLS ? CELL_SPLIT_MAX : 0);
+}
+// Ints of `order` that serve every grid of up to ncell cells.
+__host__ __device__ inline long long cell_order_len(int ncell)
+{
+    return 8LL * (cell_run_max(ncell) + CELL_SPLIT_MAX) + 35;
+}
 
 struct CellGrid {
     int nc[3] = {1, 1, 1};
@@ -45,6 +60,7 @@ struct CellGrid {
     unsigned *scatter_ticket = nullptr;  // 1: finished scatter workgroups (returns to 0)
     int *cell_start = nullptr;  // ncell + 1
     int *order = nullptr;       // cell_order_len(ncell): the runs, their lengths and the cuts (above)
+    int xcd_slots = 0;          // workgroups of the cell kernel that an XCD holds at once
     unsigned *cell_work = nullptr;  // ncell: accepted triplets of each cell's last sweep (0: none yet)
     int *cell_idx = nullptr;    // n, particle indices grouped by cell (order within a cell unspecified)
     double *xs = nullptr, *ys = nullptr, *zs = nullptr;  // n, positions in cell_idx order
@@ -206,13 +222,9 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
                        int cap, int mixed, int grad, Status *st, int count_slot, int want_energy);
 void launch_p3bca_exact(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int cap, Status *st);
-// The first `head` cells of each XCD's run are split among `parts` workgroups.
-struct CellSplit {
-    int head, parts;
-};
-// Fast cutoff sweep, one workgroup per cell or `split`, in the narrow or the wide
-// shape (4 waves, 256 staged particles and lists of 96; 8 waves, 416 and
-// 144).  With dense_on, owners it cannot stage go to `owners` for
+// Fast cutoff sweep, a workgroup per entry of the grid's order, in the narrow
+// or the wide shape (4 waves, 256 staged particles and lists of 96; 8 waves,
+// 512 and 136).  With dense_on, owners it cannot stage go to `owners` for
 // launch_p3bca_dense, which must follow on the same stream; without, such an
 // owner sets st->want_dense and st->flags[2] (the caller re-runs the pass in
 // the wide shape or with the dense-owner kernel).  Non-finite positions set
@@ -221,7 +233,7 @@ struct CellSplit {
 // `slotted`: sweep the slotted layout (needs dense_on == 0).
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, CellSplit split, int slotted = 0, int parity = -1);
+                        int wide, int slotted = 0, int parity = -1);
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
 int p3bca_cells_blocks_per_cu();
 // The cell kernel hands owners whose neighbourhood does not fit its LDS

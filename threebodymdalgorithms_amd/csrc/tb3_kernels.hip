@@ -308,7 +308,7 @@ __device__ void compute_cuts(int ncell, const Count &count, const unsigned *__re
                              float *fpart, int *cut, bool write_out = true)
 {
     const int t = threadIdx.x;
-    const int run = (ncell + 7) >> 3, cap = cell_run_cap(ncell);
+    const int run = (ncell + 7) >> 3, cap = cell_run_max(ncell);
     auto work = [&](int c) {
         const unsigned w = cell_work[c];
         if (w) return (float)w;
@@ -369,33 +369,72 @@ __device__ void compute_cuts(int ncell, const Count &count, const unsigned *__re
 // (order[8 cap + 8 ...]), which the caller loaded into cut[0..8] early
 // (overlapping that load with its own), if they fit this grid; else each
 // run takes ncell / 8 cells.  256 threads; LDS: hist (256 ints), cut (9
-// ints).
+// ints), fpart (4 floats).
+//
+// A cell of work w gets 1 + w / T entries, a workgroup each, T being its run's
+// work over split.extra, within split.least and split.most: so that cells
+// fewer than the XCD's workgroup slots fill it, and a heavy cell does not
+// outlast the rest.  At most least entries per cell and extra more.  Sweep
+// kernels at cutoff 2, density 2, unsplit and split: 1 cell of 129 181 -> 24
+// us, 64 cells 71 -> 27, 216 61 -> 33, 512 93 -> 53, 1000 92 -> 70, 1728 of 16
+// particles 114 -> 100; 48 clouds of up to 2048 in 3422 cells, most of them
+// almost empty, 446 -> 139.
+struct CellSplit {
+    int least, most, extra;
+};
+
 template <class Count>
 __device__ void order_runs(int ncell, const Count &count, const unsigned *__restrict__ cell_work,
-                           int *__restrict__ order, int *hist, int *cut, int r0, int rstep)
+                           int *__restrict__ order, int *hist, int *cut, float *fpart, CellSplit split, int r0,
+                           int rstep)
 {
     if (r0 >= 8) return;
     const int t = threadIdx.x;
     const int run = (ncell + 7) >> 3, cap = cell_run_cap(ncell);
-    auto bin = [&](int c) {
+    auto load = [&](int c) {
         const unsigned w = cell_work[c];
         const float n = (float)count(c);
-        const float k = w ? (float)w : 16.0f * n * n;
-        return 255 - min(255, (int)(16.0f * __log2f(1.0f + k)));
+        return fmaxf(1.0f, w ? (float)w : 16.0f * n * n);
     };
     __syncthreads();  // the caller's cut[] stores
     if (t == 0) {
         bool ok = cut[0] == 0 && cut[8] == ncell;
-        for (int r = 0; r < 8 && ok; ++r) ok = cut[r + 1] >= cut[r] && cut[r + 1] - cut[r] <= cap;
+        for (int r = 0; r < 8 && ok; ++r) ok = cut[r + 1] >= cut[r] && cut[r + 1] - cut[r] <= cell_run_max(ncell);
         if (!ok)
             for (int r = 0; r <= 8; ++r) cut[r] = min(r * run, ncell);
     }
     __syncthreads();
     for (int r = r0; r < 8; r += rstep) {
         const int lo = cut[r], hi = cut[r + 1];
+        // a thread's first cells stay in registers over the three walks
+        constexpr int HELD = 4;
+        float held[HELD];
+#pragma unroll
+        for (int k = 0; k < HELD; ++k) held[k] = lo + t + 256 * k < hi ? load(lo + t + 256 * k) : 0.0f;
+        auto walk = [&](auto body) {
+#pragma unroll
+            for (int k = 0; k < HELD; ++k)
+                if (lo + t + 256 * k < hi) body(lo + t + 256 * k, held[k]);
+            for (int c = lo + t + 256 * HELD; c < hi; c += 256) body(c, load(c));
+        };
+        float inv = 0.0f;  // 1 / T
+        if (split.extra > 0) {
+            float sum = 0.0f;
+            walk([&](int, float w) { sum += w; });
+#pragma unroll
+            for (int o = WAVE / 2; o; o >>= 1) sum += __shfl_xor(sum, o);
+            if ((t & (WAVE - 1)) == 0) fpart[t / WAVE] = sum;
+            __syncthreads();
+            inv = (float)split.extra / ((fpart[0] + fpart[1]) + (fpart[2] + fpart[3]));
+        }
+        auto parts = [&](float w) { return min(split.most, max(split.least, 1 + (int)(w * inv))); };
+        auto bin = [&](float w) { return 255 - min(255, (int)(16.0f * __log2f(1.0f + w))); };
         hist[t] = 0;
         __syncthreads();
-        for (int c = lo + t; c < hi; c += 256) atomicAdd(&hist[bin(c)], 1);
+        walk([&](int, float w) {
+            const int p = parts(w);
+            atomicAdd(&hist[bin(w)], p);
+        });
         __syncthreads();
         // exclusive scan of the 256 bins, one per thread (Hillis-Steele)
         const int own = hist[t];
@@ -405,17 +444,20 @@ __device__ void order_runs(int ncell, const Count &count, const unsigned *__rest
             hist[t] += u;
             __syncthreads();
         }
+        if (t == 255) order[8 * cap + r] = hist[t];
         hist[t] -= own;
         __syncthreads();
-        for (int c = lo + t; c < hi; c += 256) order[r * cap + atomicAdd(&hist[bin(c)], 1)] = c;
-        if (t == 0) order[8 * cap + r] = hi - lo;
+        walk([&](int c, float w) {
+            const int p = parts(w), at = r * cap + atomicAdd(&hist[bin(w)], p);
+            for (int k = 0; k < p; ++k) order[at + k] = p > 1 ? c | k << 16 | (p - 1) << 24 : c;
+        });
         __syncthreads();
     }
 }
 
 // Grids of at most this many cells scan their counts inside the scatter
 // kernel (k_cell_scatter_fused) and may replay on the slotted layout.
-constexpr int FUSED_SCAN_CELLS = 8192;
+constexpr int FUSED_SCAN_CELLS = CELL_SPLIT_CELLS;
 
 // The slotted cell layout (CellGrid::pad_cap) as the kernels see it.
 struct SlotsDev {
@@ -791,14 +833,16 @@ __global__ __launch_bounds__(256) void k_begin_steps_slotted(Status *st, unsigne
 // swept weigh alike).
 __global__ __launch_bounds__(256) void k_bin_slotted(DeviceState d, PassStart a, GridDev g, SlotsDev sl, Status *st,
                                                      int ncell, const unsigned *__restrict__ cell_work,
-                                                     int *__restrict__ order)
+                                                     int *__restrict__ order, CellSplit split)
 {
     const int nbin = (int)gridDim.x - 8;
     if ((int)blockIdx.x >= nbin) {
         __shared__ int hist[256], cut[9];
+        __shared__ float fpart[4];
         int *cuts = order + 8 * cell_run_cap(ncell) + 8;
         if (threadIdx.x <= 8) cut[threadIdx.x] = cuts[threadIdx.x];
-        order_runs(ncell, [](int) { return 0; }, cell_work, order, hist, cut, (int)blockIdx.x - nbin, 8);
+        order_runs(ncell, [](int) { return 0; }, cell_work, order, hist, cut, fpart, split, (int)blockIdx.x - nbin,
+                   8);
         // the cuts the first replayed update orders with (epoch 0's set)
         if (blockIdx.x == nbin && threadIdx.x <= 8) cuts[9 + threadIdx.x] = cut[threadIdx.x];
         return;
@@ -887,7 +931,7 @@ __global__ __launch_bounds__(NSLOT) void k_update_bin(DeviceState d, double hdt,
                                                      int *__restrict__ cell_cnt, int *__restrict__ cell_rank,
                                                      int ncell, const int *__restrict__ cell_start,
                                                      const unsigned *__restrict__ cell_work, int *__restrict__ order,
-                                                     SlotsDev sl)
+                                                     SlotsDev sl, CellSplit split)
 {
     // The particles' workgroups, then: (slotted) 8 that order the next
     // sweep's runs; one that cuts the XCD runs from this sweep's work; one
@@ -940,7 +984,7 @@ __global__ __launch_bounds__(NSLOT) void k_update_bin(DeviceState d, double hdt,
         int *par = cuts + 9;
         if (x < 8) {
             if (threadIdx.x <= 8) cut[threadIdx.x] = par[(e & 1u) * 9 + threadIdx.x];
-            order_runs(ncell, count, cell_work, order, hist, cut, x, 8);
+            order_runs(ncell, count, cell_work, order, hist, cut, fpart, split, x, 8);
         } else {
             compute_cuts(ncell, count, cell_work, par + ((e + 1u) & 1u) * 9, fpart, cut);
         }
@@ -966,9 +1010,10 @@ __global__ __launch_bounds__(256) void k_cell_scatter(int n, const double *__res
                                                       int *__restrict__ order, const unsigned *__restrict__ cell_work)
 {
     __shared__ int hist[256], cut[9];
+    __shared__ float fpart[4];
     if (threadIdx.x <= 8) cut[threadIdx.x] = order[8 * cell_run_cap(ncell) + 8 + threadIdx.x];
-    order_runs(ncell, [&](int c) { return cell_start[c + 1] - cell_start[c]; }, cell_work, order, hist, cut,
-               blockIdx.x, gridDim.x);
+    order_runs(ncell, [&](int c) { return cell_start[c + 1] - cell_start[c]; }, cell_work, order, hist, cut, fpart,
+               CellSplit{1, 1, 0}, blockIdx.x, gridDim.x);
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const int c = cell_of[p];
@@ -995,8 +1040,9 @@ __global__ __launch_bounds__(256) void k_cell_scatter_fused(
     const int *__restrict__ cell_of, const int *__restrict__ cell_rank, int *__restrict__ cell_cnt,
     int *__restrict__ cell_start, int *__restrict__ cell_idx, double *__restrict__ xs, double *__restrict__ ys,
     double *__restrict__ zs, int ncell, int *__restrict__ order, const unsigned *__restrict__ cell_work,
-    unsigned *__restrict__ ticket, int nsc, const Status *__restrict__ st)
+    unsigned *__restrict__ ticket, int nsc, const Status *__restrict__ st, CellSplit split)
 {
+    __shared__ float fpart[4];
     __shared__ int lst[FUSED_SCAN_CELLS + 1];
     __shared__ int part[256];
     __shared__ int hist[256], cut[9];
@@ -1046,8 +1092,8 @@ __global__ __launch_bounds__(256) void k_cell_scatter_fused(
         for (int c = t; c <= ncell; c += 256) cell_start[c] = lst[c];
     if (blockIdx.x >= nsc) {
         if (t <= 8) cut[t] = gcut;
-        order_runs(ncell, [&](int c) { return lst[c + 1] - lst[c]; }, cell_work, order, hist, cut, blockIdx.x - nsc,
-                   8);
+        order_runs(ncell, [&](int c) { return lst[c + 1] - lst[c]; }, cell_work, order, hist, cut, fpart, split,
+                   blockIdx.x - nsc, 8);
     }
 
     if (p < n) {
@@ -1384,11 +1430,11 @@ __global__ __launch_bounds__(WAVE) void k_p3bca_fast(CutDev a)
 // Fast cutoff sweep, one cell per workgroup (the default fast kernel).
 //
 // Ownership: each accepted triplet belongs to the one particle that sees both
-// others "forward": in its own cell at a later slot, or in a forward
-// neighbour cell (the half shell of positive stencil offsets, or of larger
-// cell index on grids with a 3-cell dimension; see below).  One workgroup
-// per cell c stages in LDS c's particles followed by those particles of c's
-// forward cells that lie within the cutoff of c's box: every particle
+// others "forward": in its own cell later in the owners' order (owner_key),
+// or in a forward neighbour cell (the half shell of positive stencil offsets,
+// or of larger cell index on grids with a 3-cell dimension; see below).  One
+// workgroup per cell c stages in LDS c's particles in that order, then those
+// particles of c's forward cells that lie within the cutoff of c's box: every particle
 // forward of an owner in c and within the cutoff of it is in this range.
 // Each wave then claims owners i of cell c, collects i's candidates t > i
 // within the cutoff (a contiguous LDS range, no search) into a contiguous
@@ -1403,17 +1449,17 @@ __global__ __launch_bounds__(WAVE) void k_p3bca_fast(CutDev a)
 // owner whose list is longer than LCAP, are queued for the dense-owner
 // kernel below instead.
 //
-// Where cells are few, or the heaviest would outlast the rest, the owners of
-// the first `head` cells of each XCD's run are split among `parts` workgroups
-// (part k takes owners k, k + parts, ...), each with its own staging.
+// Where cells are few, or the heaviest would outlast the rest, the owners of a
+// cell are split among `parts` workgroups (order_runs; part k takes every
+// parts-th owner), each with its own staging.
 //
 // Bound by VALU issue (70% at N = 1048576) beside LDS, with latencies between
 // them: a fifth wave per SIMD, which is what keeps the workgroup's LDS within
 // 32000 bytes (the queue holds one batch, the particles' numbers wait in
 // registers), takes N = 1048576 at cutoff 2 from 2810 to 2680 us and 25001 in
-// FP32-mixed from 108 to 94; three rows of 5 waves per workgroup instead,
-// 3485.  Of the 2680, 300 are staging, 440 the owners' lists, 690 the tests of
-// pairs and 1260 the evaluations.
+// FP32-mixed from 108 to 94; 4 workgroups of 5 waves instead, 3485.  Of the
+// 2680, 300 are staging, 440 the owners' lists, 690 the tests of pairs and 1260
+// the evaluations.
 
 struct CellsDev {
     CutDev c;
@@ -1424,17 +1470,16 @@ struct CellsDev {
     const int *order;  // each XCD's run of cells, heaviest first (k_cell_scatter)
     unsigned *cell_work;  // each cell's accepted triplets, the next sweep's dispatch key
     SlotsDev sl;          // the slotted layout (cap > 0: staged from its slot records)
-    int head, parts;      // the first cells of each XCD's run, each split among this many workgroups
 };
 
 // The two shapes of the cell kernel: waves of a workgroup, staged particles
 // and entries of a wave's list (list positions fit in the 8-bit halves of a
 // queue entry).  20 waves per CU in 5 workgroups with 32 KB of LDS each, or 16
-// in 2 with 79 KB, for neighbourhoods that the narrow one would leave to one
+// in 2 with 80 KB, for neighbourhoods that the narrow one would leave to one
 // 8-wave workgroup per owner (k_p3bca_dense).
 template <bool WIDE>
 struct CellShape {
-    static constexpr int W = WIDE ? 8 : 4, NB = WIDE ? 416 : 256, LC = WIDE ? 144 : 96;
+    static constexpr int W = WIDE ? 8 : 4, NB = WIDE ? 512 : 256, LC = WIDE ? 136 : 96;
 };
 
 // An owner that needs the dense-owner kernel when none follows this launch:
@@ -1535,6 +1580,18 @@ __device__ __forceinline__ void cell_geometry(const SysGrid &sg, int c, int k, d
     geo[4 * k + 3] = L / (double)n;
 }
 
+// Particles of one cell own their triplets among each other in the order of
+// this key (ties by slot): those near the faces towards the forward cells,
+// which have the most forward neighbours there, come last.  That evens the
+// lists out (at density 2 and cutoff 2 33 +- 10.6 entries, in the order of the
+// slots 33 +- 14.8; the longest of 8000 particles at cutoff 2.5 105 instead of
+// 129), which saves pairs to test and owners for the dense-owner kernel: N =
+// 32768 116 -> 112 us, 8000 at cutoff 2.5 126 -> 109.
+__device__ __forceinline__ double owner_key(double x, double y, double z)
+{
+    return __builtin_fma(0.3, y, __builtin_fma(0.1, x, z));
+}
+
 // Squared distance for the cutoff test.  PER: the periodic form
 // min(t, L - t) per component (Algorithm.cpp's cutoff test).  !PER: the plain
 // difference, which gives the same bits whenever every |difference| is below
@@ -1561,30 +1618,24 @@ __device__ __forceinline__ int staged_slot(const int *cst, const int *cpre, int 
     return cst[k] + (t - cpre[k]);
 }
 
-// Cell for workgroup b, or -1: workgroups are dispatched round-robin over
-// the 8 XCDs (b % 8), so each XCD gets a contiguous run of cells, whose
-// neighbourhoods overlap in its own L2, of about an eighth of the work, and
-// takes them heaviest first (order_runs).  The first `head` cells of a run
-// are each split among `parts` workgroups.
-__device__ __forceinline__ int cell_for_block(int b, int ncell, const int *order, int head, int &part, int &parts)
+// Cell for workgroup b, or -1, and which of how many parts of it: workgroups
+// are dispatched round-robin over the 8 XCDs (b % 8), so each XCD gets a
+// contiguous run of cells, whose neighbourhoods overlap in its own L2, of
+// about an eighth of the work, and takes them heaviest first (order_runs).
+__device__ __forceinline__ int cell_for_block(int b, int ncell, const int *order, int &part, int &parts)
 {
     const int cap = cell_run_cap(ncell);
-    const int r = b & 7;
-    int k = b >> 3;
-    if (k < head * parts) {
-        part = k % parts;
-        k /= parts;
-    } else {
-        k -= head * (parts - 1);
-        part = 0;
-        parts = 1;
-    }
+    const int r = b & 7, k = b >> 3;
     if (k >= cap || k >= order[8 * cap + r]) return -1;
-    return order[r * cap + k];
+    const int e = order[r * cap + k];
+    const bool may = ncell <= FUSED_SCAN_CELLS;
+    part = may ? e >> 16 & 0xff : 0;
+    parts = may ? 1 + (e >> 24) : 1;
+    return may ? e & 0xffff : e;
 }
 
 template <class T, bool GRAD, bool WANT_E, bool WIDE>
-__global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(CellsDev a)
+__global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bca_cells(CellsDev a)
 {
     constexpr int CELL_WAVES = CellShape<WIDE>::W, NBCAP = CellShape<WIDE>::NB, LCAP = CellShape<WIDE>::LC;
     using StagedIndex = typename std::conditional<(NBCAP > 256), unsigned short, unsigned char>::type;
@@ -1600,11 +1651,11 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     __shared__ unsigned short ring[CELL_WAVES][WAVE];
     __shared__ int cst[32], cpre[33], sinfo[4];
     __shared__ int s_next, s_far, s_wcnt[2][CELL_WAVES];
-    __shared__ unsigned s_work;
+    __shared__ unsigned s_work, s_long[(NBCAP + 31) / 32];
 
     const CutDev &A = a.c;
-    int part, parts = a.parts;
-    const int c = cell_for_block(blockIdx.x, a.ncell, a.order, a.head, part, parts);
+    int part, parts;
+    const int c = cell_for_block(blockIdx.x, a.ncell, a.order, part, parts);
     if (c < 0) return;
     const int tid = threadIdx.x, lane = lane_id(), wv = tid / WAVE;
     // A halted step-graph replay leaves the step to the host.  Non-finite
@@ -1646,7 +1697,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     // workgroups' arithmetic (C1 sweep 120.7 -> 117.5 us; the same priority
     // for the evaluations made it 130 us, for the owners' list builds 121 us).
     __builtin_amdgcn_s_setprio(3);
-    double *geo = wls[0][1];  // until wave 0's first list
+    double *geo = wls[0][1], *keys = wls[0][2];  // until wave 0's first list
     if (wv == 0) stage_cells(A, sg, c, cst, cpre, sinfo, scnt, a.sl.cap);
     if (wv == 1 && lane < 3) cell_geometry(sg, c, lane, geo);
     __syncthreads();
@@ -1662,6 +1713,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     // every dimension, so the cutoff tests may use plain differences
     // (cut_sq<false>); a particle outside (a wrapped neighbour cell, or one
     // outside the box) sends the workgroup to the periodic form.
+    if (tid < (NBCAP + 31) / 32) s_long[tid] = 0;
     if (tid == 0) {
         s_next = 0;
         s_work = 0;
@@ -1726,8 +1778,12 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                 s_wcnt[0][wv] = __popcll(m0);
                 s_wcnt[1][wv] = __popcll(m1);
             }
+            const bool mine = t0 == 0 && tid < own && own <= NBCAP;
+            const double key = owner_key(x[0], y[0], z[0]);
+            if (mine) keys[tid] = key;
             __syncthreads();
             // the kept candidates of the first half, then of the second, in order
+            // (c's own at their places in the owners' order)
             int pos[2] = {total + lane_prefix(m0), lane_prefix(m1)};
             for (int h = 0; h < 2; ++h) {
                 if (h == 1) pos[1] += total;
@@ -1737,14 +1793,19 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
                     total += k;
                 }
             }
+            if (mine && total <= NBCAP) {
+                pos[0] = 0;
+                for (int j = 0; j < own; ++j) pos[0] += keys[j] < key || (keys[j] == key && j < tid) ? 1 : 0;
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
+                const int t = t0 + h * NT + tid;
                 if (keep[h] && pos[h] < NBCAP) {
                     const int p = pos[h];
                     nx[p] = x[h];
                     ny[p] = y[h];
                     nz[p] = z[h];
-                    wls[p / WAVE][0][p % WAVE] = __longlong_as_double(q[h]);
+                    wls[p / WAVE][0][p % WAVE] = __longlong_as_double((long long)t << 32 | (unsigned)q[h]);
                     gxs[p] = 0.0;
                     gys[p] = 0.0;
                     gzs[p] = 0.0;
@@ -1770,9 +1831,10 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
         return;
     }
     __syncthreads();
-    // staged particle tid's number waits in a register for the end; its wave's
-    // list, not yet in use, brought it
-    const int my_id = tid < total ? (int)__double_as_longlong(wls[wv][0][lane]) : 0;
+    // staged particle tid's number and place among the candidates wait in
+    // registers for the end; its wave's list, not yet in use, brought them
+    const long long mine = tid < total ? __double_as_longlong(wls[wv][0][lane]) : 0;
+    const int my_id = (int)mine, my_cand = (int)(mine >> 32);
 
     // 3. owners of cell c, claimed one at a time by the waves; the cutoff
     // tests take the plain form unless the staging found a far particle
@@ -1784,8 +1846,9 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
         for (;;) {
             int i = 0;
             if (lane == 0) i = atomicAdd(&s_next, 1);
-            i = part + parts * __builtin_amdgcn_readfirstlane(i);
-            if (i >= own) break;
+            // the last in the owners' order, which have the longest lists, first
+            i = own - 1 - part - parts * __builtin_amdgcn_readfirstlane(i);
+            if (i < 0) break;
             const double xi = nx[i], yi = ny[i], zi = nz[i];
 
             // the owner's forward candidates within the cutoff, in staging
@@ -1817,7 +1880,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
             if (len > LCAP) {
                 // too long for this wave's list: the dense-owner kernel takes i
                 if (lane == 0) {
-                    if (a.dense_on) a.owners[atomicAdd(&A.st->dense_n, 1)] = sinfo[0] + i;
+                    if (a.dense_on) atomicOr(&s_long[i >> 5], 1u << (i & 31));
                     else want_dense_kernel(A.st, len <= CellShape<true>::LC);
                 }
                 continue;
@@ -1937,6 +2000,9 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
     else owners(std::false_type{});
     __syncthreads();
 
+    if (a.dense_on && tid < own && (s_long[tid >> 5] >> (tid & 31) & 1u))
+        a.owners[atomicAdd(&A.st->dense_n, 1)] = sinfo[0] + my_cand;
+
     // 4. add the staged particles' gradients to global memory.  Staged
     // particles that no owner of c paired with (many in the edge and corner
     // cells) hold exact zeros and are skipped: f starts at +0.0, and adding
@@ -1970,7 +2036,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, 4) void k_p3bca_cells(Cel
 //
 // One owner per workgroup of DW waves (4, 8 or 16: a tuning knob), taken from the queue the
 // cell kernel filled.  The owner's list is the same forward set the cell
-// kernel would have used (its own cell's later slots, then the forward
+// kernel would have used (those of its cell after it in the owners' order, then the forward
 // neighbour cells, within the cutoff), gathered from the cell-ordered
 // positions into LDS by all waves; the list's unordered pairs are then split
 // over the workgroup's waves in folded order, pair (r, (r + o) mod len) for
@@ -2067,11 +2133,14 @@ __global__ __launch_bounds__(DW *WAVE, 4) void k_p3bca_dense(DenseDev a)
         const int slot = w.slot, i = slot - w.info[0], nk = w.info[2], total = w.info[3];
         const double xi = a.xs[slot], yi = a.ys[slot], zi = a.zs[slot];
 
-        // the owner's forward list; when all of it lies within 0.24 L of the
+        // the owner's forward list (of its own cell, the particles after it in
+        // the owners' order); when all of it lies within 0.24 L of the
         // owner in every dimension, any two entries differ by less than L / 2
         // and the pair tests take the plain form
         bool far = false;
-        for (int t0 = i + 1; t0 < total; t0 += NT) {
+        const int mates = w.info[1];
+        const double key = owner_key(xi, yi, zi);
+        for (int t0 = 0; t0 < total; t0 += NT) {
             const int t = t0 + tid;
             bool ok = t < total;
             double xt = 0.0, yt = 0.0, zt = 0.0;
@@ -2083,6 +2152,10 @@ __global__ __launch_bounds__(DW *WAVE, 4) void k_p3bca_dense(DenseDev a)
                 zt = a.zs[st];
                 st = A.cell_idx[st];
                 ok = !(sqr_dist_periodic_min(xi, yi, zi, xt, yt, zt, Lx, Ly, Lz) > c2);
+                if (t < mates) {
+                    const double kt = owner_key(xt, yt, zt);
+                    ok = ok && (kt > key || (kt == key && t > i));
+                }
             }
             const unsigned long long m = __ballot(ok);
             int base = 0;
@@ -3197,6 +3270,22 @@ void launch_scan_i32(hipStream_t s, const int *in, int *out, int count, long lon
     scan_rec<int, int>(s, in, count, out, (long long)count + 1, tmp);
 }
 
+// How a grid's cells are split.  Fewer cells than the XCDs have workgroup
+// slots: every cell of a single system into just more workgroups than slots,
+// down to 2 owners each, and up to 16, past which their atomics on a cell's few
+// particles cost more (1 cell of 400: 16 parts 32 us, 64 48, 200 101).
+// Replicas differ too much for that, and every grid's heaviest cells go
+// further (order_runs), by the extra parts that two thirds of the slots hold.
+// (Parts by work alone leave a uniform grid near the number of slots with
+// fewer: 343 cells in the wide shape 202 us instead of 186.)
+static CellSplit cell_split(const CellGrid &g, int n)
+{
+    if (g.ncell > CELL_SPLIT_CELLS || g.ncell <= 0) return {1, 1, 0};
+    const int run = (g.ncell + 7) / 8, own = (n + g.ncell - 1) / g.ncell, slots = std::min(g.xcd_slots, CELL_SLOTS_MAX);
+    const int least = run <= slots && g.nrep <= 1 ? std::min({slots / run + 1, (own + 1) / 2, 16}) : 1;
+    return {std::max(least, 1), std::min(16, own + 1), slots * 2 / 3};
+}
+
 bool cells_fused_scan(const CellGrid &g) { return g.ncell <= FUSED_SCAN_CELLS; }
 
 void launch_bin_ranked(hipStream_t s, const DeviceState &d, int predict, double dt, int zero_f, CellGrid &g,
@@ -3213,7 +3302,7 @@ void launch_scatter_fused(hipStream_t s, const DeviceState &d, CellGrid &g, Stat
     const int nsc = blocks_for(d.n, 256);
     hipLaunchKernelGGL(k_cell_scatter_fused, dim3(nsc + 8), dim3(256), 0, s, d.n, d.x, d.y, d.z, g.cell_of,
                        g.cell_rank, g.cell_cnt, g.cell_start, g.cell_idx, g.xs, g.ys, g.zs, g.ncell, g.order,
-                       g.cell_work, g.scatter_ticket, nsc, st);
+                       g.cell_work, g.scatter_ticket, nsc, st, cell_split(g, d.n));
 }
 
 void launch_update_bin(hipStream_t s, const DeviceState &d, double hdt, const double g3[3], Status *st,
@@ -3224,7 +3313,7 @@ void launch_update_bin(hipStream_t s, const DeviceState &d, double hdt, const do
     const unsigned nb = (d.n > 0 ? blocks_for(d.n, NSLOT) : 1) + (slotted ? 10 : 2);
     hipLaunchKernelGGL(k_update_bin, dim3(nb), dim3(NSLOT), 0, s, d, hdt, g3[0], g3[1], g3[2], st, sum_roles, dt,
                        h, zero_f, grid_dev(g), g.cell_of, g.cell_cnt, g.cell_rank, g.ncell, g.cell_start,
-                       g.cell_work, g.order, slots_dev(&g, slotted));
+                       g.cell_work, g.order, slots_dev(&g, slotted), cell_split(g, d.n));
 }
 
 void launch_bin_slotted(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
@@ -3233,7 +3322,7 @@ void launch_bin_slotted(hipStream_t s, const DeviceState &d, const double *rows,
     // the particles' workgroups, then 8 that order the first sweep's cells
     const unsigned nb = (d.n > 0 ? blocks_for(d.n, 256) : 0) + 8;
     hipLaunchKernelGGL(k_bin_slotted, dim3(nb), dim3(256), 0, s, d, pass_start(rows, predict, dt, zero_f), grid_dev(g),
-                       slots_dev(&g, 1, parity), st, g.ncell, g.cell_work, g.order);
+                       slots_dev(&g, 1, parity), st, g.ncell, g.cell_work, g.order, cell_split(g, d.n));
 }
 
 void launch_cells_build(hipStream_t s, const DeviceState &d, const double *rows, int predict, double dt, int zero_f,
@@ -3296,7 +3385,7 @@ void launch_p3bca_fast(hipStream_t s, const DeviceState &d, const CellGrid &g, c
 
 void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, const CutoffSpec &c, double nu,
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
-                        int wide, CellSplit split, int slotted, int parity)
+                        int wide, int slotted, int parity)
 {
     if (d.n <= 0) return;
     CellsDev a;
@@ -3312,10 +3401,8 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
     a.cell_work = g.cell_work;
     a.sl = slots_dev(&g, slotted, parity);
     // the 8 XCDs' runs at their capacity (the workgroups past a run's length exit at once)
-    const int cap = cell_run_cap(g.ncell);
-    a.parts = split.parts;
-    a.head = split.parts > 1 ? min(split.head, cap) : 0;
-    const dim3 gr((unsigned)(8 * (cap + (a.parts - 1) * a.head)));
+    const CellSplit sp = cell_split(g, d.n);
+    const dim3 gr((unsigned)(8 * (cell_run_max(g.ncell) * sp.least + sp.extra)));
 #define TB3_CELLS(T, G, E)                                                                                \
     do {                                                                                                  \
         if (wide) hipLaunchKernelGGL((k_p3bca_cells<T, G, E, true>), gr, dim3(CellShape<true>::W * WAVE), 0, s, a); \
