@@ -72,9 +72,9 @@ __device__ __forceinline__ double wave_total(double v)
 }
 
 // Number of set bits of m below this lane.
-__device__ __forceinline__ int lane_prefix(unsigned long long m)
+__device__ __forceinline__ int lane_prefix(unsigned long long m, int base = 0)
 {
-    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)base));
 }
 
 // Orders this wave's LDS writes before its later LDS reads by other lanes
@@ -1689,7 +1689,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
     const SysGrid sg = grid_of_cell(A.g, c);
     const double Lx = sg.L[0], Ly = sg.L[1], Lz = sg.L[2];
     double esum = 0.0;
-    unsigned cnt = 0;
+    unsigned cnt = 0;  // this wave's triplets, in every lane
 
     // 1. the staged cells: c first, then its forward neighbour cells.
     // Staging is a chain of memory round trips; at the top wave priority
@@ -1865,7 +1865,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
                     ok = !(cut_sq<PER>(xi, yi, zi, xt, yt, zt, Lx, Ly, Lz) > c2);
                 }
                 const unsigned long long m = __ballot(ok);
-                const int pos = len + lane_prefix(m);
+                const int pos = lane_prefix(m, len);
                 if (ok && pos < LCAP) {
                     list[pos] = (StagedIndex)t;
                     qx[pos] = xt;
@@ -1928,25 +1928,29 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
                             lds_add(&hz[kk], __builtin_fma(cv, dkz, tz));
                         }
                         if (WANT_E) esum += (double)et;
-                        ++cnt;
                     }
                     wave_sync();
+                    cnt += (unsigned)nq;
                 };
                 // 64 / len and lane / len from one FP32 reciprocal: for
                 // len <= LCAP the fraction of (k + 0.5) / len stays 0.5 / len
                 // away from an integer, far beyond the FP32 rounding
                 const float inv = 1.0f / (float)len;
                 const int q64 = (int)(64.5f * inv), r64 = WAVE - q64 * len;
-                int o = (int)(((float)lane + 0.5f) * inv);
-                int r = lane - o * len;
-                ++o;
+                // unsigned: x - len of an x < len is past every x, so a minimum
+                // takes x mod len of an x < 2 len
+                const unsigned ulen = (unsigned)len;
+                auto wrap = [&](unsigned x) { return min(x, x - ulen); };
+                const unsigned step = wrap((unsigned)(r64 + q64));
+                unsigned r = (unsigned)(int)(((float)lane + 0.5f) * inv);
+                unsigned kk = r + 1;  // o
+                r = (unsigned)lane - r * ulen;
+                kk = wrap(r + kk);
                 auto test = [&](bool live) {
-                    int kk = r + o;
-                    kk = kk >= len ? kk - len : kk;
-                    kk = live ? kk : r;  // lanes past the last item read their own entry
-                    const bool ok = live && !(cut_sq<PER>(qx[r], qy[r], qz[r], qx[kk], qy[kk], qz[kk], Lx, Ly, Lz) > c2);
+                    const unsigned k = live ? kk : r;  // lanes past the last item read their own entry
+                    const bool ok = live && !(cut_sq<PER>(qx[r], qy[r], qz[r], qx[k], qy[k], qz[k], Lx, Ly, Lz) > c2);
                     const unsigned long long m = __ballot(ok);
-                    const int at = qn + lane_prefix(m);
+                    const int at = lane_prefix(m, qn);
                     if (ok && at < WAVE) rq[at] = (unsigned short)(r | (kk << 8));
                     qn += __popcll(m);
                     if (qn >= WAVE) {
@@ -1954,12 +1958,9 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
                         if (ok && at >= WAVE) rq[at - WAVE] = (unsigned short)(r | (kk << 8));
                         qn -= WAVE;
                     }
-                    r += r64;
-                    o += q64;
-                    if (r >= len) {
-                        r -= len;
-                        ++o;
-                    }
+                    r += (unsigned)r64;
+                    kk = wrap(kk + step + (r >= ulen ? 1u : 0u));
+                    r = wrap(r);
                 };
                 // whole rounds of 64 items, then the last partial round
                 const int full = npairs & ~(WAVE - 1);
@@ -2018,7 +2019,7 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
             }
         }
     }
-    const unsigned long long cw = wave_sum_u64(cnt);
+    const unsigned long long cw = cnt;
     const double ee = WANT_E ? wave_sum(esum) : 0.0;
     if (lane == 0) {
         if (WANT_E) add_energy(A.st, ee);
