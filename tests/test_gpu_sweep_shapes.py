@@ -206,3 +206,18 @@ def test_cutoff_uneven_cells(eng, oracle, n):
     eng.configure("p3bca", cutoff=2.0, domain_L=L, precision="fp64")
     for _ in range(3):
         check(eng, oracle, P, "fp64", cutoff=2.0, L=L)
+
+
+@pytest.mark.parametrize("crowded", [False, True])
+def test_cutoff_large_grid_slots(eng, oracle, crowded):
+    """9261 cells, past those of the fused scan: single passes fill the slots
+    there too, and go back to the contiguous list where a cell outgrows them."""
+    n = 42875
+    P = jittered(n, 77, sd=0.1)
+    if crowded:
+        P[:40] = 7.0 + np.random.default_rng(78).uniform(0.0, 1.2, (40, 3))
+    L = np.full(3, 28.0)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=1.3, domain_L=L, precision="fp64")
+    for _ in range(2):
+        check(eng, oracle, P, "fp64", cutoff=1.3, L=L)
