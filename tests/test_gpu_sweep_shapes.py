@@ -221,3 +221,23 @@ def test_cutoff_large_grid_slots(eng, oracle, crowded):
     eng.configure("p3bca", cutoff=1.3, domain_L=L, precision="fp64")
     for _ in range(2):
         check(eng, oracle, P, "fp64", cutoff=1.3, L=L)
+
+
+@pytest.mark.parametrize("n", [1, 4096, 4097])
+def test_particles_through_the_stage(eng, oracle, n):
+    """Up to 4096 particles and the forces of a sweep pass through pinned
+    memory, more through copies: the same bits come back."""
+    rng = np.random.default_rng(n)
+    P = jittered(n, 6000 + n) if n > 1 else np.full((1, 3), 0.4)
+    V, A, M = rng.normal(size=(n, 3)), rng.normal(size=(n, 3)), rng.uniform(1, 2, n)
+    eng.set_particles(P, V, A, M, ids=np.arange(n)[::-1])
+    L = np.full(3, 0.8 * np.ceil(round(n ** (1 / 3), 9)))
+    eng.configure("p3bca", cutoff=1.5, domain_L=L, precision="fp64")
+    S = oracle.force_scale(P, cutoff=1.5, L=L)
+    _, f, _, _ = eng.energy_grad()
+    got = eng.get_particles()
+    for key, want in (("pos", P), ("vel", V), ("acc", A), ("mass", M), ("id", np.arange(n)[::-1])):
+        assert np.array_equal(got[key], want), key
+    assert np.array_equal(got["f"], f)
+    *_, fo, _ = oracle.sweep(P, cutoff=1.5, L=L, mode="owner")
+    assert (np.abs(f - fo) <= 1e-12 * np.maximum(S, 1e-300)[:, None]).all()

@@ -141,7 +141,10 @@ struct Status {
 };
 
 // ---- launchers (all asynchronous on `s`) ----
-void launch_soa_from_rows(hipStream_t s, int n, const double *rows, double *x, double *y, double *z);
+void launch_state_in(hipStream_t s, const DeviceState &d, const double *pos, const double *vel, const double *acc,
+                     const double *mass);
+void launch_state_out(hipStream_t s, const DeviceState &d, double *pos, double *vel, double *acc, double *f,
+                      double *mass);
 void launch_rows_from_soa(hipStream_t s, int n, const double *x, const double *y, const double *z, double *rows);
 // Clears the status block (and halt); keep_nonfinite preserves flags[0].
 void launch_reset_status(hipStream_t s, Status *st, int keep_nonfinite);

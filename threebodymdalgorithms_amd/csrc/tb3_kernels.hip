@@ -119,14 +119,34 @@ __device__ __forceinline__ void note_list_length(Status *st, int len, int cap)
 // ---------------------------------------------------------------------------
 // Layout conversion, integrator, status.
 
-__global__ void k_soa_from_rows(int n, const double *__restrict__ rows, double *__restrict__ x,
-                                double *__restrict__ y, double *__restrict__ z)
+// The particles in from n x 3 rows and out to them, consecutive threads on
+// consecutive elements of the rows: those may lie in pinned host memory, where
+// the kernel takes the place of the copies.  k_state_in also clears the forces.
+// A null array is left out.
+__global__ void k_state_in(DeviceState d, const double *__restrict__ pos, const double *__restrict__ vel,
+                           const double *__restrict__ acc, const double *__restrict__ mass)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    x[p] = rows[3 * (long long)p + 0];
-    y[p] = rows[3 * (long long)p + 1];
-    z[p] = rows[3 * (long long)p + 2];
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3LL * d.n) return;
+    const int p = (int)(t / 3), k = (int)(t - 3LL * p);
+    (k == 0 ? d.x : (k == 1 ? d.y : d.z))[p] = pos[t];
+    (k == 0 ? d.vx : (k == 1 ? d.vy : d.vz))[p] = vel[t];
+    (k == 0 ? d.ax : (k == 1 ? d.ay : d.az))[p] = acc[t];
+    (k == 0 ? d.fx : (k == 1 ? d.fy : d.fz))[p] = 0.0;
+    if (mass && t < d.n) d.m[t] = mass[t];
+}
+
+__global__ void k_state_out(DeviceState d, double *__restrict__ pos, double *__restrict__ vel,
+                            double *__restrict__ acc, double *__restrict__ f, double *__restrict__ mass)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3LL * d.n) return;
+    const int p = (int)(t / 3), k = (int)(t - 3LL * p);
+    if (pos) pos[t] = (k == 0 ? d.x : (k == 1 ? d.y : d.z))[p];
+    if (vel) vel[t] = (k == 0 ? d.vx : (k == 1 ? d.vy : d.vz))[p];
+    if (acc) acc[t] = (k == 0 ? d.ax : (k == 1 ? d.ay : d.az))[p];
+    if (f) f[t] = (k == 0 ? d.fx : (k == 1 ? d.fy : d.fz))[p];
+    if (mass && t < d.n) mass[t] = d.m[t];
 }
 
 __global__ void k_rows_from_soa(int n, const double *__restrict__ x, const double *__restrict__ y,
@@ -3185,10 +3205,18 @@ size_t p3bca_exact_lds(int cap)
     return (size_t)cap * (sizeof(int) + 3 * sizeof(double) + (exact_roots(cap) ? sizeof(double2) : 0));
 }
 
-void launch_soa_from_rows(hipStream_t s, int n, const double *rows, double *x, double *y, double *z)
+void launch_state_in(hipStream_t s, const DeviceState &d, const double *pos, const double *vel, const double *acc,
+                     const double *mass)
 {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_soa_from_rows, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, rows, x, y, z);
+    if (d.n <= 0) return;
+    hipLaunchKernelGGL(k_state_in, dim3(blocks_for(3LL * d.n, 256)), dim3(256), 0, s, d, pos, vel, acc, mass);
+}
+
+void launch_state_out(hipStream_t s, const DeviceState &d, double *pos, double *vel, double *acc, double *f,
+                      double *mass)
+{
+    if (d.n <= 0) return;
+    hipLaunchKernelGGL(k_state_out, dim3(blocks_for(3LL * d.n, 256)), dim3(256), 0, s, d, pos, vel, acc, f, mass);
 }
 
 void launch_rows_from_soa(hipStream_t s, int n, const double *x, const double *y, const double *z, double *rows)
