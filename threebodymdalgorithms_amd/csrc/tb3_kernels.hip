@@ -1587,17 +1587,15 @@ __device__ void stage_cells(const CutDev &A, const SysGrid &sg, int c, int *cst,
     }
 }
 
-// The geometry of cell c along dimension k for the staging's box test: its
-// cell coordinate, the cells per length, 1 / cells, and the cell width.
-__device__ __forceinline__ void cell_geometry(const SysGrid &sg, int c, int k, double *geo)
+// The geometry of a cell along a dimension of n cells and length L for the
+// staging's box test: its cell coordinate, the cells per length, 1 / cells, and
+// the cell width.
+__device__ __forceinline__ void cell_geometry(int coord, int n, double L, double *geo)
 {
-    const int lc = c - sg.cbase;
-    const int n = k == 0 ? sg.nc[0] : (k == 1 ? sg.nc[1] : sg.nc[2]);
-    const double L = k == 0 ? sg.L[0] : (k == 1 ? sg.L[1] : sg.L[2]);
-    geo[4 * k + 0] = (double)(k == 0 ? lc % sg.nc[0] : (k == 1 ? lc / sg.nc[0] % sg.nc[1] : lc / (sg.nc[0] * sg.nc[1])));
-    geo[4 * k + 1] = (double)n / L;
-    geo[4 * k + 2] = 1.0 / (double)n;
-    geo[4 * k + 3] = L / (double)n;
+    geo[0] = (double)coord;
+    geo[1] = (double)n / L;
+    geo[2] = 1.0 / (double)n;
+    geo[3] = L / (double)n;
 }
 
 // Particles of one cell own their triplets among each other in the order of
@@ -1606,10 +1604,11 @@ __device__ __forceinline__ void cell_geometry(const SysGrid &sg, int c, int k, d
 // lists out (at density 2 and cutoff 2 33 +- 10.6 entries, in the order of the
 // slots 33 +- 14.8; the longest of 8000 particles at cutoff 2.5 105 instead of
 // 129), which saves pairs to test and owners for the dense-owner kernel: N =
-// 32768 116 -> 112 us, 8000 at cutoff 2.5 126 -> 109.
+// 32768 116 -> 112 us, 8000 at cutoff 2.5 126 -> 109.  (y by 0.3 to 0.5 and x
+// by 0.1 to 0.25 sweep alike.)
 __device__ __forceinline__ double owner_key(double x, double y, double z)
 {
-    return __builtin_fma(0.3, y, __builtin_fma(0.1, x, z));
+    return __builtin_fma(0.4, y, __builtin_fma(0.15, x, z));
 }
 
 // Squared distance for the cutoff test.  PER: the periodic form
@@ -1719,7 +1718,12 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
     __builtin_amdgcn_s_setprio(3);
     double *geo = wls[0][1], *keys = wls[0][2];  // until wave 0's first list
     if (wv == 0) stage_cells(A, sg, c, cst, cpre, sinfo, scnt, a.sl.cap);
-    if (wv == 1 && lane < 3) cell_geometry(sg, c, lane, geo);
+    // (a wave for each dimension: picked by a lane's index, the grid would be
+    // written to scratch memory by every thread first)
+    const int lc = c - sg.cbase;
+    if (wv == 1 && lane == 0) cell_geometry(lc % sg.nc[0], sg.nc[0], Lx, geo);
+    if (wv == 2 && lane == 0) cell_geometry(lc / sg.nc[0] % sg.nc[1], sg.nc[1], Ly, geo + 4);
+    if (wv == 3 && lane == 0) cell_geometry(lc / (sg.nc[0] * sg.nc[1]), sg.nc[2], Lz, geo + 8);
     __syncthreads();
     const int cand = sinfo[3], own = sinfo[1], nk = sinfo[2];
 
