@@ -219,9 +219,11 @@ tb3_status tb3_get_tuning(const tb3_ctx *ctx, double *cell_ratio, int *blocks_pe
  * counterpart in the reference. */
 tb3_status tb3_set_tuning(tb3_ctx *ctx, double cell_ratio, int dense_waves);
 
-/* The slotted cell layout of tb3_run's replayed steps (fast cutoff sweep on
- * one system, grids of up to 8192 cells, no dense-owner kernel): each cell
- * keeps `slots` slots that the binning pass fills directly, so that a step
+/* The slotted cell layout of tb3_run's replayed steps and of single passes
+ * (fast cutoff sweep on one system, no dense-owner kernel; replays: grids of
+ * up to 8192 cells; single passes: larger ones too, from 4 particles per cell
+ * and up to 2 GiB of slots): each cell keeps `slots` slots that the binning
+ * pass fills directly, so that a step
  * runs no scatter pass between the binning and the sweep.  slots = -1 picks
  * three times the mean cell count (at least 32), 0 turns the layout off,
  * 1 .. 256 sets it; TB3_EINVAL otherwise.  A step in which some cell gets
