@@ -241,3 +241,31 @@ def test_particles_through_the_stage(eng, oracle, n):
     assert np.array_equal(got["f"], f)
     *_, fo, _ = oracle.sweep(P, cutoff=1.5, L=L, mode="owner")
     assert (np.abs(f - fo) <= 1e-12 * np.maximum(S, 1e-300)[:, None]).all()
+
+
+def test_batch_after_single_passes(eng, oracle):
+    """A single pass leaves the status clear, but not the sums of replicas that
+    are split off after it: each replica's first counts and energies are those
+    of the replica alone."""
+    reps = [jittered(n, 7000 + n, sd=0.1) for n in (40, 3, 150, 9)]
+    P = np.concatenate(reps)
+    for first in range(2):  # the second batch meets the first one's tables
+        eng.set_particles(P)
+        eng.configure("p3bca", cutoff=1.7, precision="fp64")
+        eng.energy_grad()
+        eng.batch_set(np.concatenate([[0], np.cumsum([len(r) for r in reps])]))
+        if first == 0:
+            _, f, _, total = eng.energy_grad()
+            counts = eng.batch_counts()
+        else:
+            E, counts = eng.batch_energy()
+            assert float(E.sum()) == pytest.approx(alone_E, rel=1e-10)
+        alone, alone_E = [], 0.0
+        for r in reps:
+            eng.set_particles(r)
+            e, _, _, c = eng.energy_grad()
+            alone.append(c)
+            alone_E += e
+        assert [int(c) for c in counts] == alone
+        if first == 0:
+            assert total == sum(alone)

@@ -843,8 +843,8 @@ unsigned long long run_pass(tb3_ctx *c, hipStream_t s, DeviceState &d, bool inte
     if (slotted && !c->slots_clean) {
         launch_begin_steps(s, c->d_status, c->d_counts, &c->grid);
         c->slots_parity = 0;
-    } else if (!c->status_clean) {
-        launch_reset_status(s, c->d_status, 0);
+    } else if (!c->status_clean || c->nrep > 1) {
+        launch_reset_status(s, c->d_status, 0);  // (a clear status says nothing of the replicas' sums)
     }
     c->status_clean = false;
     const int parity = slotted ? c->slots_parity : -1;
