@@ -269,3 +269,26 @@ def test_batch_after_single_passes(eng, oracle):
         assert [int(c) for c in counts] == alone
         if first == 0:
             assert total == sum(alone)
+
+
+@pytest.mark.parametrize("nu", ["number", "host tensor", "device tensor"])
+def test_energy_waits_for_the_positions(eng, nu):
+    """Positions that torch's default stream is still about to write: the
+    energy is that of the written ones, wherever nu's value lives."""
+    import torch
+    from threebodymdalgorithms_amd.autograd import at_energy
+    P, Q = jittered(500, 1), jittered(500, 2)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=2.0, domain_L=np.full(3, 6.4), precision="fp64")
+    x, q = torch.tensor(P, device="cuda"), torch.tensor(Q, device="cuda")
+    nus = {"number": 1.0, "host tensor": torch.tensor(1.0, dtype=torch.float64),
+           "device tensor": torch.tensor(1.0, dtype=torch.float64, device="cuda")}
+    want = float(at_energy(q, 1.0, eng))
+    a = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(20):
+        a = a @ a * 1e-2
+    x.copy_(q)
+    with torch.no_grad():
+        got = at_energy(x, nus[nu], eng)
+    assert float(got) == pytest.approx(want, rel=1e-10)

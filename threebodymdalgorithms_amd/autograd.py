@@ -19,8 +19,16 @@ import torch
 from .engine import Engine
 
 
-def _stream_handle(device):
-    return torch.cuda.current_stream(device).cuda_stream
+def _stream_handle(device, done=False):
+    """torch's current stream for the engine.  The handle of the default stream
+    is 0, for which the engine takes a stream of its own that waits for
+    nothing: what torch queued there (the positions' producers, the last users
+    of memory that comes back in a new tensor) is waited for here, unless the
+    caller has just done so (a value read from the device)."""
+    stream = torch.cuda.current_stream(device)
+    if stream.cuda_stream == 0 and not done:
+        stream.synchronize()
+    return stream.cuda_stream
 
 
 def _check_pos(pos):
@@ -36,15 +44,15 @@ class _Energy(torch.autograd.Function):
         _check_pos(pos)
         pos_c = pos.detach().contiguous()
         nu_v = float(nu)
+        stream = _stream_handle(pos.device, done=nu.device == pos.device)
         E = torch.empty((), dtype=torch.float64, device=pos.device)
         grad = None
         if ctx.needs_input_grad[0]:
             # one sweep gives E and dE/dx together; backward only scales it
             grad = torch.empty_like(pos_c)
-            engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), grad.data_ptr(),
-                                   _stream_handle(pos.device))
+            engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), grad.data_ptr(), stream)
         else:
-            engine.energy_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), _stream_handle(pos.device))
+            engine.energy_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), stream)
         ctx.engine = engine
         ctx.nu_v = nu_v
         ctx.has_grad = grad is not None
@@ -84,10 +92,10 @@ class _Forces(torch.autograd.Function):
         _check_pos(pos)
         pos_c = pos.detach().contiguous()
         nu_v = float(nu)
+        stream = _stream_handle(pos.device, done=nu.device == pos.device)
         E = torch.empty((), dtype=torch.float64, device=pos.device)
         grad = torch.empty_like(pos_c)
-        engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), grad.data_ptr(),
-                               _stream_handle(pos.device))
+        engine.energy_grad_dev(pos_c.shape[0], pos_c.data_ptr(), nu_v, E.data_ptr(), grad.data_ptr(), stream)
         ctx.nu_v = nu_v
         ctx.engine = engine
         ctx.save_for_backward(grad, pos_c)
