@@ -317,6 +317,16 @@ void grid_shape(const tb3_ctx *c, const double *L, int nc[3])
     }
 }
 
+// Device memory set to zero, done on return.  (hipMemset does not wait for
+// device memory, and its null stream may be behind another program's work,
+// while the context's kernels run on streams that do not wait for that one:
+// the zeros could land on counts and orders that a pass has already written.)
+void clear_now(tb3_ctx *c, void *p, size_t bytes)
+{
+    HIPCHK(hipMemsetAsync(p, 0, bytes, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+}
+
 // Publishes the replica tables (or their absence) to the status block.
 void publish_replicas(tb3_ctx *c)
 {
@@ -390,7 +400,7 @@ void configure_grid(tb3_ctx *c)
         same = same && g.nc[k] == old_nc[k] && g.lo[k] == old_lo[k] && g.L[k] == old_L[k];
     // the per-cell work of the last sweep belongs to the old cell numbering
     if (!same && g.cell_work && g.ncell <= c->grid_cell_cap)
-        HIPCHK(hipMemset(g.cell_work, 0, (size_t)g.ncell * sizeof(unsigned)));
+        clear_now(c, g.cell_work, (size_t)g.ncell * sizeof(unsigned));
     c->cells_ok = true;  // a new grid gets a new chance at the cell kernel
     c->wide_need = false;
     c->dense_on = false;
@@ -453,7 +463,7 @@ void ensure_cell_buffers(tb3_ctx *c, int n)
     const size_t bytes = carve(nullptr);
     c->grid_cell_cap = 0;
     dev_alloc(c->cell_block, (long long)bytes);
-    HIPCHK(hipMemset(c->cell_block, 0, bytes));
+    clear_now(c, c->cell_block, bytes);
     carve(c->cell_block);
     c->grid_cell_cap = g.ncell;
 }
