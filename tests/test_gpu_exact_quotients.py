@@ -1,0 +1,157 @@
+"""The bit-exact precision where its shortened division is at its limit:
+denominators a few ulp under a power of two.
+
+The division refines an approximate reciprocal once and is within half an ulp
+and 2^-92 of 1 / b, so over b = 2^k (1 - t 2^-53) the reciprocal itself may be
+misrounded for odd t < 128, and the quotient with it if the numerator is the
+one whose quotient lies next to a midpoint (a power of two for t = 1).  The
+compiler's division refines its own estimate the same way and is wrong for t =
+5, 11 and 13.  The numerators 5 d and 3 nu of the brackets can be any number, and 5 d is a power
+of two for sides 0.1, 0.2, 0.4, 0.8, 1.6.  All comparisons are bit for bit."""
+import math
+
+import numpy as np
+import pytest
+
+import threebodymdalgorithms_amd as tb3
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    with tb3.Engine(0) as e:
+        yield e
+
+
+def hard_numerators(t, far=9):
+    """Mantissas A in [2^52, 2^53) for which A / (2^53 - t), t odd, lies next
+    to the midpoint of two doubles: (2^53 - t) M + e = A 2^k for small odd e."""
+    B = 2 ** 53 - t
+    out = set()
+    for bits in (53, 54):
+        m = 2 ** bits
+        inv = pow(B, -1, m)
+        for e in range(-far, far + 1, 2):
+            A = (B * (-e * inv % m) + e) // m
+            out |= {A << s for s in (0, 1) if 2 ** 52 <= A << s < 2 ** 53}
+    return sorted(out)
+
+
+def test_quotients_next_to_midpoints(eng):
+    """The worst numerators over every denominator 2^53 - t, with the
+    constants of the brackets, at several exponents."""
+    a, b = [], []
+    for t in range(1, 256, 2):
+        for A in hard_numerators(t) + [2 ** 52, 3 * 2 ** 51, 5 * 2 ** 50]:
+            for ea, eb in ((0, 0), (1, 40), (2, -90)):
+                for sign in (1.0, -1.0):
+                    a += 2 * [sign * math.ldexp(A, ea - 52)]
+                    b += 2 * [math.ldexp(2 ** 53 - t, eb - 52)]
+    a, b = np.array(a), np.array(b)
+    _, q = eng.selftest_fp64_inrange(a, b)
+    assert np.array_equal(q, a / b), int(np.sum(q != a / b))
+    _, q, _ = eng.selftest_fp64(a, b)
+    assert np.array_equal(q, a / b), int(np.sum(q != a / b))
+
+
+def powers_product(x, z):
+    """x^6 z^5 as the brackets form it."""
+    px = pz = 1.0
+    for _ in range(6):
+        px *= x
+    for _ in range(5):
+        pz *= z
+    return px * pz
+
+
+def place(x, d, z):
+    """k for i = 0, j = (x, 0, 0) with |k| = d and |k - j| = z as computed in
+    FP64, or None."""
+    kx = (x * x + d * d - z * z) / (2 * x)
+    if d * d <= kx * kx:
+        return None
+    ky = math.sqrt(d * d - kx * kx)
+    step = np.arange(-12, 13)
+    X = (kx + step * math.ulp(kx))[:, None]
+    Y = (ky + step * math.ulp(ky))[None, :]
+    ok = (np.sqrt(X * X + Y * Y) == d) & (np.sqrt((x - X) * (x - X) + (0.0 - Y) * (0.0 - Y)) == z)
+    at = np.argwhere(ok)
+    return None if len(at) == 0 else (X[at[0][0], 0], Y[0, at[0][1]], 0.0)
+
+
+def triangles():
+    """Sides x, z next to 1 whose x^6 z^5 has the mantissa 2^53 - t, and the
+    side d whose 5 d is a power of two (t = 1) or a hard numerator."""
+    near = [1.0 + i * 2.0 ** -52 for i in range(0, 9)] + [1.0 - i * 2.0 ** -53 for i in range(1, 17)]
+    by_t = {}
+    for x in near:
+        for z in near:
+            B = math.frexp(powers_product(x, z))[0] * 2 ** 53
+            t = int(2 ** 53 - B)
+            if t % 2 and t < 64:
+                by_t.setdefault(t, []).append((x, z))
+    out = []
+    for t, sides in sorted(by_t.items()):
+        ds = [0.2, 0.4, 0.8, 1.6] if t == 1 else []
+        for A in hard_numerators(t, 3):
+            d = math.ldexp(A, -52) / 5
+            for v in (np.nextafter(d, 0), d, np.nextafter(d, 9)):
+                v = float(v)
+                if math.frexp(5 * v)[0] * 2 ** 53 == A:
+                    ds += [v * s for s in (0.5, 1.0, 2.0, 4.0) if 0.15 < v * s < 1.95]
+        for x, z in sides[:12]:
+            for d in ds:
+                k = place(x, d, z)
+                if k is not None:
+                    out.append(np.array([(0.0, 0.0, 0.0), (x, 0.0, 0.0), k]))
+    # the same among random neighbours by a few ulp
+    rng = np.random.default_rng(5)
+    one, d = float.fromhex("0x1.ffffffffffffbp-1"), 1.6
+    k0 = (float.fromhex("-0x1.1eb851eb851f4p-2"), float.fromhex("0x1.eb851eb851ebbp-1"))
+    out.append(np.array([(0.0, 0.0, 0.0), (one, 0.0, 0.0), (*k0, 0.0)]))
+    for _ in range(3000):
+        i, j, k = rng.integers(-8, 9, 3)
+        out.append(np.array([(0.0, 0.0, 0.0), (one + i * 2.0 ** -53, 0.0, 0.0),
+                             (k0[0] + j * 2.0 ** -54, k0[1] + k * 2.0 ** -53, 0.0)]))
+    return out
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2), (1, 2, 0), (2, 0, 1)])
+def test_triangles_through_both_sweeps(eng, oracle, order):
+    """As replicas of the cutoff sweep all at once, and (every 16th and the
+    placed ones) alone through the all-triplets sweep, each corner in turn as
+    the first particle."""
+    tri = [t[list(order)] for t in triangles()]
+    want = []
+    for t in tri:
+        *_, fo, cnt = oracle.sweep(t, mode="owner")
+        assert cnt == 1
+        want.append(fo)
+    P = np.concatenate(tri)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=4.0, domain_L=np.full(3, 11.0), precision="exact")
+    eng.batch_set(3 * np.arange(len(tri) + 1))
+    assert eng.compute_forces() == len(tri)
+    f = eng.get_particles()["f"].reshape(-1, 3, 3)
+    wrong = [i for i in range(len(tri)) if not np.array_equal(f[i], want[i])]
+    assert not wrong, (len(wrong), len(tri), wrong[:5])
+    for i in [i for i in range(len(tri)) if i % 16 == 0 or i < len(tri) - 3000]:
+        eng.set_particles(tri[i])
+        eng.configure("auta", precision="exact")
+        eng.compute_forces()
+        assert np.array_equal(eng.get_particles()["f"], want[i]), i
+
+
+@pytest.mark.parametrize("t", [1, 3, 5, 11, 13, 25])
+def test_coefficient_over_a_side(eng, oracle, t):
+    """3 nu / (8 d) with a side d = 1 - t 2^-53 and the hard numerators 3 nu."""
+    side = 1.0 - t * 2.0 ** -53
+    P = np.array([(0.0, 0.0, 0.0), (side, 0.0, 0.0), (0.4, 0.9, 0.1), (0.0, -side, 0.0)])
+    for A in hard_numerators(t, 3):
+        for nu in (math.ldexp(A, -52) / 3, float(np.nextafter(math.ldexp(A, -52) / 3, 0))):
+            *_, fo, _ = oracle.sweep(P, nu=nu, mode="owner")
+            eng.set_particles(P)
+            eng.configure("auta", nu=nu, precision="exact")
+            eng.compute_forces()
+            assert np.array_equal(eng.get_particles()["f"], fo), (nu, t)

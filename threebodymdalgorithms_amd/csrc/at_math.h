@@ -81,11 +81,21 @@ __device__ __forceinline__ double sqr_dist_periodic_min(double ax, double ay, do
 // away, so with b scaled to [1, 2) that is at most ulp(q) b 2^-55 (1 + 2^-38),
 // while a quotient that is no midpoint is at least ulp(q) 2^-53 / b away from
 // it: it falls on the right side for b^2 < 4 (1 - 2^-38).  Left are b within
-// 2^-38 of 2, b = 2 - t 2^-52, whose reciprocal is misrounded for odd
-// t < 128 only; over those, in exact rational arithmetic, the result is wrong
-// just for t = 1 (a mantissa of all ones) under a power of two.  Callers
-// whose numerator may be one send the denominators with an all-ones low word
-// (div_needs_ieee) to the IEEE division.
+// 2^-38 of 2, b = 2 - t 2^-52.  There 1 / b is t^2 2^-107 past a midpoint of
+// two doubles for odd t, and the refinement, short of 1 / b by 2^-93, rounds
+// to the other side of it for odd t < 128 (how far past a midpoint the caller's
+// r has to be off: t / 2 ulp); a correctly rounded reciprocal gives the right
+// quotient.  Over those t the quotient is wrong for the one numerator that
+// comes next to a midpoint: a power of two for t = 1, some other mantissa for
+// t = 5, 11, 13, 25, ... 123, never 3 or 5 (all r within 2^-46, in exact
+// rational arithmetic).  Callers whose numerator may be anything but those
+// two send the denominators whose low word says that they may lie within 128
+// steps under a power of two (div_is_hard) to div_rn.
+//
+// div_rn is the compiler's division with that set right: its reciprocal comes
+// from two refinements of the estimate and is misrounded over t = 5, 11 and
+// 13, so over the same denominators the exact remainders of the quotient and of
+// its neighbour decide between the two (no quotient is a midpoint).
 //
 // The square root likewise: sqrt(x) rescales x when it is tiny and passes
 // +-0 and +inf through around a Newton iteration on the reciprocal
@@ -94,10 +104,9 @@ __device__ __forceinline__ double sqr_dist_periodic_min(double ax, double ay, do
 // instead of 17).  Its by-product h, half the reciprocal root, gives
 // 1 / sqrt(x) to within 2^-52 in two more, from whose powers the reciprocals
 // of the brackets' denominators are formed.
-// Both are checked bit for bit against the compiler's IEEE expansions on the
-// device (tb3_selftest_fp64_inrange).
+// Both are checked bit for bit on the device (tb3_selftest_fp64_inrange).
 __device__ __forceinline__ unsigned low_word(double b) { return (unsigned)__double_as_longlong(b); }
-__device__ __forceinline__ bool div_needs_ieee(unsigned low) { return low == 0xffffffffu; }
+__device__ __forceinline__ bool div_is_hard(unsigned low) { return low >= 0xffffff80u; }
 
 __device__ __forceinline__ double div_rn_from(double a, double b, double r)
 {
@@ -105,6 +114,17 @@ __device__ __forceinline__ double div_rn_from(double a, double b, double r)
     const double q = a * r;
     const double rem = __builtin_fma(-b, q, a);
     return __builtin_fma(rem, r, q);
+}
+
+__device__ __forceinline__ double div_rn(double a, double b)
+{
+    const double q = a / b, rem = __builtin_fma(-b, q, a);
+    const long long away = (rem < 0.0) == (a < 0.0) ? 1 : -1;  // from zero, where |a| > |b q|
+    const double next = __longlong_as_double(__double_as_longlong(q) + away);
+    // (a remainder below 2^-960 may not be exact)
+    const bool nearer =
+        (__builtin_fabs(rem) >= 0x1p-960) & (__builtin_fabs(__builtin_fma(-b, next, a)) < __builtin_fabs(rem));
+    return div_is_hard(low_word(b)) & nearer ? next : q;
 }
 
 __device__ __forceinline__ double sqrt_rn_inrange(double x, double &inv)
@@ -148,21 +168,22 @@ __device__ __forceinline__ RefSide ref_powers(double d1, double i1)
     return p;
 }
 
-// a / b: IEEE division, or the in-range sequence from r, the product of the
+// a / b: the division proper, or the in-range sequence from r, the product of the
 // sides' reciprocal powers (rounded powers and products: within 40 ulp of
 // 1 / b), when the caller has checked the operands' range.
 template <bool INRANGE>
 __device__ __forceinline__ double ref_div(double a, double b, double r)
 {
     if constexpr (INRANGE) return div_rn_from(a, b, r);
-    else return a / b;
+    else return div_rn(a, b);
 }
 
 // One dVdR bracket (AxilrodTeller.cpp:68-81) for own side x and the two other
 // sides y, z in the order the source names them: dVdRa = (a; b, c),
 // dVdRb = (b; a, c), dVdRc = (c; b, a).  Left-to-right sums and products.
 // `low` collects the largest low word of the denominators whose numerators
-// are powers of two (or may be: 3 nu), for div_needs_ieee.
+// are or may be other than 3 and 5 (powers of two, 6, 5 d and 3 nu), for
+// div_is_hard.
 template <bool INRANGE>
 __device__ __forceinline__ double ref_bracket(double nu, const RefSide &x, const RefSide &y, const RefSide &z,
                                               unsigned &low)
@@ -182,17 +203,19 @@ __device__ __forceinline__ double ref_bracket(double nu, const RefSide &x, const
         r3 = (r5 * x4) * y.d3;
         r4 = (r6 * x4) * z.d3;
     }
-    const double b1 = x.d4 * y.d3 * z.d3, b2 = y.d5 * z.d5, b5 = x.d2 * y.d3 * z.d5, b6 = x.d2 * y.d5 * z.d3;
+    const double b1 = x.d4 * y.d3 * z.d3, b2 = y.d5 * z.d5, b3 = x.d6 * z.d5, b4 = x.d6 * y.d5;
+    const double b5 = x.d2 * y.d3 * z.d5, b6 = x.d2 * y.d5 * z.d3;
     const double b0 = 8. * x.d1;
     if constexpr (INRANGE) {
         low = max(max(low, low_word(b1)), low_word(b2));
+        low = max(max(low, low_word(b3)), low_word(b4));
         low = max(max(low, low_word(b5)), low_word(b6));
         low = max(low, low_word(b0));
     }
     double t = ref_div<INRANGE>(-8., b1, r1);
     t = t - ref_div<INRANGE>(1., b2, r5 * a);
-    t = t + ref_div<INRANGE>(5. * y.d1, x.d6 * z.d5, r3);
-    t = t + ref_div<INRANGE>(5. * z.d1, x.d6 * y.d5, r4);
+    t = t + ref_div<INRANGE>(5. * y.d1, b3, r3);
+    t = t + ref_div<INRANGE>(5. * z.d1, b4, r4);
     t = t - ref_div<INRANGE>(1., b5, r5);
     t = t - ref_div<INRANGE>(1., b6, r6);
     t = t - ref_div<INRANGE>(3., x.d4 * y.d1 * z.d5, r5 * ai);
@@ -253,7 +276,8 @@ __device__ __forceinline__ double2 ref_root(double sq)
 
 // The contribution, given the three sides' ref_root.  The in-range sequences
 // run where the sides and nu allow them (nu_ok = nu_inrange(nu), hoisted by
-// the caller), the IEEE expansions elsewhere: the same bits either way.
+// the caller) and no denominator is a hard one, div_rn and the compiler's root
+// elsewhere: the same bits either way.
 template <int ROLE>
 __device__ __forceinline__ void ref_contrib(double xp, double yp, double zp, double xe, double ye, double ze,
                                             double xo, double yo, double zo, double2 ss, double2 st, double2 sm,
@@ -267,7 +291,7 @@ __device__ __forceinline__ void ref_contrib(double xp, double yp, double zp, dou
         unsigned low = 0;
         ref_pair_brackets<ROLE, true>(ref_powers<true>(ss.x, ss.y), ref_powers<true>(st.x, st.y),
                                       ref_powers<true>(sm.x, sm.y), nu, S, T, low);
-        done = !div_needs_ieee(low);
+        done = !div_is_hard(low);
     }
     if (!done) {
         unsigned low;

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(NSLOT) void k_update_fin(DeviceState d, double hdt,
         fz = d.fz[p];
     }
     const double m = d.m[p];
-    const double a0 = gx - fx / m, a1 = gy - fy / m, a2 = gz - fz / m;
+    const double a0 = gx - div_rn(fx, m), a1 = gy - div_rn(fy, m), a2 = gz - div_rn(fz, m);
     d.vx[p] = d.vx[p] + a0 * hdt;
     d.vy[p] = d.vy[p] + a1 * hdt;
     d.vz[p] = d.vz[p] + a2 * hdt;
@@ -902,7 +902,7 @@ __device__ __forceinline__ void update_bin_one(const DeviceState &d, double hdt,
         fz = d.fz[p];
     }
     const double m = d.m[p];
-    const double a0 = gx - fx / m, a1 = gy - fy / m, a2 = gz - fz / m;
+    const double a0 = gx - div_rn(fx, m), a1 = gy - div_rn(fy, m), a2 = gz - div_rn(fz, m);
     const double vx = d.vx[p] + a0 * hdt, vy = d.vy[p] + a1 * hdt, vz = d.vz[p] + a2 * hdt;
     d.vx[p] = vx;
     d.vy[p] = vy;
@@ -3107,12 +3107,13 @@ __global__ void k_selftest_fp64(long long n, const double *__restrict__ a, const
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     sq[i] = __builtin_sqrt(a[i]);
-    q[i] = a[i] / b[i];
+    q[i] = div_rn(a[i], b[i]);
     rs[i] = __builtin_amdgcn_rsq(a[i]);
 }
 
 // The in-range sequences of the bit-exact path, element-wise.  The division
-// starts from a reciprocal that is off by 2^-46 on purpose, either way.
+// starts from a reciprocal that is off by 2^-46 on purpose, either way, and is
+// left unguarded where the brackets leave it so: for the numerators 3 and 5.
 __global__ void k_selftest_fp64_inrange(long long n, const double *__restrict__ a, const double *__restrict__ b,
                                         double *__restrict__ sq, double *__restrict__ q)
 {
@@ -3124,7 +3125,8 @@ __global__ void k_selftest_fp64_inrange(long long n, const double *__restrict__ 
 #pragma unroll
     for (int k = 0; k < 2; ++k) r = __builtin_fma(r, __builtin_fma(-b[i], r, 1.0), r);
     r *= i & 1 ? 1.0 + 0x1p-46 : 1.0 - 0x1p-46;
-    q[i] = div_needs_ieee(low_word(b[i])) ? a[i] / b[i] : div_rn_from(a[i], b[i], r);
+    const double m = __builtin_fabs(a[i]);
+    q[i] = m != 3.0 && m != 5.0 && div_is_hard(low_word(b[i])) ? div_rn(a[i], b[i]) : div_rn_from(a[i], b[i], r);
 }
 
 GridDev grid_dev(const CellGrid &g)
