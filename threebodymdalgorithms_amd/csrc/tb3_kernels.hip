@@ -2959,23 +2959,25 @@ __global__ __launch_bounds__(WAVE, TILE_JB > 4 ? 3 : 4) void k_forces_tiles(Tile
     const int n = a.n;
     const int jbase = t1 * WAVE, kbase = t2 * WAVE;
     const int i = t0 * WAVE + lane, jl = jbase + lane, kl = kbase + lane;
-    // Padding slots get distinct far-away coordinates so the arithmetic on
-    // them stays finite.
-    const double far = 1.0e6 + 16.0 * lane;
-    const double xi = i < n ? a.x[i] : far, yi = i < n ? a.y[i] : far, zi = i < n ? a.z[i] : far;
-    kx[lane] = kl < n ? a.x[kl] : -far;
-    ky[lane] = kl < n ? a.y[kl] : -far;
-    kz[lane] = kl < n ? a.z[kl] : -far;
+    // Padding slots stand for the last particle.
+    const int ic = min(i, n - 1), kc = min(kl, n - 1);
+    const double xi = a.x[ic], yi = a.y[ic], zi = a.z[ic];
+    kx[lane] = a.x[kc];
+    ky[lane] = a.y[kc];
+    kz[lane] = a.z[kc];
     fkx[lane] = fky[lane] = fkz[lane] = 0.0;
 
     const T nu = (T)a.nu, K = (T)(0.375 * a.nu);
     double gix = 0.0, giy = 0.0, giz = 0.0;  // i's gradient
     double gjx = 0.0, gjy = 0.0, gjz = 0.0;  // that of j = jbase + lane
     double esum = 0.0;
-    // tiles in which some (i, k) is no pair (wrong order, itself or padding):
-    // such a pair's side is set to 1, so that only finite numbers meet the
-    // zeros of the triplet's other sides
-    const bool edge = t0 == t2 || kbase + WAVE > n;
+    // tiles in which some (i, k) is one particle.  A side of a particle to
+    // itself is set to 1, every other one is the true side, also of pairs in
+    // the wrong order: the zero powers then meet the numbers of a triplet that
+    // counts somewhere, or of a triangle with two equal sides and this one,
+    // which are finite where the sweep's own are (a made-up side among far
+    // apart particles is not: A B C of sides 1, r, r' goes with r^6)
+    const bool edge = t0 == t2;
 
     for (int j0 = jlo; j0 < jhi; j0 += TILE_JB) {
         if (jbase + j0 >= n) break;
@@ -2990,7 +2992,7 @@ __global__ __launch_bounds__(WAVE, TILE_JB > 4 ? 3 : 4) void k_forces_tiles(Tile
             const double dx = xj - xi, dy = yj - yi, dz = zj - zi;
             const double uu = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
             const bool ij = i < j && j < n;
-            u[q] = ij ? uu : 1.0;
+            u[q] = ic != jc ? uu : 1.0;
             if constexpr (FP64) su[q] = ij ? rsqrt_f64(uu) : 0.0;
             else su[q] = ij ? T(1) : T(0);
             cu_sum[q] = 0.0;
@@ -2998,7 +3000,7 @@ __global__ __launch_bounds__(WAVE, TILE_JB > 4 ? 3 : 4) void k_forces_tiles(Tile
             const double ex = kx[lane] - xj, ey = ky[lane] - yj, ez = kz[lane] - zj;
             const double ww = __builtin_fma(ex, ex, __builtin_fma(ey, ey, ez * ez));
             const bool jk = j < kl && kl < n;
-            pw[q][lane] = jk ? ww : 1.0;
+            pw[q][lane] = jc != kc ? ww : 1.0;
             if constexpr (FP64) ps[q][lane] = jk ? rsqrt_f64(ww) : 0.0;
             else ps[q][lane] = jk ? T(1) : T(0);
             if (GRAD) pc[q][lane] = 0.0;
@@ -3016,7 +3018,7 @@ __global__ __launch_bounds__(WAVE, TILE_JB > 4 ? 3 : 4) void k_forces_tiles(Tile
             const int kk = WAVE - m + ((lane + s) & (m - 1));
             const double dx = kx[kk] - xi, dy = ky[kk] - yi, dz = kz[kk] - zi;
             double v = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
-            if (edge && !(i < kbase + kk && kbase + kk < n)) v = 1.0;
+            if (edge && ic == min(kbase + kk, n - 1)) v = 1.0;
             T sv = T(1);
             if constexpr (FP64) sv = rsqrt_f64(v);
             double cv_sum = 0.0;
