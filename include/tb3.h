@@ -156,7 +156,8 @@ tb3_status tb3_energy_grad(tb3_ctx *ctx, double *E, double *dEdx, double *dEdnu,
  * row-major device array; results land in device memory; `stream` is a
  * hipStream_t (NULL: the context's stream).  They use the context's
  * algorithm, cutoff, domain and precision but not its particles, and leave
- * the context's particle state untouched.  The work is ordered on `stream`
+ * the context's particle state untouched; a call that fails leaves d_E and
+ * d_dEdx untouched too.  The work is ordered on `stream`
  * after what the caller queued there before, and is complete on return: the
  * context's status block and scratch memory, which its next call reuses, are
  * read by then.  n_triplets (host) may be NULL. */

@@ -536,7 +536,9 @@ __device__ void cuts_workgroup(int ncell, const int *__restrict__ cell_start, co
 // stores the energy (e, may be null) and publishes the status, the next
 // (with a cell list, ncell > 0) cuts the XCD runs of the next sweep, the
 // others take the particles' role sums (exact path; SumUpParticles,
-// Algorithm.cpp:245-249) and forces to rows (may be null).
+// Algorithm.cpp:245-249) and forces to rows (may be null).  A pass that is to
+// be repeated, or refused, leaves e and rows alone (flags[2]; the fold's clear
+// happens only when it is already zero, so every workgroup sees one value).
 __global__ __launch_bounds__(NSLOT) void k_finish(DeviceState d, Status *st, Status *host, double *e, int sum_roles,
                                                   double *rows, int ncell, const int *__restrict__ cell_start,
                                                   const unsigned *__restrict__ cell_work, int *__restrict__ order,
@@ -544,7 +546,7 @@ __global__ __launch_bounds__(NSLOT) void k_finish(DeviceState d, Status *st, Sta
 {
     if (blockIdx.x == 0) {
         fold_slots(st);
-        if (threadIdx.x == 0 && e) *e = st->energy;
+        if (threadIdx.x == 0 && e && !st->flags[2]) *e = st->energy;
         publish_status(st, host, threadIdx.x, NSLOT);
         return;
     }
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(NSLOT) void k_finish(DeviceState d, Status *st, Sta
         fy = d.fy[p];
         fz = d.fz[p];
     }
-    if (rows) {
+    if (rows && !st->flags[2]) {
         rows[3 * (long long)p + 0] = fx;
         rows[3 * (long long)p + 1] = fy;
         rows[3 * (long long)p + 2] = fz;
