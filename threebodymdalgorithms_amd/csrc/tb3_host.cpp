@@ -167,6 +167,7 @@ struct tb3_ctx {
     bool cells_ok = true;  // the cell-per-workgroup kernel staged every neighbourhood so far
     bool wide_need = false;  // some owner needed its wide shape (else: where the density makes that likely)
     bool dense_on = false;  // the dense-owner kernel follows the cell kernel (once some owner needed it)
+    bool dense_known = false;  // a sweep in the wide shape with it behind showed whether some owner does
     // the slotted cell layout of replayed steps (CellGrid::pad_cap): slots
     // per cell asked for (-1: three times the mean cell count, 0: off), and
     // whether a cell outgrew its slots in this particle system's grid (the
@@ -404,6 +405,7 @@ void configure_grid(tb3_ctx *c)
     c->cells_ok = true;  // a new grid gets a new chance at the cell kernel
     c->wide_need = false;
     c->dense_on = false;
+    c->dense_known = false;
     c->slots_failed = false;
     c->slots_clean = false;
     if (!same) ++c->epoch;
@@ -590,9 +592,11 @@ int next_pow2(int v)
 // 460 staged on average most cells would be handed on in either: 20000 at
 // cutoff 2.75 510 us in both.
 constexpr int WIDE_CELLS = 3000;
-bool wide_expected(const CellGrid &g, double cutoff, long long n)
+struct CellNeeds {
+    double staged, list;  // particles staged for a cell and entries of the longest list, on average
+};
+CellNeeds cell_needs(const CellGrid &g, double cutoff, long long n)
 {
-    if (g.nrep > 1 || n < 3) return false;
     double w[3], area = 1.0, box = 1.0, vol = 1.0;
     int ext = 0;
     bool three = false;
@@ -612,15 +616,64 @@ bool wide_expected(const CellGrid &g, double cutoff, long long n)
         reach = box + 2 * c * (w[0] * w[1] + w[1] * w[2] + w[0] * w[2]) + pi * c * c * (w[0] + w[1] + w[2]) +
                 4.0 / 3.0 * pi * c * c * c;
     const double density = (double)n / vol;
-    const double staged = density * (three ? reach : 0.5 * (box + reach));
-    const double list = 0.8 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n);
-    if (staged > 460.0) return false;
+    return {density * (three ? reach : 0.5 * (box + reach)),
+            0.8 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n)};
+}
+
+bool wide_expected(const CellGrid &g, double cutoff, long long n)
+{
+    if (g.nrep > 1 || n < 3) return false;
+    const CellNeeds e = cell_needs(g, cutoff, n);
+    if (e.staged > 460.0) return false;
     const bool few = g.ncell <= WIDE_CELLS;
     const double zs = few ? std::sqrt(2.0 * std::log(std::max(g.ncell, 2))) + 0.3 : 2.0, zl = few ? 4.0 : 2.5;
-    return staged + zs * std::sqrt(staged) > 256.0 || list + zl * std::sqrt(list) > 96.0;
+    return e.staged + zs * std::sqrt(e.staged) > 256.0 || e.list + zl * std::sqrt(e.list) > 96.0;
+}
+
+// Whether a first sweep in the wide shape should have the dense-owner kernel
+// behind it: a sweep that one owner outgrows is repeated whole, which costs far
+// more than the launch (N = 67500 at density 2, cutoff 2.6: 1519 us and 773
+// from then on; the launch, and the contiguous cell list that it needs, 20 to
+// 30).  So where a tenth of a neighbourhood past 512 or a list past 136 is to
+// be expected.  2.4% of the owners of a uniform system have a list as long as that
+// of the corner (counted at densities 1.5 to 2.2, cutoffs 2.5 to 2.7, N = 4000
+// to 67500: of the tail of a normal distribution about it 2.1 to 2.4%).  What
+// that sweep shows holds for the next ones (note_dense).  N = 67500 at cutoff
+// 2.6 773 us from the first sweep on; a liquid of as many, which never needs it,
+// 728 and then 706.
+bool dense_expected(const CellGrid &g, double cutoff, long long n)
+{
+    if (g.nrep > 1 || n < 3) return false;
+    const CellNeeds e = cell_needs(g, cutoff, n);
+    auto past = [](double mean, double most) { return 0.5 * std::erfc((most - mean) / std::sqrt(2.0 * mean)); };
+    return (double)g.ncell * past(e.staged, 512.0) + 0.024 * (double)n * past(e.list, 136.0) > 0.1;
 }
 
 bool cells_wide(const tb3_ctx *c, long long n) { return c->wide_need || wide_expected(c->grid, c->cutoff, n); }
+
+// Whether the dense-owner kernel follows the cell kernel: where some owner
+// needed it, and behind the first sweep in the wide shape where the density
+// makes that likely, or a sweep in the narrow one asked for the wide (it knows
+// the neighbourhoods, not the lists).
+bool cells_dense(const tb3_ctx *c, long long n)
+{
+    if (c->dense_on) return true;
+    return !c->dense_known && cells_wide(c, n) && (c->wide_need || dense_expected(c->grid, c->cutoff, n));
+}
+
+// Whether a fast sweep of n particles would find that out.
+bool dense_tried(const tb3_ctx *c, long long n)
+{
+    return uses_cutoff(c) && n >= 3 && c->cells_ok && !c->dense_on && cells_dense(c, n);
+}
+
+// After a completed pass that ran a fast sweep (the status is on the host).
+void note_dense(tb3_ctx *c, long long n)
+{
+    if (!dense_tried(c, n)) return;
+    c->dense_known = true;
+    c->dense_on = c->h_status->dense_n > 0;
+}
 
 // The n x n table of pair lengths that the bit-exact all-triplets sweep reads
 // (16 bytes a pair, 256 MiB at the most).  Without it (more particles, or no
@@ -663,11 +716,10 @@ void launch_sweep(tb3_ctx *c, hipStream_t s, DeviceState &d, bool grad, bool ene
         if (fast_grad || energy) {
             const int slot = (exact && grad) ? 1 : 0;  // the exact pass owns count[0]
             if (cut && c->cells_ok) {
-                const bool wide = cells_wide(c, d.n);
+                const bool wide = cells_wide(c, d.n), dense = cells_dense(c, d.n);
                 launch_p3bca_cells(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
-                                   energy ? 1 : 0, c->d_owners, c->dense_on ? 1 : 0, wide ? 1 : 0, slotted ? 1 : 0,
-                                   parity);
-                if (c->dense_on)
+                                   energy ? 1 : 0, c->d_owners, dense ? 1 : 0, wide ? 1 : 0, slotted ? 1 : 0, parity);
+                if (dense)
                     launch_p3bca_dense(s, d, c->grid, cs, c->nu, mixed, fast_grad ? 1 : 0, c->d_status, slot,
                                        energy ? 1 : 0, c->d_owners, c->dense_grid, c->dense_waves);
             }
@@ -809,6 +861,7 @@ void finish_overflowed(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate
         if (c->recording) HIPCHK(hipEventRecord(c->ev[4], s));
         HIPCHK(hipStreamSynchronize(s));
     }
+    if ((grad && !exact) || energy) note_dense(c, d.n);
 }
 
 // Whether a single pass over n particles runs on the slotted layout (then
@@ -816,7 +869,7 @@ void finish_overflowed(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate
 // slots itself and no scatter kernel runs.
 bool slotted_pass(tb3_ctx *c, int n)
 {
-    if (!uses_cutoff(c) || n < 3 || !c->cells_ok || c->dense_on || c->slots_distrust) return false;
+    if (!uses_cutoff(c) || n < 3 || !c->cells_ok || cells_dense(c, n) || c->slots_distrust) return false;
     if (cells_fused_scan(c->grid)) {
         ensure_slot_buffers(c, n);
     } else {
@@ -904,7 +957,8 @@ bool fused_steps(const tb3_ctx *c) { return uses_cutoff(c) && c->state.d.n >= 3 
 // grid.pad_cap first.
 bool slotted_steps(const tb3_ctx *c)
 {
-    return fused_steps(c) && c->precision != TB3_FP64_EXACT && c->cells_ok && !c->dense_on && c->grid.pad_cap > 0;
+    return fused_steps(c) && c->precision != TB3_FP64_EXACT && c->cells_ok && !cells_dense(c, c->state.d.n) &&
+           c->grid.pad_cap > 0;
 }
 
 template <class F>
@@ -933,7 +987,7 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
     const int slots = slotted_steps(c) ? c->grid.pad_cap : 0;
     if (c->step_exec && c->graph_epoch == c->epoch && c->graph_dt == dt && c->graph_g[0] == g[0] &&
         c->graph_g[1] == g[1] && c->graph_g[2] == g[2] && c->graph_cap == c->list_cap &&
-        c->graph_cells_ok == c->cells_ok && c->graph_dense_on == c->dense_on &&
+        c->graph_cells_ok == c->cells_ok && c->graph_dense_on == cells_dense(c, c->n) &&
         c->graph_wide == cells_wide(c, c->n) && c->graph_fused == fused &&
         c->graph_slots == slots)
         return;
@@ -987,7 +1041,7 @@ void capture_step_graph(tb3_ctx *c, double dt, const double *g)
     for (int k = 0; k < 3; ++k) c->graph_g[k] = g[k];
     c->graph_cap = c->list_cap;
     c->graph_cells_ok = c->cells_ok;
-    c->graph_dense_on = c->dense_on;
+    c->graph_dense_on = cells_dense(c, c->n);
     c->graph_wide = cells_wide(c, c->n);
 }
 
@@ -1028,6 +1082,14 @@ void run_steps_graph(tb3_ctx *c, int steps, double dt, const double *g, uint64_t
                 if (counts) step_counts(c, counts + (size_t)done * per);
             }
             return;
+        }
+        // whether the replays need the dense-owner kernel: a step by itself
+        // finds out (replays that turned out wrong would be captured again)
+        if (c->precision != TB3_FP64_EXACT && dense_tried(c, d.n)) {
+            run_pass(c, s, d, true, dt, g, true, false, false);
+            if (counts) step_counts(c, counts + (size_t)done * per);
+            ++done;
+            continue;
         }
         // what a step would allocate is allocated before the capture
         if (uses_cutoff(c) && d.n >= 3) {
@@ -1745,7 +1807,8 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
         // buffers replaced by the scratch array: the dense-owner kernel once
         // an owner needs it, the per-owner kernel with a growing list
         // capacity once a neighbourhood is too large for the cell kernel
-        bool cells = true, dense = false, wide = wide_expected(g, c->cutoff, n);
+        bool cells = true, wide = wide_expected(g, c->cutoff, n);
+        bool dense = wide && dense_expected(g, c->cutoff, n);
         int cap = c->list_cap;
         Status h;
         for (int attempt = 0;; ++attempt) {
@@ -1772,7 +1835,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             if (attempt >= 8) throw Fail(TB3_EHIP, "the cutoff sweep kept overflowing its LDS staging");
             if (h.flags[3]) cells = false;
             if (h.want_dense == 1 && ncell <= WIDE_CELLS && !wide) wide = true;
-            else if (h.want_dense) dense = true;
+            if (h.want_dense) dense = true;
             if (!cells && h.flags[1] > cap) {
                 if (h.flags[1] > MAX_LIST)
                     throw Fail(TB3_EUNSUPPORTED, "a particle has " + std::to_string(h.flags[1]) +

@@ -116,7 +116,7 @@ struct Status {
                                   // kernel skips itself), [3] the cell kernel could not stage a
                                   // neighbourhood (re-run with the per-owner kernel)
     int dqueue[2];                // owner queue of the dense-owner kernel; returns to zero after each launch
-    int dense_n;                  // owners the cell kernel handed to the dense-owner kernel
+    int dense_n;                  // owners the cell kernel handed to the dense-owner kernel (until the pass's clear)
     int want_dense;               // the cell kernel had owners for a dense-owner kernel that was not launched:
                                   // 1 if its wide shape would take them all, 2 or 3 otherwise
     Slots *slots;                 // partial sums of the sweep kernels

@@ -243,6 +243,7 @@ __device__ __forceinline__ void publish_status(Status *st, Status *host, int t, 
         for (int k = 0; k < 4; ++k) host->flags[k] = st->flags[k];
         host->want_dense = st->want_dense;
         host->pad_over = st->pad_over;
+        host->dense_n = st->dense_n;
     }
     __syncthreads();
     if (!over && st->nrep <= 1) {
@@ -2331,7 +2332,6 @@ __global__ __launch_bounds__(DW *WAVE, 4) void k_p3bca_dense(DenseDev a)
         if (done == (int)gridDim.x - 1) {
             atomicExch(&a.queue[0], 0);
             atomicExch(&a.queue[1], 0);
-            atomicExch(&A.st->dense_n, 0);
         }
     }
 }
