@@ -229,7 +229,8 @@ tb3_status tb3_set_tuning(tb3_ctx *ctx, double cell_ratio, int dense_waves);
  * three times the mean cell count (at least 32), 0 turns the layout off,
  * 1 .. 256 sets it; TB3_EINVAL otherwise.  A step in which some cell gets
  * more particles than slots is finished on the contiguous layout, which the
- * rest of the run (and later runs on the same grid) then keeps.
+ * rest of the run (and later runs on the same grid) then keeps; single passes
+ * keep it until tb3_configure or tb3_set_cell_slots.
  * tb3_get_cell_slots reports the setting and the slots per cell that the
  * last captured step graph used (0: contiguous, or a cell has outgrown its
  * slots since).  No counterpart in the reference, whose cell lists are host

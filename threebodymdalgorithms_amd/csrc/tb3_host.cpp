@@ -180,9 +180,9 @@ struct tb3_ctx {
     // pass's parity are zero (its predecessor's sweep cleared them)
     bool slots_clean = false;
     int slots_parity = 0;
-    // a single pass failed on a full slot since tb3_configure: single passes
-    // stay off the layout, also with other particles (a clustered system fails
-    // every time)
+    // a single pass failed on a full slot since tb3_configure or
+    // tb3_set_cell_slots: single passes stay off the layout, also with other
+    // particles (a clustered system fails every time)
     bool slots_distrust = false;
     int dense_grid = 1;    // persistent grid of the dense-owner kernel (workgroups that fit the GPU)
     int dense_waves = 8;   // waves per owner in the dense-owner kernel (tuned: 4, 8 or 16)
@@ -1994,7 +1994,7 @@ tb3_status tb3_set_cell_slots(tb3_ctx *c, int slots)
     if (!(slots == -1 || slots == 0 || (slots >= 1 && slots <= 256)))
         return fail(c, TB3_EINVAL, "slots must be -1 (automatic), 0 (off) or 1 .. 256");
     c->slots_req = slots;
-    c->slots_failed = false;
+    c->slots_failed = c->slots_distrust = false;
     ++c->epoch;
     return TB3_OK;
 }
