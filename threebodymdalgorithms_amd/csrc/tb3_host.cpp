@@ -187,6 +187,7 @@ struct tb3_ctx {
     int dense_grid = 1;    // persistent grid of the dense-owner kernel (workgroups that fit the GPU)
     int dense_waves = 8;   // waves per owner in the dense-owner kernel (tuned: 4, 8 or 16)
     int ncu = 1;           // compute units of the device
+    int cells_blocks[2] = {1, 1};  // workgroups of the cell kernel that a CU holds: narrow shape (5), wide (2)
     // tuned by tb3_autotune: cell width / cutoff, resident cell-kernel workgroups per CU
     double cell_ratio = 1.0;
     int cells_per_cu = 0;  // resident cell-kernel workgroups per CU at the tuned width
@@ -442,8 +443,8 @@ struct Carver {
 
 bool cells_wide(const tb3_ctx *c, long long n);
 
-// Workgroups of the cell kernel that an XCD holds at once (5 or, wide, 2 per CU).
-int xcd_slots(const tb3_ctx *c, bool wide) { return std::max(1, c->ncu / 8 * (wide ? 2 : 5)); }
+// Workgroups of the cell kernel that an XCD holds at once.
+int xcd_slots(const tb3_ctx *c, bool wide) { return std::max(1, c->ncu / 8 * c->cells_blocks[wide ? 1 : 0]); }
 
 // The per-cell arrays of the current grid, zeroed when allocated, and the
 // workgroup slots that its cells fill.
@@ -1228,6 +1229,7 @@ tb3_status tb3_create(int device, tb3_ctx **out)
         int ncu = 0;
         HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
         c->ncu = std::max(1, ncu);
+        for (int wide = 0; wide < 2; ++wide) c->cells_blocks[wide] = p3bca_cells_blocks_per_cu(wide != 0);
         p3bca_dense_setup();
         init_scratch_address(device);
         c->dense_grid = std::max(1, ncu) * p3bca_dense_blocks_per_cu(c->dense_waves);
@@ -1922,8 +1924,8 @@ tb3_status tb3_autotune(tb3_ctx *c, int reps, double *best_ms, double *cell_rati
         };
         // 1. the cell width: the cell kernel runs one workgroup per cell, so
         // the width is its one free parameter (the hardware keeps
-        // p3bca_cells_blocks_per_cu of them resident on each CU)
-        const int max_per_cu = p3bca_cells_blocks_per_cu();
+        // cells_blocks of them resident on each CU)
+        const int max_per_cu = c->cells_blocks[0];
         const double ratios[] = {1.0, 1.15, 1.3, 1.5, 1.75, 2.0};
         double best = 1e300, best_ratio = c->cell_ratio;
         int best_blocks = c->cells_per_cu;

@@ -238,7 +238,7 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
                         int mixed, int grad, Status *st, int count_slot, int want_energy, int *owners, int dense_on,
                         int wide, int slotted = 0, int parity = -1);
 // Workgroups of launch_p3bca_cells that fit on one CU at once.
-int p3bca_cells_blocks_per_cu();
+int p3bca_cells_blocks_per_cu(bool wide);
 // The cell kernel hands owners whose neighbourhood does not fit its LDS
 // staging to this kernel (one owner per workgroup, lists of up to 1440
 // particles); owners beyond that set st->flags[2] and [3]

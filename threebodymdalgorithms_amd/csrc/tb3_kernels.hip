@@ -3465,13 +3465,13 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
 #undef TB3_CELLS
 }
 
-int p3bca_cells_blocks_per_cu()
+int p3bca_cells_blocks_per_cu(bool wide)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb,
-                                                     reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, false>),
-                                                     CellShape<false>::W * WAVE, 0) != hipSuccess || nb < 1)
-        nb = 1;
+    const void *kernel = wide ? reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, true>)
+                              : reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, false>);
+    const int threads = (wide ? CellShape<true>::W : CellShape<false>::W) * WAVE;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0) != hipSuccess || nb < 1) nb = 1;
     return nb;
 }
 
