@@ -871,20 +871,19 @@ void finish_overflowed(tb3_ctx *c, hipStream_t s, DeviceState &d, bool integrate
 bool slotted_pass(tb3_ctx *c, int n)
 {
     if (!uses_cutoff(c) || n < 3 || !c->cells_ok || cells_dense(c, n) || c->slots_distrust) return false;
-    if (cells_fused_scan(c->grid)) {
+    // larger grids than the fused scan's too, unless they are nearly empty:
+    // 64000 cells of 16 particles are binned in 70 us instead of 137 for the
+    // counts, their scan and the scatter
+    if (!cells_fused_scan(c->grid) &&
+        ((long long)c->grid.ncell * 4 > n || (long long)c->grid.ncell * slots_for(c, n) > SLOTS_MAX))
+        return false;
+    // a pass can do without the layout where memory is short
+    try {
         ensure_slot_buffers(c, n);
-    } else {
-        // larger grids too, unless they are nearly empty or memory is short:
-        // 64000 cells of 16 particles are binned in 70 us instead of 137 for the
-        // counts, their scan and the scatter
-        if ((long long)c->grid.ncell * 4 > n || (long long)c->grid.ncell * slots_for(c, n) > SLOTS_MAX) return false;
-        try {
-            ensure_slot_buffers(c, n);
-        } catch (const Fail &) {
-            (void)hipGetLastError();
-            c->slots_failed = true;
-            c->grid.pad_cap = 0;
-        }
+    } catch (const Fail &) {
+        (void)hipGetLastError();
+        c->slots_failed = true;
+        c->grid.pad_cap = 0;
     }
     if (c->grid.pad_cap == 0) return false;
     ensure_cell_buffers(c, n);
