@@ -3,6 +3,7 @@
 // Compiled with -ffp-contract=off: the bit-exact path depends on every FP64
 // expression rounding as written; the fast paths spell their fused
 // multiply-adds out with fma().
+#include <atomic>
 #include <climits>
 #include <type_traits>
 
@@ -3467,11 +3468,15 @@ void launch_p3bca_cells(hipStream_t s, const DeviceState &d, const CellGrid &g, 
 
 int p3bca_cells_blocks_per_cu(bool wide)
 {
-    int nb = 0;
+    // asked once (25 us); every gfx950 gives the same answer
+    static std::atomic<int> known[2];
+    int nb = known[wide ? 1 : 0].load();
+    if (nb > 0) return nb;
     const void *kernel = wide ? reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, true>)
                               : reinterpret_cast<const void *>(k_p3bca_cells<double, true, false, false>);
     const int threads = (wide ? CellShape<true>::W : CellShape<false>::W) * WAVE;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0) != hipSuccess || nb < 1) nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0) != hipSuccess || nb < 1) return 1;
+    known[wide ? 1 : 0].store(nb);
     return nb;
 }
 
