@@ -358,7 +358,7 @@ def main():
                    "integrate_ms": fp64["integrate_ms"], "tuned": fp64["tuned"]},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": FP64_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_VECTOR_PEAK_TFLOPS, "traffic": profiled_traffic(),
-                     "kernel": "tb3::k_p3bca_cells<double, true, false>", "flop_per_triplet": FLOP_PER_TRIPLET},
+                     "kernel": "tb3::k_p3bca_cells<double, true, false, false>", "flop_per_triplet": FLOP_PER_TRIPLET},
         "step_frac": step_frac(fp64),
         "fp64_vs_exact": fp64_vs_exact,
         "cpu_baseline": cpu,

@@ -56,7 +56,13 @@ tb3_status tb3_device_count(int *count);
 
 /* Replaces the construction of Simulation + topology + decomposition
  * (main.cpp:32-105, Simulation.hpp:28-31) for one GPU.  Creates a context on
- * `device` with its own stream. */
+ * `device` with its own stream.  What it allocates on the way it keeps until
+ * tb3_destroy: beside the particles (about 180 bytes each, twice with device
+ * calls) and the cell lists, the slots of the slotted cell layout (32 bytes
+ * each, up to 2 GiB; tb3_set_cell_slots) and, in the bit-exact all-triplets
+ * sweep of up to 4096 particles, their pair lengths (16 n^2 bytes, up to 256
+ * MiB).  Where memory is short, that sweep does without its table and single
+ * passes without the slots. */
 tb3_status tb3_create(int device, tb3_ctx **out);
 tb3_status tb3_destroy(tb3_ctx *ctx);
 
@@ -260,9 +266,10 @@ tb3_status tb3_selftest_fp64(tb3_ctx *ctx, int64_t n, const double *a, const dou
                              double *a_div_b, double *rsq_a);
 
 /* Diagnostic: the bit-exact path's in-range sequences for sqrt(a) and a / b
- * (the compiler's IEEE expansions without their range-scaling steps, used on
- * operands within 2^-500 .. 2^500), element-wise, for checking that they give
- * the IEEE results' bits on such operands.  No counterpart in the reference. */
+ * (the compiler's expansions without their range-scaling steps, the division
+ * from an approximate reciprocal; used on operands within 2^-500 .. 2^500),
+ * element-wise, for checking that they give the IEEE results' bits on such
+ * operands.  No counterpart in the reference. */
 tb3_status tb3_selftest_fp64_inrange(tb3_ctx *ctx, int64_t n, const double *a, const double *b, double *sqrt_a,
                                      double *a_div_b);
 

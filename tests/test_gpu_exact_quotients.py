@@ -55,6 +55,34 @@ def test_quotients_next_to_midpoints(eng):
     assert np.array_equal(q, a / b), int(np.sum(q != a / b))
 
 
+def roots_mod(rho, bits):
+    """All m with m^2 = rho mod 2^bits (rho = 1 mod 8)."""
+    found = {m for m in range(8) if (m * m - rho) % 8 == 0}
+    for b in range(4, bits + 1):
+        found = {v for m in found for v in (m, m + 2 ** (b - 1)) if (v * v - rho) % 2 ** b == 0}
+    return found
+
+
+def test_roots_next_to_midpoints(eng):
+    """Square roots next to a midpoint m (54 bits, odd) of two doubles: the
+    arguments X 2^k = m^2 - rho for small rho."""
+    x = []
+    for rho in range(-4095, 4096, 8):  # 1 mod 8
+        for k in (54, 55):
+            for m in roots_mod(rho, k):
+                m += 2 ** 53 if m < 2 ** 53 else 0
+                while m < 2 ** 54:
+                    X = (m * m - rho) >> k
+                    if 2 ** 52 <= X < 2 ** 53 and (X << k) + rho == m * m:
+                        x += [math.ldexp(X, k % 2 + e) for e in (-52, -60, -20)]
+                    m += 2 ** k
+    x = np.array(x)
+    assert len(x) > 1000
+    one = np.ones_like(x)
+    assert np.array_equal(eng.selftest_fp64(x, one)[0], np.sqrt(x))
+    assert np.array_equal(eng.selftest_fp64_inrange(x, one)[0], np.sqrt(x))
+
+
 def powers_product(x, z):
     """x^6 z^5 as the brackets form it."""
     px = pz = 1.0

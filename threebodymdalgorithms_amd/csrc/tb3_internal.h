@@ -25,9 +25,11 @@ struct DeviceState {
 // runs cut to about equal work (so their lengths vary around ncell / 8),
 // each sorted heaviest first, a heavy cell in several parts (order_runs).
 // `order` holds 8 runs of cell_run_cap(ncell) entries (the cell, in grids of
-// up to CELL_SPLIT_CELLS with its part in bits 16-23 and parts - 1 above), then the 8 run lengths, then the 9 cuts (run r is cells
-// [cut r, cut r+1)) that the last integrating pass's update computed, then
-// two more sets of 9 that replays on the slotted layout alternate between.
+// up to CELL_SPLIT_CELLS with its part in bits 16-23 and parts - 1 above),
+// then the 8 run lengths, then the 9 cuts (run r is cells [cut r, cut r+1))
+// that the last kernel of the last pass computed (single passes past 8192
+// cells leave them), then two more sets of 9 that replays on the slotted
+// layout alternate between.
 constexpr int CELL_SPLIT_CELLS = 8192;  // the largest grids that split cells
 constexpr int CELL_SLOTS_MAX = 160;     // workgroup slots of an XCD that the parts are counted for
 // Entries a run may have beyond one per cell: a part of every cell per slot and
@@ -77,8 +79,8 @@ struct CellGrid {
     unsigned long long *rep_count = nullptr;   // device, nrep: accepted triplets per replica
     double *rep_energy = nullptr;              // device, nrep: energy per replica
 
-    // Slotted cell layout of replayed steps (one system, fast sweep, no
-    // dense-owner kernel): cell c's particles sit at slots [c pad_cap,
+    // Slotted cell layout of replayed steps and single passes (one system, fast
+    // sweep, no dense-owner kernel): cell c's particles sit at slots [c pad_cap,
     // c pad_cap + count), written by the binning pass itself, so that no
     // scatter pass runs between the binning and the sweep.  The counts
     // alternate between two arrays by the parity of an epoch that each
@@ -107,7 +109,8 @@ struct Slots {
     double energy[NSLOT * SLOT_STRIDE];
 };
 
-// Small device status block, read back with one copy per step.
+// Small device status block: published to pinned memory by a single pass's last
+// kernel, read back with one copy per run of replays.
 struct Status {
     unsigned long long count[2];  // [0] accepted triplets, [1] discarded count of an auxiliary pass
     double energy;
@@ -135,8 +138,8 @@ struct Status {
     double *rep_energy;
     // a cell of the slotted layout received more particles than it has
     // slots (the sweep then fails the pass); cleared only by
-    // launch_begin_steps for a slotted run, never by a status clear, since the binning that
-    // sets it runs beside the clear of the replayed step's last kernel
+    // launch_begin_steps with the grid, never by a status clear, since the
+    // binning that sets it runs beside the clear of the replayed step's last kernel
     int pad_over;
 };
 

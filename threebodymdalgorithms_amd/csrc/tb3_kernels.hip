@@ -577,11 +577,12 @@ __global__ __launch_bounds__(NSLOT) void k_finish(DeviceState d, Status *st, Sta
     }
 }
 
-// The last kernel of an integrating pass.  Workgroup 0 first folds the
+// The last kernel of an integrating pass.  Its last workgroup folds the
 // sweep's slot sums into the status block (k_finalize); with `record` (a
 // replayed step graph) it then appends the step's count and, unless the
-// step halted, clears the status block for the next replay.  Every thread
-// then applies Particle::Update (structs.hpp:57-99) to its particle:
+// step halted, clears the status block for the next replay; with `host` (a
+// single pass) it publishes the status.  The particles' workgroups apply
+// Particle::Update (structs.hpp:57-99), a thread each:
 // a = g - f/m, v = v + a*(dt*0.5), with f = b0 + (b1 + b2) first when
 // `sum_roles` (Algorithm::SumUpParticles, Algorithm.cpp:245-249).  Nothing
 // is updated when the sweep overflowed (the host re-runs it first); the
@@ -1608,8 +1609,14 @@ __device__ __forceinline__ void cell_geometry(int coord, int n, double L, double
 // lists out (at density 2 and cutoff 2 33 +- 10.6 entries, in the order of the
 // slots 33 +- 14.8; the longest of 8000 particles at cutoff 2.5 105 instead of
 // 129), which saves pairs to test and owners for the dense-owner kernel: N =
-// 32768 116 -> 112 us, 8000 at cutoff 2.5 126 -> 109.  (y by 0.3 to 0.5 and x
-// by 0.1 to 0.25 sweep alike.)
+// 32768 116 -> 112 us, 8000 at cutoff 2.5 126 -> 109.  y by 0.3 to 0.5 and x
+// by 0.1 to 0.25 sweep alike, so speed does not fix the weights.  These two were
+// taken over 0.3 and 0.1 for a chaotic run that is compared with single steps
+// to 1e-12: which triplets share an owner decides the rounding of a sum, and
+// under 0.3 and 0.1 one particle's position lay on a rounding tie there, either
+// side of which the atomics' order takes (252 of 576 pairs of runs differed by
+// more; 0 under these, 112 under 0.5 and 0.2).  Nothing makes that hold for
+// another system or another kernel.
 __device__ __forceinline__ double owner_key(double x, double y, double z)
 {
     return __builtin_fma(0.4, y, __builtin_fma(0.15, x, z));
@@ -1687,9 +1694,10 @@ __global__ __launch_bounds__(CellShape<WIDE>::W *WAVE, WIDE ? 4 : 5) void k_p3bc
     // values.)
     if (A.st->halt) return;
     // The slotted layout: this sweep's counts, and cell c's counter of the
-    // next binning cleared (every cell has one workgroup).  A cell that had
-    // more particles than slots fails the pass; the host re-runs the step
-    // on the contiguous layout.
+    // next binning cleared (every cell has one entry with part 0, and no
+    // workgroup of this sweep reads the counts of that parity).  A cell that
+    // had more particles than slots fails the pass; the host re-runs the
+    // step on the contiguous layout.
     const int *scnt = nullptr;
     if (a.sl.cap > 0) {
         const unsigned e = a.sl.epoch();
