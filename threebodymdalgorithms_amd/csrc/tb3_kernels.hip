@@ -2702,8 +2702,8 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
 // Bound by VALU issue (88% busy): of an owner's ~9200 instructions at N =
 // 32768 and cutoff 2 (67 neighbours, 1044 triplets in 3 x 6 batches of 64)
 // two thirds are the batches' ~270 each, then the 35 rounds of pair tests and
-// the fold (one subtraction per triplet and component).  The lists hold each
-// entry's side to the owner, items are decoded without 32-bit products (a
+// the fold (one subtraction per triplet and component).  Lists of up to 128 hold
+// each entry's side to the owner (exact_roots), items are decoded without 32-bit products (a
 // quarter of the rate), and the sort ranks as many entries per lane as the
 // list needs: 10 steps 7.5 -> 6.4 ms with the quotients of at_math.h.
 constexpr int EXACT_GATHER = 4;  // candidates per lane and round
@@ -3214,8 +3214,13 @@ size_t p3bca_fast_lds(int cap)
     return (size_t)cap * (6 * sizeof(double) + sizeof(int)) + RING * sizeof(unsigned) + 64 * sizeof(int);
 }
 
-// The exact sweep's lists hold roots where that leaves them under 64 KB.
-static bool exact_roots(int cap) { return cap <= 1024; }
+// The exact sweep's lists hold roots where their 16 bytes an entry leave room
+// for the 16 waves per CU that the registers allow (10 KB a wave): up to 128
+// entries, 8 KB with roots.  There they gain 4-8% (N = 32768 at cutoff 2 680
+// against 730 us, 20000 at 2.2 674 against 723).  Past it they cost waves and
+// lose: 256 entries (11 waves) N = 20000 at cutoff 2.5 1535 against 1410, 512 (6)
+// N = 8000 at 3 2609 against 2283, 1024 (3) N = 8000 at 3.8 18.0 against 12.8 ms.
+static bool exact_roots(int cap) { return cap <= 128; }
 
 // sorted ids, then (16-byte aligned, cap is a multiple of 64) the positions
 // and the roots
