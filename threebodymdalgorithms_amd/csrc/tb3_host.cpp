@@ -681,7 +681,7 @@ void note_dense(tb3_ctx *c, long long n)
 // memory) the sweep computes every length where it needs it.
 void ensure_pair_roots(tb3_ctx *c, int n)
 {
-    if (n > PAIR_ROOTS_MAX || n <= c->pair_roots_cap) return;
+    if (n <= AUTA_SMALL || n > PAIR_ROOTS_MAX || n <= c->pair_roots_cap) return;
     dev_free(c->pair_roots);
     c->pair_roots_cap = 0;
     ++c->epoch;

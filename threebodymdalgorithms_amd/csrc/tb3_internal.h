@@ -257,8 +257,10 @@ void launch_p3bca_dense(hipStream_t s, const DeviceState &d, const CellGrid &g, 
                         int waves);
 
 // All-triplet sweeps (NATA / AUTA, or P3BCA without a cutoff).
+// (roots: an n x n table the launch fills, or null; up to AUTA_SMALL particles
+// it uses none.)
+constexpr int AUTA_SMALL = 128;
 void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *st, double2 *roots);
-// (roots: an n x n table the launch fills, or null.)
 // Tile triples t0 <= t1 <= t2 of 64 particles; accumulates into fx/fy/fz (zero first).
 void launch_forces_tiles(hipStream_t s, const DeviceState &d, const unsigned long long *triples,
                          long long ntriples, double nu, int mixed, int grad, Status *st, int count_slot,

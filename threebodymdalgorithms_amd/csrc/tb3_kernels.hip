@@ -2387,7 +2387,11 @@ struct ExactShared {
 //    with the longest stream, 3 times the mean: N = 1000 14.6 -> 5.9 ms, N =
 //    2048 90 -> 46.7, N = 3000 233 -> 145 ms.
 // S = 2 below 700 particles, where S = 4 leaves CUs without a workgroup (N =
-// 400 0.81 against 1.17 ms, N = 1000 6.6 against 6.0).
+// 400 0.81 against 1.17 ms, N = 1000 6.6 against 6.0).  Up to AUTA_SMALL the
+// sweep is a chain of launches and round trips: a workgroup of 4 waves takes one
+// role of one particle, and there is no table to fill first (a call of 8 21.5 us
+// against 33 as below, 60 33 against 50, 129 75 against 97, 150 104 against 117,
+// but 175 172 against 147).
 struct AutaExactDev {
     int n;
     const double *x, *y, *z;
@@ -2405,7 +2409,7 @@ __global__ __launch_bounds__(256) void k_pair_roots(int n, const double *__restr
     if (j < n) roots[(long long)i * n + j] = ref_root(ref_sqr(x[j] - x[i], y[j] - y[i], z[j] - z[i]));
 }
 
-constexpr int AUTA_WAVES = 8;
+constexpr int AUTA_WAVES = 8, AUTA_SMALL_WAVES = 4;
 constexpr int AUTA_ROUNDS = 4;  // rounds a wave may run ahead of the fold
 
 template <int W, int S>
@@ -2520,10 +2524,12 @@ __global__ __launch_bounds__(WAVE * W, 4) void k_auta_exact(AutaExactDev a)
 {
     __shared__ __attribute__((aligned(16))) AutaExactShared<W, S> sh;
     const int p0 = (int)blockIdx.x * S;
-    auta_exact_role<0, W, S, ROOTS>(a, p0, sh);
-    auta_exact_role<1, W, S, ROOTS>(a, p0, sh);
-    auta_exact_role<2, W, S, ROOTS>(a, p0, sh);
-    if ((int)threadIdx.x < S && p0 + (int)threadIdx.x < a.n) {
+    // with gridDim.y == 3 one of the roles each
+    const bool all = gridDim.y == 1;
+    if (all || blockIdx.y == 0) auta_exact_role<0, W, S, ROOTS>(a, p0, sh);
+    if (all || blockIdx.y == 1) auta_exact_role<1, W, S, ROOTS>(a, p0, sh);
+    if (all || blockIdx.y == 2) auta_exact_role<2, W, S, ROOTS>(a, p0, sh);
+    if (blockIdx.y == 0 && (int)threadIdx.x < S && p0 + (int)threadIdx.x < a.n) {
         const unsigned long long above = (unsigned long long)(a.n - 1 - (p0 + (int)threadIdx.x));
         add_count(a.st, 0, above ? above * (above - 1) / 2 : 0ull);
     }
@@ -2703,9 +2709,10 @@ __device__ void exact_role_staged(const StagedList &L, double xp, double yp, dou
 // 32768 and cutoff 2 (67 neighbours, 1044 triplets in 3 x 6 batches of 64)
 // two thirds are the batches' ~270 each, then the 35 rounds of pair tests and
 // the fold (one subtraction per triplet and component).  Lists of up to 128 hold
-// each entry's side to the owner (exact_roots), items are decoded without 32-bit products (a
-// quarter of the rate), and the sort ranks as many entries per lane as the
-// list needs: 10 steps 7.5 -> 6.4 ms with the quotients of at_math.h.
+// each entry's side to the owner (exact_roots), items are decoded without
+// 32-bit products (a quarter of the rate), and the sort ranks as many entries
+// per lane as the list needs: 10 steps 7.5 -> 6.4 ms with the quotients of
+// at_math.h.
 constexpr int EXACT_GATHER = 4;  // candidates per lane and round
 
 // 4 waves per SIMD: within 96 VGPRs, for a fifth, the brackets' reciprocals
@@ -3585,7 +3592,10 @@ void launch_auta_exact(hipStream_t s, const DeviceState &d, double nu, Status *s
     a.st = st;
     a.roots = roots;
     const dim3 blk(AUTA_WAVES * WAVE), grid2(blocks_for(d.n, 2)), grid4(blocks_for(d.n, 4));
-    if (roots) {
+    if (d.n <= AUTA_SMALL) {
+        hipLaunchKernelGGL((k_auta_exact<AUTA_SMALL_WAVES, 1, false>), dim3((unsigned)d.n, 3), dim3(AUTA_SMALL_WAVES * WAVE),
+                           0, s, a);
+    } else if (roots) {
         hipLaunchKernelGGL(k_pair_roots, dim3(blocks_for(d.n, 256), (unsigned)d.n), dim3(256), 0, s, d.n, d.x, d.y, d.z,
                            roots);
         if (d.n < 700) hipLaunchKernelGGL((k_auta_exact<AUTA_WAVES, 2, true>), grid2, blk, 0, s, a);
