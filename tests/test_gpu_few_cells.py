@@ -1,0 +1,86 @@
+"""Grids of a few cells with long neighbour lists, whose owners go to the
+dense-owner kernel, in the order of their key where a whole cell goes.  Counts
+bit for bit against the CPU oracle, forces within 1e-12 of the summed
+contribution lengths (against its squared-distance form)."""
+import time
+
+import numpy as np
+import pytest
+
+import threebodymdalgorithms_amd as tb3
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    with tb3.Engine(0) as e:
+        yield e
+
+
+def line(n, cells, cutoff, seed):
+    """n particles at density 2 in a box of so many cells in x, one in y and z."""
+    long = cells * cutoff * 1.01
+    side = (n / 2.0 / long) ** 0.5
+    L = np.array([long, side, side])
+    assert side < 3 * cutoff
+    return np.random.default_rng(seed).uniform(0.0, 1.0, (n, 3)) * L, L
+
+
+def box(n, ratio, seed):
+    """n particles at density 2 in one cell, the box `ratio` cutoffs wide."""
+    side = (n / 2.0) ** (1.0 / 3.0)
+    return np.random.default_rng(seed).uniform(0.0, side, (n, 3)), np.full(3, side), side / ratio
+
+
+def check(eng, oracle, P, L, cutoff, precision="fp64"):
+    fo, _, co = oracle.forces_fast(P, cutoff=cutoff, L=L)
+    S = oracle.force_scale(P, cutoff=cutoff, L=L)
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=cutoff, domain_L=L, precision=precision)
+    bar = {"fp64": 1e-12, "fp32": 2e-6}[precision]
+    for _ in range(3):
+        _, f, _, cnt = eng.energy_grad()
+        assert cnt == co and np.all(np.linalg.norm(f - fo, axis=1) <= bar * S)
+    assert eng.energy()[1] == co
+    assert list(eng.run(3, 0.0)) == [co] * 3
+
+
+@pytest.mark.parametrize("n,ratio", [(110, 2.0), (150, 1.3), (255, 2.4), (257, 1.8), (257, 2.9), (300, 2.2), (500, 2.0),
+                                     (520, 2.5), (900, 0.9)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_one_cell(eng, oracle, n, ratio, precision):
+    check(eng, oracle, *box(n, ratio, n), precision)
+
+
+@pytest.mark.parametrize("n,cells,cutoff", [(400, 3, 2.0), (400, 3, 3.0), (600, 4, 2.6), (600, 5, 2.6), (1000, 6, 3.0)])
+def test_lines_of_cells(eng, oracle, n, cells, cutoff):
+    check(eng, oracle, *line(n, cells, cutoff, n + cells), cutoff)
+
+
+def test_cells_handed_on_from_outside_the_box(eng, oracle):
+    """Owners past both ends of the key's steps: particles left and right of the
+    box, in cells that go on whole."""
+    P, L, cutoff = box(700, 2.0, 7)
+    P[:60] -= 0.4 * L
+    P[60:120] += 0.4 * L
+    check(eng, oracle, P, L, cutoff)
+
+
+def median_time(eng, P, L, cutoff):
+    eng.set_particles(P)
+    eng.configure("p3bca", cutoff=cutoff, domain_L=L, precision="fp64")
+    times = []
+    for k in range(30):
+        start = time.perf_counter()
+        eng.compute_forces()
+        if k >= 5:
+            times.append(time.perf_counter() - start)
+    return np.median(times)
+
+
+def test_longest_lists_first(eng):
+    """Complete lists: 900 particles (5.2 times the triplets of 520) take 3.1
+    times as long, 4 times with the longest lists anywhere in the queue."""
+    times = median_time(eng, *box(520, 1.2, 2)), median_time(eng, *box(900, 1.2, 2))
+    assert times[1] < 3.55 * times[0], times
