@@ -79,6 +79,12 @@ def median_time(eng, P, L, cutoff):
     return np.median(times)
 
 
+def test_long_lists_in_one_cell(eng):
+    """450 particles in one cell: lists three times as long cost 1.2 times the
+    call (2.3 times when 16 wide workgroups sweep them first)."""
+    assert median_time(eng, *box(450, 2.0, 1)) < 1.75 * median_time(eng, *box(450, 2.9, 1))
+
+
 def test_longest_lists_first(eng):
     """Complete lists: 900 particles (5.2 times the triplets of 520) take 3.1
     times as long, 4 times with the longest lists anywhere in the queue."""

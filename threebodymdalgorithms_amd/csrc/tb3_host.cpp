@@ -621,31 +621,47 @@ CellNeeds cell_needs(const CellGrid &g, double cutoff, long long n)
             0.8 * std::min(density * 4.0 / 3.0 * pi * c * c * c, (double)n)};
 }
 
+// Whether the owners that outgrow the narrow shape should go to the dense-owner
+// kernel all the same: on a few cells, whose 16 workgroups each do not fill the
+// chip, while that kernel takes a workgroup per owner.  Below 9 cells where the
+// longest lists pass 105 on average (4 cells of 150, lists of 118: 79 us against
+// 118; one cell of 256, 107: 121 against 146; but of 130, 104: 95 in both, and 9
+// cells of 67, 118: 89 against 84), and in one cell too large for the narrow
+// shape, all of which goes on at once, where they pass 42 (300 particles, 73: 62
+// us against 78; 41: 62 against 59; 500, 209: 98 against 204).
+bool dense_alone(const CellGrid &g, const CellNeeds &e)
+{
+    if (g.nrep > 1 || g.ncell >= 9) return false;
+    return e.list > 105.0 || (g.ncell == 1 && e.staged > 256.0 && e.list > 42.0);
+}
+
 bool wide_expected(const CellGrid &g, double cutoff, long long n)
 {
     if (g.nrep > 1 || n < 3) return false;
     const CellNeeds e = cell_needs(g, cutoff, n);
-    if (e.staged > 460.0) return false;
+    if (e.staged > 460.0 || dense_alone(g, e)) return false;
     const bool few = g.ncell <= WIDE_CELLS;
     const double zs = few ? std::sqrt(2.0 * std::log(std::max(g.ncell, 2))) + 0.3 : 2.0, zl = few ? 4.0 : 2.5;
     return e.staged + zs * std::sqrt(e.staged) > 256.0 || e.list + zl * std::sqrt(e.list) > 96.0;
 }
 
-// Whether a first sweep in the wide shape should have the dense-owner kernel
-// behind it: a sweep that one owner outgrows is repeated whole, which costs far
-// more than the launch (N = 67500 at density 2, cutoff 2.6: 1519 us and 773
-// from then on; the launch, and the contiguous cell list that it needs, 20 to
-// 30).  So where a tenth of a neighbourhood past 512 or a list past 136 is to
-// be expected.  2.4% of the owners of a uniform system have a list as long as that
-// of the corner (counted at densities 1.5 to 2.2, cutoffs 2.5 to 2.7, N = 4000
-// to 67500: of the tail of a normal distribution about it 2.1 to 2.4%).  What
-// that sweep shows holds for the next ones (note_dense).  N = 67500 at cutoff
-// 2.6 773 us from the first sweep on; a liquid of as many, which never needs it,
-// 728 and then 706.
+// Whether a first sweep should have the dense-owner kernel behind it.  That of a
+// few cells with long lists (dense_alone) should, and one in the wide shape that
+// an owner may outgrow: it would be repeated whole, which costs far more than
+// the launch (N = 67500 at density 2, cutoff 2.6: 1519 us and 773 from then on;
+// the launch, and the contiguous cell list that it needs, 20 to 30).  So where a
+// tenth of a neighbourhood past 512 or a list past 136 is to be expected.  2.4%
+// of the owners of a uniform system have a list as long as that of the corner
+// (counted at densities 1.5 to 2.2, cutoffs 2.5 to 2.7, N = 4000 to 67500: of the
+// tail of a normal distribution about it 2.1 to 2.4%).  What that sweep shows
+// holds for the next ones (note_dense).  N = 67500 at cutoff 2.6 773 us from the
+// first sweep on; a liquid of as many, which never needs it, 728 and then 706.
 bool dense_expected(const CellGrid &g, double cutoff, long long n)
 {
     if (g.nrep > 1 || n < 3) return false;
     const CellNeeds e = cell_needs(g, cutoff, n);
+    if (dense_alone(g, e)) return true;
+    if (!wide_expected(g, cutoff, n)) return false;
     auto past = [](double mean, double most) { return 0.5 * std::erfc((most - mean) / std::sqrt(2.0 * mean)); };
     return (double)g.ncell * past(e.staged, 512.0) + 0.024 * (double)n * past(e.list, 136.0) > 0.1;
 }
@@ -653,13 +669,19 @@ bool dense_expected(const CellGrid &g, double cutoff, long long n)
 bool cells_wide(const tb3_ctx *c, long long n) { return c->wide_need || wide_expected(c->grid, c->cutoff, n); }
 
 // Whether the dense-owner kernel follows the cell kernel: where some owner
-// needed it, and behind the first sweep in the wide shape where the density
-// makes that likely, or a sweep in the narrow one asked for the wide (it knows
-// the neighbourhoods, not the lists).
+// needed it, and behind the first sweep where the density makes that likely, or
+// a sweep in the narrow shape asked for the wide one (it knows the
+// neighbourhoods, not the lists).
 bool cells_dense(const tb3_ctx *c, long long n)
 {
     if (c->dense_on) return true;
-    return !c->dense_known && cells_wide(c, n) && (c->wide_need || dense_expected(c->grid, c->cutoff, n));
+    return !c->dense_known && (c->wide_need || dense_expected(c->grid, c->cutoff, n));
+}
+
+// Whether a narrow sweep that asked for the wide shape should get it.
+bool wide_taken(const CellGrid &g, double cutoff, long long n)
+{
+    return g.ncell <= WIDE_CELLS && !dense_alone(g, cell_needs(g, cutoff, n));
 }
 
 // Whether a fast sweep of n particles would find that out.
@@ -806,7 +828,7 @@ bool grow_after_overflow(tb3_ctx *c, long long n)
     // (or, where the cell kernel's wide shape is enough, that).  Replicas that
     // need it take both: their densities lie wide apart (48 clouds of up to
     // 2048: 1.50 ms in both kernels, with the narrow shape 1.66)
-    if (c->h_status->want_dense == 1 && c->grid.ncell <= WIDE_CELLS && !cells_wide(c, n)) {
+    if (c->h_status->want_dense == 1 && wide_taken(c->grid, c->cutoff, n) && !cells_wide(c, n)) {
         c->wide_need = true;
     } else if (c->h_status->want_dense) {
         c->dense_on = true;
@@ -1809,7 +1831,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
         // an owner needs it, the per-owner kernel with a growing list
         // capacity once a neighbourhood is too large for the cell kernel
         bool cells = true, wide = wide_expected(g, c->cutoff, n);
-        bool dense = wide && dense_expected(g, c->cutoff, n);
+        bool dense = dense_expected(g, c->cutoff, n);
         int cap = c->list_cap;
         Status h;
         for (int attempt = 0;; ++attempt) {
@@ -1835,7 +1857,7 @@ tb3_status tb3_energy_grad_dev_noalloc(tb3_ctx *c, int64_t n, const double *d_po
             if (!h.flags[2]) break;
             if (attempt >= 8) throw Fail(TB3_EHIP, "the cutoff sweep kept overflowing its LDS staging");
             if (h.flags[3]) cells = false;
-            if (h.want_dense == 1 && ncell <= WIDE_CELLS && !wide) wide = true;
+            if (h.want_dense == 1 && wide_taken(g, c->cutoff, n)) wide = true;
             if (h.want_dense) dense = true;
             if (!cells && h.flags[1] > cap) {
                 if (h.flags[1] > MAX_LIST)
